@@ -509,8 +509,8 @@ def main():
         # the batched workload counts SGC flips, the plain one canonical swaps (two flips each)
         "batched_over_plain_flips": value / (2.0 * plain_value),
         "roofline": roofline,
-        "launch_shape": {"shape": autotune.shape_name(tune_w), "waves_per_chain": tune_w[0],
-                         "moves_per_round": tune_w[1] if tune_w[2] != autotune.PATH_FIELDS else None,
+        "launch_shape": {"shape": autotune.shape_name(tune_w), "waves_per_chain": batch.launch_shape(0)[0],
+                         "moves_per_round": tune_w[1] if tune_w[1] > 0 else None,
                          "energy_path": "fields" if tune_w[2] == autotune.PATH_FIELDS else "evaluate",
                          "autotune_moves_per_s": {autotune.shape_name(k): v for k, v in tune_rates.items()}},
     }

@@ -10,8 +10,9 @@ The kernel variant (records per lane, energy tables in LDS or HBM) follows
 from the shape and the model.  More waves split each move's sub-clusters
 further (shorter dependent chain per move, one barrier per move or round
 more), fewer waves leave more CUs to other chains; fields make rejected
-moves cheap and accepted ones dearer.  A shape is (waves, moves per round,
-path); its name is "fields" or "WxK".  Results are cached per workload
+moves cheap and accepted ones dearer.  The automatic choice, which takes
+the patch kernel where the chain allows it, is timed beside them.  A shape is
+(waves, moves per round, path); its name is "auto", "fields" or "WxK".  Results are cached per workload
 signature in memory and, optionally, in a JSON file.
 """
 from __future__ import annotations
@@ -21,7 +22,7 @@ import os
 
 import numpy as np
 
-from .batch import PATH_EVALUATE, PATH_FIELDS, ChainBatch
+from .batch import PATH_AUTO, PATH_EVALUATE, PATH_FIELDS, ChainBatch
 
 _cache = {}
 
@@ -36,12 +37,19 @@ def signature(models, chains):
     return ";".join("%s:%d" % kv for kv in sorted(sig.items()))
 
 
+AUTO = (0, 0, PATH_AUTO)
+
+
 def shape_name(shape):
+    if tuple(shape) == AUTO:
+        return "auto"
     return "fields" if shape[2] == PATH_FIELDS else "%dx%d" % (shape[0], shape[1])
 
 
 def parse_shape(name):
-    """"fields" or "WxK" -> (waves, moves per round, path)."""
+    """"auto", "fields" or "WxK" -> (waves, moves per round, path)."""
+    if name == "auto":
+        return AUTO
     if name == "fields":
         return (1, 1, PATH_FIELDS)
     w, k = (int(v) for v in name.split("x"))
@@ -64,7 +72,7 @@ def tune(models, chains, candidates=(1, 2, 4, 8), per_round=(1, 8), fields=True,
         return tuple(entry["best"]), {parse_shape(k): r for k, r in entry["rates"].items()}
     scratch = ChainBatch(models, chains)
     moves = np.array([max(64, int(sweeps * m.n_sites)) for m in models], dtype=np.int64)
-    shapes = []
+    shapes = [AUTO]
     if fields:
         scratch.set_energy_path(PATH_FIELDS)
         if any(scratch.energy_path(c) == PATH_FIELDS for c in range(scratch.n_chains)):

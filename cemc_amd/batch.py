@@ -184,7 +184,8 @@ class ChainBatch:
         _capi.check(self._lib.cemc_batch_set_waves(self.handle, int(waves)))
 
     def set_moves_per_round(self, moves):
-        """0 (default): eight consecutive moves evaluated together wherever
+        """0 (default): the patch kernel's rounds where the chain allows it
+        (see launch_shape); else eight consecutive moves evaluated together wherever
         the chain's kernel variant allows it and the moves of a round seldom
         conflict (interacting sites, times 4 for swaps, at most 12% of the
         lattice), else one at a time; 1: every move on
@@ -193,7 +194,7 @@ class ChainBatch:
         of the round (periodic lattices whose records fit one wave; other
         chains take rounds of eight); wide rounds pay on large lattices at
         low acceptance, so the autotuner times them rather than choosing
-        them by default.  Same results bit for bit."""
+        them by default.  1 to 64 give the same results bit for bit."""
         _capi.check(self._lib.cemc_batch_set_moves_per_round(self.handle, int(moves)))
 
     def set_energy_path(self, path):
@@ -210,7 +211,9 @@ class ChainBatch:
         return v.value
 
     def launch_shape(self, chain):
-        """(waves per chain, records per lane in registers, tables in LDS)."""
+        """(waves per chain, records per lane in registers, sub-cluster tables
+        in LDS); on the patch kernel the second is its patches per lane and
+        the third False (its own tables replace them)."""
         w, r, g = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
         _capi.check(self._lib.cemc_batch_get_launch_shape(self.handle, int(chain), ctypes.byref(w),
                                                           ctypes.byref(r), ctypes.byref(g)))

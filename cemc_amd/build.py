@@ -44,6 +44,8 @@ def _units():
         for p in (0, 1):
             units.append(("ce_sweep_w%d_p%d" % (w, p), "ce_sweep_inst.hip",
                           ["-DCEMC_SWEEP_WAVES=%d" % w, "-DCEMC_SWEEP_PERIODIC=%d" % p]))
+    for w in SWEEP_WAVES:
+        units.append(("ce_patch_w%d" % w, "ce_patch_inst.hip", ["-DCEMC_PATCH_WAVES=%d" % w]))
     for p in (0, 1):
         for sgc in (0, 1):
             units.append(("ce_wl_p%d_s%d" % (p, sgc), "ce_wl_inst.hip",

@@ -57,6 +57,20 @@ constexpr uint32_t kRecUnused1 = 1u << 28;
 constexpr uint32_t kRecUnused2 = 1u << 29;
 constexpr uint32_t kRecValid = 1u << 31;
 
+// Patch (ce_patches.h): up to kPatchMembers members whose species index one
+// table holding all the sub-clusters inside the patch.
+//   m[q]    members as in FatRec (places the patch does not use address the
+//           reference site; the table repeats over their species)
+//   base    first double of its table in ModelDev::ptab
+//   w_last  index weight of the last place's species (0: the place is unused
+//           and the table does not hold its codes); place q before it weighs
+//           n_species^q
+struct PatchRec {
+  int32_t m[6];
+  uint32_t base;
+  uint32_t w_last;
+};
+
 // Cluster entry = one (translation group, orbit) pair with its record range.
 struct ClusterEntry {
   int32_t rec_begin;   // into the model's record array
@@ -123,6 +137,13 @@ struct ModelDev {
   double fx_scale;
   const int64_t* gtab_fx;
   const uint32_t* duals;
+  // Patches of the one translation group (n_patch 0: none were found or the
+  // model has several groups): their tables as [code][d], d < n_bfs, the
+  // first table all zeros (padding patches read it).
+  int32_t n_patch;
+  int32_t ptab_size;  // doubles
+  const PatchRec* patches;
+  const double* ptab;
 };
 
 // Per-chain parameters (host written).

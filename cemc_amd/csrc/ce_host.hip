@@ -24,6 +24,7 @@
 
 #include "cemc_gpu.h"
 #include "ce_kernels.h"
+#include "ce_patches.h"
 
 using namespace cemc;
 
@@ -167,7 +168,17 @@ struct cemc_model {
     return p;
   }
 
+  // patches of the one translation group (ce_patches.h)
+  PatchCover cover;
+  std::vector<PatchRec> patches;
+  std::vector<double> ptab;
+  std::vector<uint32_t> ptab_base;  // per table of the cover
+  PatchRec* d_patches = nullptr;
+  double* d_ptab = nullptr;
+
   void build_gtab(const std::vector<double>& J);
+  void build_patches();
+  void build_ptab();
   void build_gtab_il();
   void build_gtab_fx();
   void build_duals();
@@ -184,6 +195,8 @@ cemc_model::~cemc_model() {
   dev_free(d_gtab);
   dev_free(d_gtab_il);
   dev_free(d_gtab_fx);
+  dev_free(d_patches);
+  dev_free(d_ptab);
   dev_free(d_duals);
   dev_free(d_trans);
   dev_free(d_cells);
@@ -404,6 +417,128 @@ void cemc_model::build_duals() {
   field_ok = true;
 }
 
+// Patches (ce_patches.h) of models on closed-form lattices with one
+// translation group and up to four species.  Positions of a cluster that
+// every correlation function on it treats alike (its decorations keep their
+// counts when the two are exchanged) are interchangeable whatever the ECIs
+// are; bringing records into one order under these exchanges lets symmetry
+// images of a patch share a table.
+void cemc_model::build_patches() {
+  cover = PatchCover();
+  patches.clear();
+  ptab_base.clear();
+  const int q = patch_members(n_species);
+  if (q == 0 || !spec_ok) return;
+  // per entry: the position permutations that keep every function
+  std::vector<std::vector<std::array<int, 4>>> alike(n_entries);
+  for (int c = 0; c < n_entries; ++c) {
+    const int n = entry_size[c];
+    std::array<int, 4> p{0, 1, 2, 3};
+    do {
+      bool keeps = true;
+      for (int k = 0; keeps && k < n_cf; ++k) {
+        if (cf_kind[k] != CEMC_CF_CLUSTER || cf_entry[entry_group[c] * n_cf + k] != c) continue;
+        std::vector<uint32_t> a, b;
+        for (int e = cf_eq_off[k]; e < cf_eq_off[k + 1]; ++e) {
+          uint32_t u = 0, v = 0;
+          for (int pos = 0; pos < n; ++pos) {
+            u |= ((eq_decos[e] >> (8 * pos)) & 0xFFu) << (8 * pos);
+            v |= ((eq_decos[e] >> (8 * pos)) & 0xFFu) << (8 * p[pos]);
+          }
+          a.push_back(u);
+          b.push_back(v);
+        }
+        std::sort(a.begin(), a.end());
+        std::sort(b.begin(), b.end());
+        keeps = a == b;
+      }
+      if (keeps) alike[c].push_back(p);
+    } while (std::next_permutation(p.begin(), p.begin() + n));
+  }
+  // records in search form: sites are the translation columns
+  const int block = deco_slices() << (3 * code_bits());
+  std::vector<int> col_of_site, site_of_col(K, -1);
+  std::vector<PatchInput> in;
+  for (size_t r = 0; r < recs.size(); ++r) {
+    const int c = rec_entry[r], n = entry_size[c], ref = rec_refpos(recs[r]);
+    int at[4] = {-1, -1, -1, -1};  // column at each position
+    for (int pos = 0, t = 0; pos < n; ++pos)
+      if (pos != ref) at[pos] = int(rec_slot(recs[r], t++));
+    // the permutation that takes the reference site to the lowest position
+    const std::array<int, 4>* best = &alike[c][0];
+    for (const auto& p : alike[c])
+      if (p[ref] < (*best)[ref]) best = &p;
+    const int ref2 = (*best)[ref];
+    int now[4] = {-1, -1, -1, -1};
+    for (int pos = 0; pos < n; ++pos) now[(*best)[pos]] = at[pos];
+    PatchInput x;
+    x.n = 0;
+    int member_at[4] = {0, 0, 0, 0};
+    for (int pos = 0; pos < n; ++pos) {
+      if (pos == ref2) continue;
+      int& site = site_of_col[now[pos]];
+      if (site < 0) {
+        site = int(col_of_site.size());
+        col_of_site.push_back(now[pos]);
+      }
+      member_at[pos] = x.n;
+      x.site[x.n++] = site;
+    }
+    for (int i = x.n; i < 3; ++i) x.site[i] = -1;
+    x.block = uint32_t(entry_goff[c] + ref2 * block);
+    for (const auto& p : alike[c]) {
+      if (p[ref2] != ref2) continue;
+      std::array<int, 3> o{0, 1, 2};
+      for (int pos = 0; pos < n; ++pos)
+        if (pos != ref2) o[member_at[pos]] = member_at[p[pos]];
+      x.orders.push_back(o);
+    }
+    in.push_back(x);
+  }
+  if (!PatchSearch(int(col_of_site.size()), in, q).run(&cover)) {
+    cover = PatchCover();
+    return;
+  }
+  // tables: a zero one for padding lanes, then one per type; a type that
+  // leaves the last place unused holds no codes of it
+  int part = n_bfs;
+  for (int i = 0; i < q - 1; ++i) part *= n_species;
+  std::vector<uint32_t> w_last;
+  uint32_t off = uint32_t(part);
+  for (const auto& terms : cover.tables) {
+    bool full = false;
+    for (const auto& t : terms)
+      for (int m = 0; m < t.n; ++m) full = full || t.place[m] == q - 1;
+    ptab_base.push_back(off);
+    w_last.push_back(full ? uint32_t(part / n_bfs) : 0u);
+    off += uint32_t(full ? part * n_species : part);
+  }
+  ptab.assign(off, 0.0);
+  for (const auto& p : cover.patches) {
+    PatchRec rec{{0, 0, 0, 0, 0, 0}, ptab_base[p.table], w_last[p.table]};
+    for (int i = 0; i < q; ++i) {
+      if (p.site[i] < 0) continue;
+      const int* o = &signed_cells[3 * col_of_site[p.site[i]]];
+      rec.m[i] = (o[0] * pdims[1] + o[1]) * pdims[2] + o[2];
+    }
+    patches.push_back(rec);
+  }
+  build_ptab();
+}
+
+// The patch tables from the sub-clusters' (after build_gtab).
+void cemc_model::build_ptab() {
+  const int q = patch_members(n_species);
+  int part = 1;
+  for (int i = 0; i < q - 1; ++i) part *= n_species;
+  for (size_t t = 0; t < ptab_base.size(); ++t) {
+    const uint32_t end = t + 1 < ptab_base.size() ? ptab_base[t + 1] : uint32_t(ptab.size());
+    const bool full = end - ptab_base[t] > uint32_t(part * n_bfs);
+    patch_table(cover.tables[t], n_species, full ? q : q - 1, n_bfs, n_bfs, code_bits(), gtab.data(),
+                ptab.data() + ptab_base[t]);
+  }
+}
+
 void cemc_model::refresh_view() {
   ModelDev& v = view;
   std::memset(&v, 0, sizeof v);
@@ -450,6 +585,10 @@ void cemc_model::refresh_view() {
   v.eci = d_eci;
   v.field_ok = field_ok ? 1 : 0;
   v.fx_scale = fx_scale;
+  v.n_patch = int(patches.size());
+  v.ptab_size = int(ptab.size());
+  v.patches = d_patches;
+  v.ptab = d_ptab;
   v.gtab_fx = d_gtab_fx;
   v.duals = d_duals;
   if (!d_view) HIP_CHECK(hipMalloc(&d_view, sizeof(ModelDev)));
@@ -687,6 +826,11 @@ static void build_model(cemc_model* m, const cemc_model_desc* d) {
   m->d_gtab = upload(m->gtab);
   m->build_gtab_il();
   if (!m->gtab_il.empty()) m->d_gtab_il = upload(m->gtab_il);
+  m->build_patches();
+  if (!m->patches.empty()) {
+    m->d_patches = upload(m->patches);
+    m->d_ptab = upload(m->ptab);
+  }
   m->build_duals();
   m->build_gtab_fx();
   m->d_gtab_fx = upload(m->gtab_fx);
@@ -1335,6 +1479,8 @@ struct cemc_batch {
     bool field;  // local-field kernel
     bool hooks;  // constraints and bias
     int nm;      // members gathered per record
+    int kg;      // patch kernel: lanes per move (0: another kernel)
+    bool trk_lds;  // patch kernel: the tracker in LDS
     int begin, count;
     uint32_t lds;
   };
@@ -1557,6 +1703,8 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     bool field;
     bool hooks;
     int nm;
+    int kg = 0;
+    bool trk_lds = true;
     uint32_t lds;
   };
   // waves per chain: enough chains x waves to give every SIMD of the
@@ -1717,6 +1865,37 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       }
       k.nm = (k.kr > 0 && m->max_members <= 2) ? 2 : 3;
     }
+    // patches, where no launch shape was asked for: a row of 16 lanes per
+    // move up to 64 patches, else the wave; about one wave per SIMD over the
+    // device as above, but four waves at most for rows (rounds of 16) and two
+    // at least for whole waves.  Measured with 1, 2, 4 and 8 waves: 1024
+    // binary SGC chains 95.8, 97.2, 124.8 ms; 256 ternary chains 36.7, 30.7,
+    // 29.4 ms; 128 quaternary chains (two waves up) 31.3, 20.6, 18.6 ms.  The
+    // sweep kernel on the same passes: 150, 55.6 and 56.7 ms.
+    if (forced_waves == 0 && b->spec_moves == 0 && !k.field && !k.hooks && !m->patches.empty() &&
+        (!canon || m->n_sites <= 65535)) {
+      const int P = int(m->patches.size());
+      const uint32_t room = limit + sweep_static_lds() - kPatchStaticLds;
+      const int kg = P <= 64 ? 16 : 64;
+      const int kr = P <= 16 ? 1 : (P <= 32 ? 2 : (P <= 64 ? 4 : (P <= 128 ? 2 : (P <= 256 ? 4 : 8))));
+      const int waves = kg == 16 ? std::min(batch_waves, 4) : std::max(2, batch_waves);
+      bool trk_lds = true;
+      uint32_t need = patch_lds_bytes(occ_bytes, trk_sites, int(m->ptab.size()));
+      if (canon && need > room) {
+        trk_lds = false;
+        need = patch_lds_bytes(occ_bytes, 0, int(m->ptab.size()));
+      }
+      if (P <= 512 && need <= room && patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon)) {
+        k.kg = kg;
+        k.kr = kr;
+        k.waves = waves;
+        k.trk_lds = trk_lds;
+        k.spec = 1;
+        k.glds = false;  // the sub-clusters' tables are not read
+        k.nm = 3;
+        k.lds = need;
+      }
+    }
     keys[c] = k;
   }
   for (int c0 = 0; c0 < n_chains; ++c0) {
@@ -1728,7 +1907,8 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       const Key& k = keys[c];
       if (done[c] || k.periodic != k0.periodic || k.canonical != k0.canonical || k.kr != k0.kr ||
           k.glds != k0.glds || k.kbm != k0.kbm || k.waves != k0.waves || k.spec != k0.spec ||
-          k.field != k0.field || k.hooks != k0.hooks || k.nm != k0.nm)
+          k.field != k0.field || k.hooks != k0.hooks || k.nm != k0.nm || k.kg != k0.kg ||
+          k.trk_lds != k0.trk_lds)
         continue;
       done[c] = true;
       ids.push_back(c);
@@ -1740,7 +1920,7 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       return int64_t(mx->n_sites) * mx->recs.size() > int64_t(my->n_sites) * my->recs.size();
     });
     b->classes.push_back(cemc_batch::Class{k0.periodic, k0.canonical, k0.kr, k0.glds, k0.kbm, k0.waves, k0.spec,
-                                           k0.field, k0.hooks, k0.nm, int(order.size()), int(ids.size()), lds});
+                                           k0.field, k0.hooks, k0.nm, k0.kg, k0.trk_lds, int(order.size()), int(ids.size()), lds});
     order.insert(order.end(), ids.begin(), ids.end());
   }
   if (order.size() > b->order_cap || b->d_order == nullptr) {
@@ -1824,6 +2004,8 @@ void enqueue_sweeps(cemc_batch* b, uint32_t* d_log, int64_t log_words, int64_t t
     a.field = cl.field;
     a.hooks = cl.hooks ? b->d_hooks : nullptr;
     a.nm = cl.nm;
+    a.kg = cl.kg;
+    a.trk_lds = cl.trk_lds;
     a.accept_log = d_log;
     a.log_words = log_words;
     a.time_limit = time_limit;
@@ -2187,6 +2369,10 @@ int cemc_model_set_ecis(cemc_model* m, const double* eci) {
     if (!m->gtab_il.empty())
       HIP_CHECK(hipMemcpy(m->d_gtab_il, m->gtab_il.data(), sizeof(double) * m->gtab_il.size(),
                           hipMemcpyHostToDevice));
+    if (!m->patches.empty()) {
+      m->build_ptab();
+      HIP_CHECK(hipMemcpy(m->d_ptab, m->ptab.data(), sizeof(double) * m->ptab.size(), hipMemcpyHostToDevice));
+    }
     m->build_gtab_fx();
     HIP_CHECK(hipMemcpy(m->d_gtab_fx, m->gtab_fx.data(), sizeof(int64_t) * m->gtab_fx.size(),
                         hipMemcpyHostToDevice));

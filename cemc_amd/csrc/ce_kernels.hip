@@ -24,6 +24,7 @@
 #include <mutex>
 
 #include "ce_sweep.h"
+#include "ce_patch_kernel.h"
 #include "ce_wl.h"
 
 
@@ -814,6 +815,29 @@ CEMC_DECLARE_SWEEP_FN(8, 0)
 CEMC_DECLARE_SWEEP_FN(8, 1)
 #undef CEMC_DECLARE_SWEEP_FN
 
+const void* patch_fn_w1(bool canonical, int kbm, int kg, int kr, bool trk_lds);
+const void* patch_fn_w2(bool canonical, int kbm, int kg, int kr, bool trk_lds);
+const void* patch_fn_w4(bool canonical, int kbm, int kg, int kr, bool trk_lds);
+const void* patch_fn_w8(bool canonical, int kbm, int kg, int kr, bool trk_lds);
+
+static const void* patch_fn(bool canonical, int kbm, int kg, int kr, int waves, bool trk_lds) {
+  switch (waves) {
+    case 1: return patch_fn_w1(canonical, kbm, kg, kr, trk_lds);
+    case 2: return patch_fn_w2(canonical, kbm, kg, kr, trk_lds);
+    case 4: return patch_fn_w4(canonical, kbm, kg, kr, trk_lds);
+    case 8: return patch_fn_w8(canonical, kbm, kg, kr, trk_lds);
+    default: return nullptr;
+  }
+}
+
+bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool canonical) {
+  return patch_fn(canonical, kbm, kg, kr, waves, trk_lds) != nullptr;
+}
+
+uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles) {
+  return patch_layout(occ_bytes, trk_sites, tab_doubles).total;
+}
+
 const void* field_fn(bool canonical, int kr, int kbm);
 const void* wl_fn_p0s0(int kr, bool glds, int kbm, int nm, int mode);
 const void* wl_fn_p1s0(int kr, bool glds, int kbm, int nm, int mode);
@@ -897,6 +921,23 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
               if (e != hipSuccess) return e;
             }
   for (int cn = 0; cn < 2; ++cn)
+    for (int w : {1, 2, 4, 8})
+      for (int kg : {16, 64})
+        for (int kr : {1, 2, 4, 8})
+          for (int kbm : {1, 2, 3})
+            for (int tl = 0; tl < 2; ++tl) {
+              const void* fn = patch_fn(cn != 0, kbm, kg, kr, w, tl != 0);
+              if (fn == nullptr) continue;
+              hipFuncAttributes attr;
+              hipError_t e = hipFuncGetAttributes(&attr, fn);
+              if (e != hipSuccess) return e;
+              if (attr.sharedSizeBytes > kPatchStaticLds) return hipErrorInvalidValue;
+              const int dyn = int(bytes) - int(attr.sharedSizeBytes);
+              if (dyn <= 0) return hipErrorInvalidValue;
+              e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
+              if (e != hipSuccess) return e;
+            }
+  for (int cn = 0; cn < 2; ++cn)
     for (int kr : {2, 4, 8})
       for (int kbm : {1, 2, 3}) {
         const void* fn = field_fn(cn != 0, kr, kbm);
@@ -914,7 +955,10 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
 
 hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   const void* fn = nullptr;
-  if (a.field) {
+  if (a.kg != 0) {
+    if (!a.periodic || a.field || a.hooks != nullptr) return hipErrorInvalidValue;
+    fn = patch_fn(a.canonical, a.kbm, a.kg, a.kr, a.waves, a.trk_lds);
+  } else if (a.field) {
     if (!a.periodic || a.waves != 1 || a.hooks != nullptr) return hipErrorInvalidValue;
     fn = field_fn(a.canonical, a.kr, a.kbm);
   } else {
@@ -935,6 +979,10 @@ hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   int64_t log_words = a.log_words;
   HookDev* hooks = a.hooks;
   int64_t time_limit = a.time_limit;
+  if (a.kg != 0) {
+    void* pargs[] = {&params, &states, &models, &occ_pool, &trk_pool, &order, &n_moves, &log, &log_words, &time_limit};
+    return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), pargs, a.lds_bytes, stream);
+  }
   if (a.field) {
     void* fargs[] = {&params, &states, &models, &occ_pool, &trk_pool, &order, &n_moves, &log, &log_words, &hooks};
     return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), fargs, a.lds_bytes, stream);

@@ -276,8 +276,12 @@ CEMC_API int cemc_batch_set_waves(cemc_batch* batch, int32_t waves);
  * move of the round affects (that move is evaluated again); 1 evaluates
  * every move on its own; 0 (default) takes 8 wherever the chain's variant
  * allows it and the moves of a round seldom conflict (the sites a move
- * interacts with, times 4 for swaps, are at most 12% of the lattice), else 1.
- * All give the same moves, energies and accept sequence, bit for bit; rounds
+ * interacts with, times 4 for swaps, are at most 12% of the lattice), else 1,
+ * where the chain does not run on the patch kernel (see
+ * cemc_batch_get_launch_shape), whose rounds have 8 or 16 moves.
+ * The values 1 to 64 give the same moves, energies and accept sequence, bit
+ * for bit (the patch kernel: the same moves and accept sequence, energies
+ * within rounding); rounds
  * share one wave reduction, one barrier and one decision step among their
  * moves.  No counterpart in the reference (its moves are
  * sequential). */
@@ -300,7 +304,12 @@ CEMC_API int cemc_batch_set_energy_path(cemc_batch* batch, int32_t path);
 /* Energy path a chain runs on (CEMC_PATH_EVALUATE or CEMC_PATH_FIELDS). */
 CEMC_API int cemc_batch_get_energy_path(cemc_batch* batch, int32_t chain, int32_t* path);
 /* Launch shape of one chain: waves per chain, sub-cluster records per lane
- * held in registers (0: records in LDS), energy tables in LDS (1) or HBM (0). */
+ * held in registers (0: records in LDS), the sub-clusters' energy tables in
+ * LDS (1) or HBM (0).  By default (no waves, moves per round or field path
+ * asked for) chains on closed-form periodic lattices with one translation
+ * group and up to four species run on the patch kernel, which reads tables
+ * of whole groups of sub-clusters from LDS instead: it reports its patches
+ * per lane as the second value and 0 as the third. */
 CEMC_API int cemc_batch_get_launch_shape(cemc_batch* batch, int32_t chain, int32_t* waves,
                                          int32_t* records_per_lane, int32_t* tables_in_lds);
 /* Temperature of one chain (parallel tempering uses it to exchange replicas). */

@@ -428,7 +428,7 @@ void cemc_model::build_patches() {
   patches.clear();
   ptab_base.clear();
   const int q = patch_members(n_species);
-  if (q == 0 || !spec_ok) return;
+  if (q == 0 || !spec_ok || std::max({dims[0], dims[1], dims[2]}) > 127) return;
   // per entry: the position permutations that keep every function
   std::vector<std::vector<std::array<int, 4>>> alike(n_entries);
   for (int c = 0; c < n_entries; ++c) {
@@ -1865,27 +1865,35 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       }
       k.nm = (k.kr > 0 && m->max_members <= 2) ? 2 : 3;
     }
-    // patches, where no launch shape was asked for: a row of 16 lanes per
-    // move up to 64 patches, else the wave; about one wave per SIMD over the
-    // device as above, but four waves at most for rows (rounds of 16) and two
-    // at least for whole waves.  Measured with 1, 2, 4 and 8 waves: 1024
-    // binary SGC chains 95.8, 97.2, 124.8 ms; 256 ternary chains 36.7, 30.7,
-    // 29.4 ms; 128 quaternary chains (two waves up) 31.3, 20.6, 18.6 ms.  The
-    // sweep kernel on the same passes: 150, 55.6 and 56.7 ms.
+    // patches, where no launch shape was asked for.  Up to 64 patches: about
+    // one wave per SIMD over the device as above, four at most, which then
+    // evaluate a round of 16 moves together (one wave: a quad per move;
+    // more: a row of 16 lanes per move).  More patches: a wave per move,
+    // rounds of eight over two to eight waves.  Measured with 1, 2 and 4
+    // waves: 1024 binary SGC chains 71, 81, 114 ms; 256 ternary chains 25.5,
+    // 19.4, 19.6 ms; a mix of 48 chains 2.25, 1.83, 1.78 ms; one binary
+    // chain 12.0 ms with any.  128 quaternary chains with 2, 4 and 8 waves:
+    // 31, 21 and 18 ms.
     if (forced_waves == 0 && b->spec_moves == 0 && !k.field && !k.hooks && !m->patches.empty() &&
         (!canon || m->n_sites <= 65535)) {
       const int P = int(m->patches.size());
       const uint32_t room = limit + sweep_static_lds() - kPatchStaticLds;
-      const int kg = P <= 64 ? 16 : 64;
-      const int kr = P <= 16 ? 1 : (P <= 32 ? 2 : (P <= 64 ? 4 : (P <= 128 ? 2 : (P <= 256 ? 4 : 8))));
-      const int waves = kg == 16 ? std::min(batch_waves, 4) : std::max(2, batch_waves);
+      int waves = P <= 64 ? std::min(batch_waves, 4) : std::max(2, batch_waves);
+      if (P > 60 && waves == 1) waves = 2;
+      const int kg = P > 64 ? 64 : (waves == 1 ? 4 : 16);
+      int kr = 0;
+      for (int r : {3, 6, 9, 15})
+        if (kg == 4 && kr == 0 && P <= 4 * r) kr = r;
+      for (int r : {1, 2, 4, 7})
+        if (kg != 4 && kr == 0 && P <= kg * r) kr = r;
+      const int near_slots = canon && kg != 64 ? kg * kr : 0;
       bool trk_lds = true;
-      uint32_t need = patch_lds_bytes(occ_bytes, trk_sites, int(m->ptab.size()));
+      uint32_t need = patch_lds_bytes(occ_bytes, trk_sites, int(m->ptab.size()), near_slots);
       if (canon && need > room) {
         trk_lds = false;
-        need = patch_lds_bytes(occ_bytes, 0, int(m->ptab.size()));
+        need = patch_lds_bytes(occ_bytes, 0, int(m->ptab.size()), near_slots);
       }
-      if (P <= 512 && need <= room && patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon)) {
+      if (kr > 0 && need <= room && patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon)) {
         k.kg = kg;
         k.kr = kr;
         k.waves = waves;

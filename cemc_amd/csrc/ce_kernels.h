@@ -26,7 +26,7 @@ struct LaunchSweep {
   int kbm;         // decoration slices read per record: n_bfs for up to 4 species (1, 2, 3), else 7
   int waves;       // wavefronts per chain: 1, 2, 4 or 8 (more than 1: kr > 0)
   int spec;        // moves per round: 1, or kSpecMoves (periodic, kr > 0)
-  int kg;          // patch kernel (ce_patch_kernel.h): lanes per move, 16 or 64 (0: the sweep kernel); kr is then
+  int kg;          // patch kernel (ce_patch_kernel.h): lanes per move, 4, 16 or 64 (0: the sweep kernel); kr is then
                    // the patches per lane
   bool trk_lds;    // patch kernel: the tracker is held in LDS
   bool field;      // local-field kernel (periodic, one wave, kr > 0, kbm <= 3)
@@ -47,9 +47,11 @@ bool sweep_variant_ok(int kr, bool gtab_lds, int kbm, int waves, int spec, bool 
 // Dynamic LDS of one chain on the local-field kernel: padded occupation and
 // its site map, tracker entries, n_sites x B integer fields, integer tables.
 uint32_t field_lds_bytes(int occ_bytes, int trk_sites, int n_fields, int gtab_ints);
-// Dynamic LDS of one chain on the patch kernel, and that kernel's static LDS.
-uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles);
-constexpr uint32_t kPatchStaticLds = 5u * 1024u;  // bound, checked when the limits are raised
+// Dynamic LDS of one chain on the patch kernel (near_slots: patch slots of a
+// canonical chain with a quad or row per move, else 0), and a bound on that
+// kernel's static LDS.
+uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles, int near_slots);
+constexpr uint32_t kPatchStaticLds = 7u * 1024u;  // bound, checked when the limits are raised
 bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool canonical);
 // Raises the dynamic-LDS limit of every sweep kernel instantiation to
 // `bytes` minus that kernel's static LDS.

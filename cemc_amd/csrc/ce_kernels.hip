@@ -834,8 +834,8 @@ bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool can
   return patch_fn(canonical, kbm, kg, kr, waves, trk_lds) != nullptr;
 }
 
-uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles) {
-  return patch_layout(occ_bytes, trk_sites, tab_doubles).total;
+uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles, int near_slots) {
+  return patch_layout(occ_bytes, trk_sites, tab_doubles, kNearCells * near_slots).total;
 }
 
 const void* field_fn(bool canonical, int kr, int kbm);
@@ -922,8 +922,8 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
             }
   for (int cn = 0; cn < 2; ++cn)
     for (int w : {1, 2, 4, 8})
-      for (int kg : {16, 64})
-        for (int kr : {1, 2, 4, 8})
+      for (int kg : {4, 16, 64})
+        for (int kr : {1, 2, 3, 4, 6, 7, 9, 15})
           for (int kbm : {1, 2, 3})
             for (int tl = 0; tl < 2; ++tl) {
               const void* fn = patch_fn(cn != 0, kbm, kg, kr, w, tl != 0);

@@ -1,9 +1,9 @@
 // Instantiations of the patch kernel for one number of waves per chain,
 // CEMC_PATCH_WAVES (1, 2, 4, 8), one object each; exposes
 // patch_fn_w<W>(canonical, kbm, kg, kr, trk_lds), the kernel's address or nullptr
-// for a variant that is not built.  A row of 16 lanes per move: up to 64
-// patches, one, two or four waves; a wave per move: up to 512 patches, two,
-// four or eight waves.
+// for a variant that is not built.  One wave: a quad per move, up to 60
+// patches; two or four waves: a row of 16 lanes per move, up to 64 patches;
+// two, four or eight waves: a wave per move, up to 448 patches.
 #include "ce_patch_kernel.h"
 
 #ifndef CEMC_PATCH_WAVES
@@ -18,8 +18,13 @@ constexpr int W = CEMC_PATCH_WAVES;
 
 template <bool C, int KBM>
 const void* row_fn(int kr) {
-  if constexpr (W <= 4) {
-    constexpr int kP = W == 1 ? 2 : 1;
+  if constexpr (W == 1) {
+    if (kr == 3) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 4, 3, 1, 1, true>);
+    if (kr == 6) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 4, 6, 1, 1, true>);
+    if (kr == 9) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 4, 9, 1, 1, true>);
+    if (kr == 15) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 4, 15, 1, 1, true>);
+  } else if constexpr (W <= 4) {
+    constexpr int kP = 4 / W;
     if (kr == 1) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 16, 1, W, kP, true>);
     if (kr == 2) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 16, 2, W, kP, true>);
     if (kr == 4) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 16, 4, W, kP, true>);
@@ -33,17 +38,18 @@ const void* wave_fn(int kr) {
     constexpr int kP = 8 / W;
     if (kr == 2) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 64, 2, W, kP, T>);
     if (kr == 4) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 64, 4, W, kP, T>);
-    if (kr == 8) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 64, 8, W, kP, T>);
+    if (kr == 7) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 64, 7, W, kP, T>);
   }
   return nullptr;
 }
 
 template <bool C>
 const void* pick(int kbm, int kg, int kr, bool trk_lds) {
-  if (kg == 16) {
+  if (kg == (W == 1 ? 4 : 16)) {
     if (!trk_lds) return nullptr;
     return kbm == 1 ? row_fn<C, 1>(kr) : (kbm == 2 ? row_fn<C, 2>(kr) : (kbm == 3 ? row_fn<C, 3>(kr) : nullptr));
   }
+  if (kg != 64) return nullptr;
   if (!C || trk_lds)
     return kbm == 1 ? wave_fn<C, 1, true>(kr)
                     : (kbm == 2 ? wave_fn<C, 2, true>(kr) : (kbm == 3 ? wave_fn<C, 3, true>(kr) : nullptr));

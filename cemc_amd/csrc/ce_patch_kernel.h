@@ -4,46 +4,63 @@
 //
 // One workgroup of kW waves owns one chain on a closed-form periodic lattice
 // with one translation group; the padded occupation box, the species tracker
-// and the patch tables stay in LDS for the launch.  Moves are made in rounds
-// of kK: all are evaluated against the same state, then committed in order
-// up to the first one that reads what an accepted earlier one changed.
+// and the patch tables stay in LDS for the launch.
+//
+// Rounds.  The first kK moves of the 64-move block that are still open are
+// evaluated against the same state.  A move that an accepted earlier one of
+// the round reaches (reads a site or shares a tracker slot with) is blocked,
+// and so is one that a blocked one reaches; the others are made at once, in
+// any order, since none reads what another writes.  Blocked moves stay open
+// for the next round.  (Ending the round at the first blocked move instead
+// made 5.6 moves of eight at the highest acceptances, now about 11 of 16.)
 //
 // Work split.  A flip needs 12 (two species, pairs to the 4th shell and
 // triplets to the 2nd), 59 (three species, four-body clusters) or 426 (four
 // species, four-body to the 3rd shell) patch entries where it needed 114, 494
-// and 1746 sub-cluster entries.  kG lanes evaluate one move, kR patches each:
-// a row of 16 lanes for up to 64 patches, so that a wave evaluates four moves
-// at once and each sum takes four DPP levels inside a row; the whole wave for
-// more.
+// and 1746 sub-cluster entries.  One wave takes 16 moves at once, a quad of
+// lanes each; several waves take a row of 16 lanes per move, or a wave per
+// move above 64 patches.
 //
-// What bounds it: the dependent chain of a round (move fetch, gathers, table
-// reads, sum, verdict, commit), not bandwidth.  So everything that does not
-// depend on the verdict is done while the reads are in flight: which moves of
-// the round affect which, where the commits would go; and everything that
-// the next round does not need is put off to the end of the 64-move block,
-// where lane l still holds move l: energies by one prefix sum over the lanes,
-// sample sums in per-lane accumulators added up once per launch.
+// What bounds it: instruction issue and LDS latency of the dependent chain of
+// a round, not bandwidth (binary SGC chains, counters per move: 18 VALU, 4
+// LDS and 3 scalar instructions, 27 of 45 quad-cycles issuing, 16 waiting;
+// the sweep kernel issued 43 VALU and 10 LDS).  So the loads of a phase are
+// issued together before the first wait (one binary chain, 40000 swaps: 14.6
+// -> 12.0 ms by that and by reading the tracker in the round instead of
+// comparing every commit with every lane); which moves reach which is tested
+// while the members are in flight; and what the next round does not need is
+// put off to the end of the block, where lane l holds move l: energies by one
+// prefix sum over the lanes, sample sums in per-lane accumulators added up
+// once per launch.  Four-species models are bound by LDS reads instead (two
+// thirds of the cycles at eight waves).
+//
+// Measured against the sweep kernel's automatic shapes, per pass: 1024 binary
+// SGC chains of 500 sweeps 150 -> 71.5 ms, 256 ternary chains of 512-4096
+// sites 55.6 -> 18.9 ms, a mix of 48 binary and ternary chains 5.8 -> 1.8 ms,
+// 128 quaternary 32^3 replicas 56.7 -> 16.5 ms, one binary chain 23.9 -> 11.7
+// ms, 128 quaternary 8^3 chains 5.4 -> 3.0 ms (1.2 ms of it the kernel).
 #pragma once
 
 #include "ce_sweep.h"
 
 namespace cemc {
 
-// Dynamic LDS: padded occupation | tracker (canonical, when held in LDS) | patch tables.
+// Dynamic LDS: padded occupation | tracker (canonical, when held in LDS) |
+// patch tables | weights of the members by offset (canonical, near_cells x slots).
 struct PatchLayout {
-  uint32_t trk, tab, total;
+  uint32_t trk, tab, near, total;
 };
-__host__ __device__ inline PatchLayout patch_layout(int occ_bytes, int trk_sites, int tab_doubles) {
+__host__ __device__ inline PatchLayout patch_layout(int occ_bytes, int trk_sites, int tab_doubles, int near_bytes) {
   PatchLayout L;
   L.trk = align16(uint32_t(occ_bytes));
   L.tab = L.trk + align16(uint32_t(trk_sites) * 2u);
-  L.total = L.tab + uint32_t(tab_doubles) * 8u;
+  L.near = L.tab + uint32_t(tab_doubles) * 8u;
+  L.total = L.near + align16(uint32_t(near_bytes));
   return L;
 }
+constexpr int kNearCells = 126;  // offsets within a halo of 2, and one for "none"
 
 namespace {
-
-constexpr int kNoPatch = 1 << 24;  // no lattice offset: the second site of a swap does not see the first
 
 template <int kCtrl, int kRows>
 __device__ __attribute__((always_inline)) inline double dpp_or0_f64(double v) {
@@ -63,27 +80,31 @@ __device__ __attribute__((always_inline)) inline double wave_scan_f64(double v) 
   return v;
 }
 
-// Sum over the row of 16 lanes; every lane of the row ends with it.
-__device__ __attribute__((always_inline)) inline double row_sum_f64(double v) {
-  v += dpp_f64<0x128>(v);
-  return octet_sum_f64(v);
-}
+// n / d for n, d < 2^16 by one multiplication: inv = ceil(2^32 / d) is at most
+// d / 2^32 too large, so the quotient is exact.
+__device__ __attribute__((always_inline)) inline uint32_t div16(uint32_t n, uint32_t inv) { return __umulhi(n, inv); }
 
-// Padded-lattice offset of site i as seen from site j when it lies within
-// the halo of j along every axis (then a member offset of j equals it exactly
-// when the member is i), else kNoPatch.
-__device__ __attribute__((always_inline)) inline int near_offset(const SweepCtx& c, const Ref& i, const Ref& j) {
-  auto axis = [&](int d, int L) {
-    d += d > c.h ? -L : 0;
-    d += d < -c.h ? L : 0;
-    return d;
-  };
-  const int dx = axis(i.x - j.x, c.L1), dy = axis(i.y - j.y, c.L2), dz = axis(i.z - j.z, c.L3);
-  const bool in = dx >= -c.h && dx <= c.h && dy >= -c.h && dy <= c.h && dz >= -c.h && dz <= c.h;
-  return in ? (dx * c.P2 + dy) * c.P3 + dz : kNoPatch;
+// Sum over the kG lanes of a group (4: a quad, 16: a row, 64: the wave);
+// every lane of the group ends with it.
+template <int kG>
+__device__ __attribute__((always_inline)) inline double group_lanes_sum_f64(double v) {
+  if constexpr (kG == 4) {
+    v += dpp_f64<0xB1>(v);
+    v += dpp_f64<0x4E>(v);
+    return v;
+  } else if constexpr (kG == 16) {
+    v += dpp_f64<0x128>(v);
+    return octet_sum_f64(v);
+  } else {
+    return wave_sum_f64(v);
+  }
 }
 
 }  // namespace
+
+// A rejected move in the block's list of energy changes: a NaN that no
+// accepted change can be (its comparison with the threshold fails).
+constexpr long long kRejected = 0x7FF8DEAD00000000ll;
 
 // kBM: basis functions, one less than the species (1, 2, 3).  kP: moves that
 // a lane group evaluates per round.  kTrkLds: the tracker is held in LDS,
@@ -93,22 +114,32 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
     const ChainParams* __restrict__ params, ChainState* __restrict__ states, const ModelDev* __restrict__ models,
     int8_t* __restrict__ occ_pool, uint16_t* __restrict__ trk_pool, const int32_t* __restrict__ chain_order,
     const int64_t* __restrict__ n_moves, uint32_t* __restrict__ accept_log, int64_t log_words, int64_t time_limit) {
-  static_assert(kG == 16 || kG == 64, "a row or the whole wave evaluates a move");
+  static_assert(kG == 4 || kG == 16 || kG == 64, "a quad, a row or the whole wave evaluates a move");
   constexpr int kS = kBM + 1;
   constexpr int kQ = kBM == 1 ? 6 : (kBM == 2 ? 5 : 4);  // members per patch (patch_members)
   constexpr int kPer = 64 / kG;                           // moves a wave evaluates side by side
   constexpr int kK = kW * kP * kPer;                       // moves per round
-  static_assert(kK == 8 || (kK == 16 && kW == 4), "rounds of 8, or of 16 on four waves");
+  static_assert(kK == (kG == 64 ? 8 : 16), "rounds of 16, or of 8 with a wave per move");
+  constexpr bool kNear = kCanonical && kG != 64;  // member weights by offset in LDS
+  constexpr int kSlots = kG * kR;
   constexpr int kThreads = 64 * kW;
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ double dphi_tab[kS * kS * kBM];  // [(old*S+new)*B + d]
   __shared__ double dsingle_tab[kS * kS];
   __shared__ double phi_tab[kBM * kS];
-  __shared__ uint4 mv_a[64];  // canonical: p_i, p_j, offset of i seen from j, a | b << 8; SGC: p, cell, image, species offset
-  __shared__ uint4 mv_b[kCanonical ? 64 : 1];  // canonical: cell_i, cell_j, image_i, image_j
-  __shared__ uint2 mv_s[kCanonical ? 64 : 1];  // canonical: site_i | site_j << 16, slot_a | slot_b << 16
-  __shared__ double red[2][kK];                // sums of the round's moves, by parity
-  __shared__ uint16_t conf_l[kK];               // rounds of 16: earlier moves that affect each
+  // the round's moves, one copy per wave (no barrier between filling and
+  // reading them)
+  __shared__ uint4 slot_a[kW][kK];  // canonical: p_i, p_j, place of i seen from j, a | b << 8 | lane << 16
+                                    // SGC: p, cell, image, species offset | lane << 16
+  __shared__ uint4 slot_b[kW][kCanonical ? kK : 1];  // canonical: cell_i, cell_j, image_i, image_j
+  __shared__ uint2 slot_s[kW][kCanonical ? kK : 1];  // canonical: site_i | site_j << 16, tracker slots alike
+  __shared__ double2 slot_t[kW][kK];                 // accept below, reject above
+  __shared__ double red[2][kK];                      // sums of the round's moves, by parity
+  __shared__ uint64_t conf_l[2];                     // rounds of 16 on several waves: the pair bits
+  __shared__ double de_l[64];                        // the block's accepted energy changes (kRejected: none)
+  __shared__ uint32_t on_l[kCanonical ? 1 : 64];     // SGC: species change of each, old | new << 8
+  __shared__ uint8_t axis_tab[3][256];               // pair test, see pair_hits
+  __shared__ uint8_t mask_tab[608];
   __shared__ int stop_flag[2];
   const int chain = chain_order[blockIdx.x];
   const int tid = int(threadIdx.x);
@@ -138,9 +169,11 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
   c.trans = nullptr;
   const uint64_t im0 = m.imask[0], im1 = m.imask[1];
   const int occ_bytes = m.pdims[0] * c.P2 * c.P3;
-  const PatchLayout L = patch_layout(occ_bytes, kCanonical && kTrkLds ? N : 0, m.ptab_size);
+  const PatchLayout L =
+      patch_layout(occ_bytes, kCanonical && kTrkLds ? N : 0, m.ptab_size, kNear ? kNearCells * kSlots : 0);
   uint8_t* occ = reinterpret_cast<uint8_t*>(lds);
   double* tab = reinterpret_cast<double*>(lds + L.tab);
+  [[maybe_unused]] uint8_t* near_w = lds + L.near;
   uint16_t* gtrk = trk_pool + pp->trk_off;
   uint16_t* trk = kTrkLds ? reinterpret_cast<uint16_t*>(lds + L.trk) : gtrk;
 
@@ -176,6 +209,36 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
     }
     dsingle_tab[i] = ds;
   }
+  // pair test: a change at cell a reaches a flip at cell b when a - b, wrapped,
+  // is an offset of the model's interaction mask.  With cells packed a byte
+  // per axis, a + L - b has the axes' differences in its bytes (L <= 127); each
+  // axis' table gives its share of the mask index, or 200 outside the halo,
+  // and the mask table ends in zeros.
+  {
+    const int w = 2 * c.h + 1;
+    for (int i = tid; i < 3 * 256; i += kThreads) {
+      const int ax = i >> 8, Ld = ax == 0 ? c.L1 : (ax == 1 ? c.L2 : c.L3);
+      int e = (i & 255) - Ld + c.h;
+      e += e < 0 ? Ld : 0;
+      e -= e >= Ld ? Ld : 0;
+      axis_tab[ax][i & 255] = uint8_t(e >= 0 && e < w ? e * (ax == 0 ? w * w : (ax == 1 ? w : 1)) : 200);
+    }
+    for (int i = tid; i < 608; i += kThreads)
+      mask_tab[i] = i < 128 ? uint8_t(((i < 64 ? im0 : im1) >> (i & 63)) & 1u) : 0;
+  }
+  if constexpr (kNear)
+    for (int i = tid; i < kNearCells * kSlots; i += kThreads) near_w[i] = 0;
+  // slots that a round does not fill hold a move from before; at first the
+  // cell (0, 0, 0)
+  if (lane < kK) {
+    const uint32_t p0 = uint32_t((c.h * c.P2 + c.h) * c.P3 + c.h);
+    slot_a[wave][lane] = kCanonical ? uint4{p0, p0, uint32_t(kNearCells - 1), 0} : uint4{p0, 0, p0, 0};
+    if constexpr (kCanonical) {
+      slot_b[wave][lane] = uint4{0, 0, p0, p0};
+      slot_s[wave][lane] = uint2{0, 0};
+    }
+    slot_t[wave][lane] = double2{0.0, 0.0};
+  }
   // this lane's patches (past the last: table 0, all zeros)
   int mo[kR][kQ], base[kR], wl[kR];
   {
@@ -192,7 +255,22 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
     }
   }
   __syncthreads();
+  if constexpr (kNear) {
+    // a swap's second flip sees its first site changed: the index weight of
+    // the member at each offset, per patch slot
+    const int w = 2 * c.h + 1, shift = (c.h * c.P2 + c.h) * c.P3 + c.h;
+    for (int i = tid; i < m.n_patch * kQ; i += kThreads) {
+      const int it = i / kQ, q = i - it * kQ, off = m.patches[it].m[q];
+      if (off == 0) continue;  // an unused place
+      int weight = q == kQ - 1 ? int(m.patches[it].w_last) : 1;
+      for (int t = 0; q != kQ - 1 && t < q; ++t) weight *= kS;
+      const int lin = off + shift, x = lin / (c.P2 * c.P3), rem = lin - x * c.P2 * c.P3, y = rem / c.P3, z = rem - y * c.P3;
+      near_w[((x * w + y) * w + z) * kSlots + it] = uint8_t(weight);
+    }
+    __syncthreads();
+  }
   const double dphi01 = dphi_tab[kBM], dphi10 = dphi_tab[kS * kBM];  // two species: 0 -> 1 and 1 -> 0
+  [[maybe_unused]] const double dsin01 = dsingle_tab[1], dsin10 = dsingle_tab[kS];
 
   double energy = states[chain].energy;
   const uint64_t t0 = states[chain].moves_done;
@@ -218,7 +296,6 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
     for (int d = 0; d < kBM; ++d) sing[d] = wave_sum_f64(part[d]) / double(N);
   }
   const double kT = pp->kT;
-  const double inv_kT = 1.0 / kT;
   const uint64_t seed = pp->seed, uid = pp->uid;
   const uint32_t np = uint32_t(pp->n_present);
   const uint32_t present_pk = pp->present_pk;
@@ -232,46 +309,56 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
   // ordered by barriers
   auto own_order = [] { __atomic_signal_fence(__ATOMIC_SEQ_CST); };
 
-  // one flip's table sum over this lane's patches around padded site p: the
-  // slices' sums, or with dphi the change; `off`: this padded offset holds a
-  // species `ds` higher than the lattice says
-  auto flip = [&](int p, const double (&dphi)[kBM], bool patched, int off, int ds) {
-    int idx[kR];
+  // One flip over this lane's patches, in phases so that the loads of a
+  // round go out together: member species, table indexes, entries, sum (two
+  // species: plain, else the change for dphi).
+  const int sub = lane & (kG - 1);
+  typedef uint32_t Members[kR][kQ];
+  typedef double Entries[kR][kBM];
+  auto gather = [&](int p, Members& s) {
+#pragma unroll
+    for (int k = 0; k < kR; ++k)
+#pragma unroll
+      for (int q = 0; q < kQ; ++q) s[k][q] = occ[p + mo[k][q]];
+  };
+  auto index = [&](const Members& s, int (&idx)[kR]) {
 #pragma unroll
     for (int k = 0; k < kR; ++k) {
-      uint32_t s[kQ];
+      uint32_t v = s[k][kQ - 2];
 #pragma unroll
-      for (int q = 0; q < kQ; ++q) s[q] = occ[p + mo[k][q]];
-      uint32_t v = s[kQ - 2];
-#pragma unroll
-      for (int q = kQ - 3; q >= 0; --q) v = v * uint32_t(kS) + s[q];
-      idx[k] = int(v + __umul24(s[kQ - 1], uint32_t(wl[k])));
+      for (int q = kQ - 3; q >= 0; --q) v = v * uint32_t(kS) + s[k][q];
+      idx[k] = int(v + __umul24(s[k][kQ - 1], uint32_t(wl[k])));
     }
-    if (patched) {
+  };
+  // The member at padded offset `lin` holds a species `ds` higher than the
+  // lattice says (lin 0: no member).
+  auto index_shift = [&](int lin, int ds, int (&idx)[kR]) {
 #pragma unroll
-      for (int k = 0; k < kR; ++k) {
-        int w = mo[k][kQ - 1] == off ? wl[k] : 0, pw = 1;
+    for (int k = 0; k < kR; ++k) {
+      int w = mo[k][kQ - 1] == lin ? wl[k] : 0, pw = 1;
 #pragma unroll
-        for (int q = 0; q < kQ - 1; ++q) {
-          w = mo[k][q] == off ? pw : w;
-          pw *= kS;
-        }
-        idx[k] += w * ds;
+      for (int q = 0; q < kQ - 1; ++q) {
+        w = mo[k][q] == lin ? pw : w;
+        pw *= kS;
       }
+      idx[k] += lin != 0 ? w * ds : 0;
     }
-    double g[kR][kBM];
+  };
+  auto entries = [&](const int (&idx)[kR], Entries& g) {
 #pragma unroll
     for (int k = 0; k < kR; ++k) {
       const double* t = tab + (base[k] + kBM * idx[k]);
       if constexpr (kBM == 2) {
         const dbl2_t two = load_pair(t);
         g[k][0] = two.x;
-        g[k][1] = two.y;
+        g[k][kBM - 1] = two.y;
       } else {
 #pragma unroll
         for (int d = 0; d < kBM; ++d) g[k][d] = t[d];
       }
     }
+  };
+  auto total = [&](const Entries& g, const double (&dphi)[kBM]) {
     double v = 0.0;
 #pragma unroll
     for (int k = 0; k < kR; ++k) {
@@ -283,6 +370,64 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
       }
     }
     return v;
+  };
+  // keeps the scheduler from moving a phase's loads behind the waits of the
+  // phase before
+  auto phase = [] { __builtin_amdgcn_sched_barrier(0); };
+
+  const uint32_t bias = uint32_t(c.L1) | (uint32_t(c.L2) << 8) | (uint32_t(c.L3) << 16);
+  struct Axes {
+    uint32_t x, y, z;
+  };
+  auto axes = [&](uint32_t cell_a, uint32_t cell_b) {
+    const uint32_t d = cell_a + bias - cell_b;
+    return Axes{axis_tab[0][d & 255u], axis_tab[1][(d >> 8) & 255u], axis_tab[2][d >> 16]};
+  };
+  // padded offset of a cell of the halo box
+  auto offset_of = [&](uint32_t cell) {
+    const uint32_t w = uint32_t(2 * c.h + 1), x = cell / (w * w), r = cell - x * w * w, y = r / w, z = r - y * w;
+    return ((int(x) - c.h) * c.P2 + int(y) - c.h) * c.P3 + int(z) - c.h;
+  };
+  const uint32_t inv23 = 0xFFFFFFFFu / uint32_t(c.L23) + 1u, inv3 = 0xFFFFFFFFu / uint32_t(c.L3) + 1u;
+  // image `im` of the site with image word w: an image that does not exist
+  // repeats another one, so every lane may write
+  const int im = lane & 7;
+  const int step_x = (im & 1) ? c.DX : 0, step_y = (im & 2) ? c.DY : 0, step_z = (im & 4) ? c.DZ : 0;
+  auto image = [&](uint32_t w) {
+    const int ex = int(w << 10) >> 30, ey = int(w << 8) >> 30, ez = int(w << 6) >> 30;
+    return int(w & 0xFFFFFu) + __mul24(ex, step_x) + __mul24(ey, step_y) + __mul24(ez, step_z);
+  };
+  uint4* const my_a = slot_a[wave];
+  uint4* const my_b = slot_b[wave];
+  uint2* const my_s = slot_s[wave];
+  double2* const my_t = slot_t[wave];
+  const int kd = lane & (kK - 1);  // the slot this lane decides
+  // the first slot it commits (four waves: sites i and j of four moves a wave)
+  const int ck = kK == 8 || kW == 1 ? lane >> 3 : (kW == 2 ? 8 * wave + (lane >> 3) : 4 * wave + (lane >> 4));
+  // Pairs (a, b), a < b, of the round that a lane tests.  Rounds of 8: one
+  // byte per b.  Rounds of 16: two words of four 16-bit rows; row r = 1..8
+  // holds b = r (r pairs), then b = 16 - r (16 - r pairs).
+  int pair_a[2], pair_b[2], conf_word = 0, conf_shift = 0;
+  uint32_t conf_mask = (1u << kd) - 1u;
+  if constexpr (kK == 8) {
+    pair_a[0] = pair_a[1] = lane & 7;
+    pair_b[0] = pair_b[1] = lane >> 3;
+  } else {
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const int r = 4 * (kW > 1 ? (wave & 1) : v) + (lane >> 4) + 1, j = lane & 15;
+      pair_b[v] = j < r ? r : 16 - r;
+      pair_a[v] = j < r ? j : j - r;
+    }
+    const int r = kd <= 8 ? (kd > 0 ? kd : 1) : 16 - kd;
+    conf_word = (r - 1) >> 2;
+    conf_shift = 16 * ((r - 1) & 3) + (kd <= 8 ? 0 : r);
+  }
+  // two packed tracker slots each: not zero when some slot is in both
+  // (a zero half of v borrows into its own top bit of (v - 1) & ~v)
+  auto shared_half = [](uint32_t s, uint32_t t) {
+    const uint32_t x = s ^ t, y = s ^ __builtin_rotateright32(t, 16);
+    return (((x - 0x00010001u) & ~x) | ((y - 0x00010001u) & ~y)) & 0x80008000u;
   };
 
   uint32_t rnd = 0;
@@ -302,240 +447,328 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
     }
     // lane l decodes move blk0 + l
     const Philox4 blk = philox4x64_10(t0 + uint64_t(blk0) + uint64_t(lane), 0, 0, 0, seed, uid);
-    const double log_u = log(unit_double(blk.w3));
     const int n_in = int(nmov - blk0 < 64 ? nmov - blk0 : 64);
-    uint32_t v_old = 0, v_new = 0;  // canonical: species a and b
-    int v_ta = 0, v_tb = 0;         // canonical: tracker slots
-    int v_p = 0;                    // SGC: padded site
-    uint32_t v_off = 0;             // SGC: offset of the new species
-    // canonical: the sites now in the move's slots, to registers and LDS
-    auto look_up = [&] {
-      const int si = trk[v_ta], sj = trk[v_tb];
-      const Ref ri = ref_of<true>(c, si), rj = ref_of<true>(c, sj);
-      const uint32_t ci = uint32_t(ri.x) | (uint32_t(ri.y) << 8) | (uint32_t(ri.z) << 16);
-      const uint32_t cj = uint32_t(rj.x) | (uint32_t(rj.y) << 8) | (uint32_t(rj.z) << 16);
-      mv_a[lane] = uint4{uint32_t(ri.p), uint32_t(rj.p), uint32_t(near_offset(c, ri, rj)), v_old | (v_new << 8)};
-      mv_b[lane] = uint4{ci, cj, image_word<true>(c, ri), image_word<true>(c, rj)};
-      mv_s[lane] = uint2{uint32_t(si) | (uint32_t(sj) << 16), uint32_t(v_ta) | (uint32_t(v_tb) << 16)};
+    // Metropolis test of the reference (montecarlo.py:950-956): accept when
+    // dE < 0 or u <= exp(-dE / kT).  dE against -kT log u decides it outside a
+    // margin far above the rounding of log and exp; inside, exp is evaluated.
+    const double t_u = -kT * log(unit_double(blk.w3));
+    const double margin = 2e-12 * (kT + t_u);
+    const double2 thr{t_u - margin, t_u + margin};
+    uint4 v_a{0, 0, 0, 0}, v_b{0, 0, 0, 0};
+    uint2 v_s{0, 0};
+    // padded index, packed cell and image word of a site
+    auto place = [&](uint32_t site, uint32_t& p, uint32_t& cell, uint32_t& img) {
+      const uint32_t x = div16(site, inv23), r = site - __umul24(x, uint32_t(c.L23));
+      const uint32_t y = div16(r, inv3), z = r - __umul24(y, uint32_t(c.L3));
+      p = __umul24(__umul24(x + c.h, uint32_t(c.P2)) + y + c.h, uint32_t(c.P3)) + z + c.h;
+      cell = x | (y << 8) | (z << 16);
+      Ref ref;
+      ref.p = int(p);
+      ref.x = int(x);
+      ref.y = int(y);
+      ref.z = int(z);
+      img = image_word<true>(c, ref);
+    };
+    // canonical: the sites in the move's tracker slots
+    auto set_sites = [&](uint32_t si, uint32_t sj) {
+      place(si, v_a.x, v_b.x, v_b.z);
+      place(sj, v_a.y, v_b.y, v_b.w);
+      v_s.x = si | (sj << 16);
+      const Axes at = axes(v_b.x, v_b.y);
+      const uint32_t cell = at.x + at.y + at.z;  // of i in the halo box around j; 125 and more: outside
+      v_a.z = kNear ? (cell < uint32_t(kNearCells - 1) ? cell : uint32_t(kNearCells - 1))
+                    : (cell < uint32_t(kNearCells - 1) ? uint32_t(offset_of(cell)) : 0u);
     };
     if constexpr (kCanonical) {
       const uint32_t ia = bounded32(uint32_t(blk.w0 >> 32), np);
       uint32_t ib = ia + 1u + bounded32(uint32_t(blk.w0), np - 1u);
       ib -= ib >= np ? np : 0u;
-      v_old = (present_pk >> (4u * ia)) & 15u;
-      v_new = (present_pk >> (4u * ib)) & 15u;
-      v_ta = unpack16(seg_lo, seg_hi, ia) + int(bounded64(blk.w1, uint64_t(unpack16(cnt_lo, cnt_hi, ia))));
-      v_tb = unpack16(seg_lo, seg_hi, ib) + int(bounded64(blk.w2, uint64_t(unpack16(cnt_lo, cnt_hi, ib))));
-      look_up();
+      v_a.w = ((present_pk >> (4u * ia)) & 15u) | (((present_pk >> (4u * ib)) & 15u) << 8) | (uint32_t(lane) << 16);
+      const int ta = unpack16(seg_lo, seg_hi, ia) + int(bounded64(blk.w1, uint64_t(unpack16(cnt_lo, cnt_hi, ia))));
+      const int tb = unpack16(seg_lo, seg_hi, ib) + int(bounded64(blk.w2, uint64_t(unpack16(cnt_lo, cnt_hi, ib))));
+      v_s.y = uint32_t(ta) | (uint32_t(tb) << 16);
+      set_sites(trk[ta], trk[tb]);
     } else {
       const Ref r = ref_of<true>(c, int(bounded64(blk.w1, uint64_t(N))));
-      v_p = r.p;
-      v_off = bounded32(uint32_t(blk.w0), uint32_t(kS - 1));
-      mv_a[lane] = uint4{uint32_t(r.p), uint32_t(r.x) | (uint32_t(r.y) << 8) | (uint32_t(r.z) << 16),
-                         image_word<true>(c, r), v_off};
+      v_a = uint4{uint32_t(r.p), uint32_t(r.x) | (uint32_t(r.y) << 8) | (uint32_t(r.z) << 16), image_word<true>(c, r),
+                  bounded32(uint32_t(blk.w0), uint32_t(kS - 1)) | (uint32_t(lane) << 16)};
     }
-    // every wave writes the same values; the slowest wave may still be
-    // reading the last block's, which it no longer uses (see the round's end)
-    if constexpr (kW > 1)
-      __syncthreads();
-    else
-      own_order();
-    uint64_t acc_bits = 0;
-    double de_made = 0.0;           // this lane's move: its energy change if accepted
-    uint32_t o_made = 0, n_made = 0;  // SGC: its species change (equal: rejected)
-    int l0 = 0;
-    while (l0 < n_in) {
-      const int n = n_in - l0 < kK ? n_in - l0 : kK;
-      auto at = [&](int k) { return l0 + k < 63 ? l0 + k : 63; };
-      // SGC: the species at this lane's own site
-      uint32_t o_l = v_old, n_l = v_new;
-      if constexpr (!kCanonical) {
-        o_l = occ[v_p];
-        n_l = o_l + 1u + v_off;
-        n_l -= n_l >= uint32_t(kS) ? uint32_t(kS) : 0u;
-      }
-      // ---- this wave's moves
-      double part[kP];
-#pragma unroll
-      for (int t = 0; t < kP; ++t) {
-        const int k = (wave * kP + t) * kPer + (kG == 64 ? 0 : lane / kG);
-        const uint4 a = mv_a[at(k)];
-        double dphi[kBM];
+    if (kW == 1 || wave == 0) {
+      de_l[lane] = __longlong_as_double(kRejected);
+      if constexpr (!kCanonical) on_l[lane] = 0;
+    }
+    uint64_t open = n_in < 64 ? (uint64_t(1) << n_in) - 1u : ~uint64_t(0);  // moves not made yet
+    while (open != 0) {
+      // ---- the first kK open moves fill the slots
+      const int rank = int(__builtin_amdgcn_mbcnt_hi(uint32_t(open >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(open), 0)));
+      const bool in = ((open >> lane) & 1u) != 0 && rank < kK;
+      const int n_open = int(__builtin_popcountll(open));
+      const int n = n_open < kK ? n_open : kK;
+      if (in) {
+        my_a[rank] = v_a;
+        my_t[rank] = thr;
         if constexpr (kCanonical) {
-          const int o = int(a.w & 255u), nw = int(a.w >> 8);
-#pragma unroll
-          for (int d = 0; d < kBM; ++d) dphi[d] = kBM == 1 ? 0.0 : dphi_tab[(o * kS + nw) * kBM + d];
-          const bool any = __builtin_amdgcn_ballot_w64(int(a.z) != kNoPatch) != 0;
-          const double vi = flip(int(a.x), dphi, false, 0, 0);
-          // the swap's second flip sees site i already changed (ce_updater.cpp:845-852)
-          const double vj = flip(int(a.y), dphi, any, int(a.z), nw - o);
-          part[t] = vi - vj;
-        } else {
-          if constexpr (kBM > 1) {
-            const int o = occ[a.x];
-            int nw = o + 1 + int(a.w);
-            nw -= nw >= kS ? kS : 0;
-#pragma unroll
-            for (int d = 0; d < kBM; ++d) dphi[d] = dphi_tab[(o * kS + nw) * kBM + d];
-          } else {
-            dphi[0] = 0.0;
-          }
-          part[t] = flip(int(a.x), dphi, false, 0, 0);
+          my_b[rank] = v_b;
+          my_s[rank] = v_s;
         }
       }
-      // ---- which earlier moves of the round affect which: lane (b, a)
-      constexpr int kA = kK == 16 ? 16 : 8;
-      const int pb = lane / kA + (kK == 16 ? 4 * wave : 0), pa = lane & (kA - 1);
-      bool hit = false;
-      int com_i = -1, com_j = -1;  // this lane's commit: padded images of sites i and j
-      uint32_t com_o = 0, com_n = 0, com_sites = 0, com_slots = 0;
-      const int ck = kK == 16 ? 4 * wave + (lane >> 4) : lane >> 3;  // the move it commits
-      const int cim = lane & 7;
+      // canonical: the tracker slots of the round's moves may have got other
+      // sites since they were read
+      uint32_t now_i = 0, now_j = 0;
       if constexpr (kCanonical) {
-        const uint4 vb = mv_b[at(pb)], va = mv_b[at(pa)];
-        const uint32_t slb = mv_s[at(pb)].y, sla = mv_s[at(pa)].y;
-        const uint32_t ta_a = sla & 0xFFFFu, tb_a = sla >> 16, ta_b = slb & 0xFFFFu, tb_b = slb >> 16;
-        hit = cells_interact(va.x, vb.x, c, im0, im1) || cells_interact(va.x, vb.y, c, im0, im1) ||
-              cells_interact(va.y, vb.x, c, im0, im1) || cells_interact(va.y, vb.y, c, im0, im1) || ta_a == ta_b ||
-              ta_a == tb_b || tb_a == ta_b || tb_a == tb_b;
-        const uint4 cb = mv_b[at(ck)];
-        const uint2 cs = mv_s[at(ck)];
-        const uint32_t on = mv_a[at(ck)].w;
-        com_sites = cs.x;
-        com_slots = cs.y;
-        com_o = on & 255u;
-        com_n = on >> 8;
-        if constexpr (kK == 16) {
-          com_i = image_of(c, (lane & 8) ? cb.w : cb.z, cim);
-        } else {
-          com_i = image_of(c, cb.z, cim);
-          com_j = image_of(c, cb.w, cim);
-        }
-      } else {
-        hit = cells_interact(mv_a[at(pa)].y, mv_a[at(pb)].y, c, im0, im1);
-        const uint4 ca = mv_a[at(ck)];
-        com_i = image_of(c, ca.z, cim);
-        if (kK == 16 && (lane & 8)) com_i = -1;
-        com_n = occ[ca.x] + 1u + ca.w;
-        com_n -= com_n >= uint32_t(kS) ? uint32_t(kS) : 0u;
+        now_i = trk[v_s.y & 0xFFFFu];
+        now_j = trk[v_s.y >> 16];
       }
-      const uint64_t conf = __builtin_amdgcn_ballot_w64(hit && pa < pb);
+      own_order();
+      // ---- the slots: what this lane evaluates, tests, commits and decides
+      constexpr int kPairs = kK == 16 && kW == 1 ? 2 : 1;
+      constexpr int kCom = kK == 16 && kW == 1 ? 2 : 1;
+      uint4 ev[kP];
+      uint2 pa[kPairs], pb[kPairs];  // cells (canonical: i, j)
+      uint32_t sa[kPairs], sb[kPairs];
+      uint4 ca[kCom];
+      uint2 cimg[kCom], cs[kCom];
+#pragma unroll
+      for (int t = 0; t < kP; ++t) ev[t] = my_a[(wave * kP + t) * kPer + (kG == 64 ? 0 : lane / kG)];
+#pragma unroll
+      for (int v = 0; v < kPairs; ++v) {
+        if constexpr (kCanonical) {
+          pa[v] = *reinterpret_cast<const uint2*>(&my_b[pair_a[v]]);
+          pb[v] = *reinterpret_cast<const uint2*>(&my_b[pair_b[v]]);
+          sa[v] = my_s[pair_a[v]].y;
+          sb[v] = my_s[pair_b[v]].y;
+        } else {
+          pa[v].x = my_a[pair_a[v]].y;
+          pb[v].x = my_a[pair_b[v]].y;
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < kCom; ++v) {
+        ca[v] = my_a[ck + 8 * v];
+        if constexpr (kCanonical) {
+          cimg[v] = reinterpret_cast<const uint2*>(&my_b[ck + 8 * v])[1];
+          cs[v] = my_s[ck + 8 * v];
+        }
+      }
+      const uint4 da = my_a[kd];
+      const double2 dt = my_t[kd];
+      if constexpr (kCanonical) {
+        const bool stale = in && (now_i | (now_j << 16)) != v_s.x;
+        if (__builtin_amdgcn_ballot_w64(stale) != 0) {
+          set_sites(now_i, now_j);
+          continue;  // nothing was done yet: fill the slots again
+        }
+      }
+      phase();
+      // ---- members of this wave's moves; cell differences of the pairs
+      double part[kP];
+      // flips whose loads go out together: all of this wave's, or one after the
+      // other where their members and entries would overflow the registers
+      constexpr int kF = kCanonical ? 2 : 1;  // flips per move
+      constexpr int kFlips = kP * kF;
+      constexpr int kT = kFlips * kR * kQ <= 100 ? kFlips : 1;
+      Axes ax[kPairs][kCanonical ? 4 : 1];
+      uint32_t c_o[kCom], d_s = 0;
+      auto other_loads = [&] {
+#pragma unroll
+        for (int v = 0; v < kPairs; ++v) {
+          ax[v][0] = axes(pa[v].x, pb[v].x);
+          if constexpr (kCanonical) {
+            ax[v][1] = axes(pa[v].x, pb[v].y);
+            ax[v][2] = axes(pa[v].y, pb[v].x);
+            ax[v][3] = axes(pa[v].y, pb[v].y);
+          }
+        }
+        if constexpr (!kCanonical) {
+#pragma unroll
+          for (int v = 0; v < kCom; ++v) c_o[v] = occ[ca[v].x];
+          d_s = occ[da.x];
+        }
+      };
+      uint32_t hit[kPairs];
+      auto other_masks = [&] {
+#pragma unroll
+        for (int v = 0; v < kPairs; ++v) {
+          hit[v] = 0;
+#pragma unroll
+          for (int u = 0; u < (kCanonical ? 4 : 1); ++u) hit[v] |= mask_tab[ax[v][u].x + ax[v][u].y + ax[v][u].z];
+        }
+      };
+#pragma unroll
+      for (int f0 = 0; f0 < kFlips; f0 += kT) {
+        Members mem[kT];
+        uint32_t near[kT][kNear ? kR : 1];
+        uint32_t own[kT];
+#pragma unroll
+        for (int u = 0; u < kT; ++u) {
+          const uint4 e = ev[(f0 + u) / kF];
+          const bool second = kCanonical && (f0 + u) % 2 == 1;  // site j of a swap
+          if constexpr (!kCanonical && kBM > 1) own[u] = occ[e.x];
+          gather(int(second ? e.y : e.x), mem[u]);
+          if (kNear && second)
+#pragma unroll
+            for (int k = 0; k < kR; ++k) near[u][kNear ? k : 0] = near_w[__umul24(e.z, uint32_t(kSlots)) + sub + kG * k];
+        }
+        if (f0 == 0) other_loads();
+        phase();
+        Entries g[kT];
+        double dphi[kT][kBM];
+#pragma unroll
+        for (int u = 0; u < kT; ++u) {
+          const uint4 e = ev[(f0 + u) / kF];
+          const bool second = kCanonical && (f0 + u) % 2 == 1;
+          int idx[kR];
+          index(mem[u], idx);
+          int o = int(e.w & 255u), nw = int((e.w >> 8) & 255u);
+          if (second) {
+            // the swap's second flip sees site i already changed (ce_updater.cpp:845-852)
+            if constexpr (kNear) {
+#pragma unroll
+              for (int k = 0; k < kR; ++k) idx[k] += __mul24(int(near[u][k]), nw - o);
+            } else if (e.z != 0u) {
+              index_shift(int(e.z), nw - o, idx);
+            }
+          }
+          entries(idx, g[u]);
+          if constexpr (kBM > 1) {
+            if constexpr (!kCanonical) {
+              nw = int(own[u]) + 1 + o;
+              o = int(own[u]);
+              nw -= nw >= kS ? kS : 0;
+            }
+#pragma unroll
+            for (int d = 0; d < kBM; ++d) dphi[u][d] = dphi_tab[(o * kS + nw) * kBM + d];
+          } else {
+            dphi[u][0] = 0.0;
+          }
+        }
+        if (f0 == 0) other_masks();
+        phase();
+#pragma unroll
+        for (int u = 0; u < kT; ++u) {
+          const double v = total(g[u], dphi[u]);
+          const int t = (f0 + u) / kF;
+          if (kCanonical && (f0 + u) % 2 == 1)
+            part[t] -= v;
+          else
+            part[t] = v;
+        }
+      }
+      // ---- which earlier moves of the round reach which
+      uint64_t conf[2] = {0, 0};
+#pragma unroll
+      for (int v = 0; v < kPairs; ++v) {
+        if constexpr (kCanonical) hit[v] |= shared_half(sa[v], sb[v]);
+        conf[v] = __builtin_amdgcn_ballot_w64(hit[v] != 0);
+      }
+      if constexpr (kK == 16 && kW > 1)
+        if (wave < 2 && lane == 0) conf_l[wave] = conf[0];
+      // the slot this lane decides
+      uint32_t d_o = da.w & 255u, d_n = (da.w >> 8) & 255u;
+      if constexpr (!kCanonical) {
+        d_n = d_s + 1u + d_o;
+        d_o = d_s;
+        d_n -= d_n >= uint32_t(kS) ? uint32_t(kS) : 0u;
+      }
       // ---- sums of the round's moves
       double* rs = red[rnd & 1u];
 #pragma unroll
       for (int t = 0; t < kP; ++t) {
-        const double s = kG == 16 ? row_sum_f64(part[t]) : wave_sum_f64(part[t]);
+        const double s = group_lanes_sum_f64<kG>(part[t]);
         if ((lane & (kG - 1)) == 0) rs[(wave * kP + t) * kPer + (kG == 64 ? 0 : lane / kG)] = s;
-      }
-      if constexpr (kK == 16) {
-        if (lane < 4) conf_l[4 * wave + lane] = uint16_t(conf >> (16 * lane));
       }
       if constexpr (kW > 1)
         __syncthreads();
       else
         own_order();
-      // ---- every lane decides the move it decoded
-      const int r = lane - l0;
-      const bool valid = r >= 0 && r < n;
-      const double tot = rs[valid ? r : 0];
-      uint32_t conf_r = 0;
-      if constexpr (kK == 16) conf_r = conf_l[valid ? r : 0];
+      // ---- decide: lane l slot l mod kK, so that a ballot repeats the round's verdicts
+      const double tot = rs[kd];
+      // earlier moves of the round that reach the slot's
+      uint32_t conf_d;
+      if constexpr (kK == 8) {
+        conf_d = uint32_t(conf[0] >> (8 * kd)) & conf_mask;
+      } else {
+        const uint64_t word = kW > 1 ? conf_l[conf_word] : (conf_word ? conf[1] : conf[0]);
+        conf_d = uint32_t(word >> conf_shift) & conf_mask;
+      }
       double dE;
       if constexpr (kBM == 1) {
-        const double d0 = o_l == 0 ? dphi01 : dphi10;
-        dE = kCanonical ? __dmul_rn(d0, tot) : fma(d0, tot, dsingle_tab[o_l == 0 ? 1 : kS]);
+        const double d0 = d_o == 0 ? dphi01 : dphi10;
+        dE = kCanonical ? __dmul_rn(d0, tot) : fma(d0, tot, d_o == 0 ? dsin01 : dsin10);
       } else {
-        dE = kCanonical ? tot : tot + dsingle_tab[int(o_l) * kS + int(n_l)];
+        dE = kCanonical ? tot : tot + dsingle_tab[int(d_o) * kS + int(d_n)];
       }
-      // the Metropolis test of the sweep kernel (ce_sweep.h)
-      const double x = -dE * inv_kT;
-      const double margin = 1e-12 * (1.0 + fabs(x));
-      int verdict = (dE < 0.0 || log_u < x - margin) ? 1 : (log_u > x + margin ? 0 : 2);
-      if (valid && verdict == 2) verdict = int(unit_double(blk.w3) <= exp(-dE / kT));
-      const uint64_t acc = __builtin_amdgcn_ballot_w64(valid && verdict == 1) >> l0;  // bit k: move k of the round
-      int stop = n;
-      if constexpr (kK == 16) {
-        const uint64_t hits = __builtin_amdgcn_ballot_w64(valid && (conf_r & uint32_t(acc)) != 0) >> l0;
-        if (hits != 0) stop = int(__builtin_ctzll(hits));
-      } else {
-        uint32_t dup = uint32_t(acc) & 0xFFu;
-        dup |= dup << 8;
-        dup |= dup << 16;
-        const uint64_t hits = conf & ((uint64_t(dup) << 32) | dup);  // byte b: accepted moves that affect move b
-        if (hits != 0) {
-          const int first = int(__builtin_ctzll(hits)) >> 3;
-          stop = first < stop ? first : stop;
-        }
+      const bool valid = kd < n;
+      bool yes = dE < dt.x;
+      if (__builtin_amdgcn_ballot_w64(valid && !yes && !(dE > dt.y)) != 0) {
+        const double u = unit_double(__shfl(blk.w3, int(da.w >> 16), 64));
+        if (!yes && !(dE > dt.y)) yes = dE < 0.0 || u <= exp(-dE / kT);
       }
-      const uint32_t com = uint32_t(acc) & ((1u << stop) - 1u);
+      const uint32_t acc = uint32_t(__builtin_amdgcn_ballot_w64(valid && yes)) & ((1u << kK) - 1u);
+      // A move that an accepted, or a blocked, earlier one reaches is blocked:
+      // it stays open.  The others are made; they do not read what a blocked
+      // one may change, nor it what they change, so their order does not
+      // matter.
+      uint32_t blocked = 0;
+      for (uint32_t next = acc; next != 0;) {
+        const uint32_t b = uint32_t(__builtin_amdgcn_ballot_w64(valid && (conf_d & (acc | blocked)) != 0)) & ((1u << kK) - 1u);
+        next = b & ~blocked;
+        blocked = b;
+      }
+      const uint32_t com = acc & ~blocked;
       if (com != 0) {
-        if ((com >> ck) & 1u) {
+#pragma unroll
+        for (int v = 0; v < kCom; ++v) {
+          if (((com >> (ck + 8 * v)) & 1u) == 0) continue;
           if constexpr (kCanonical) {
-            if constexpr (kK == 16) {
-              if (com_i >= 0) occ[com_i] = uint8_t((lane & 8) ? com_o : com_n);
+            const uint8_t o = uint8_t(ca[v].w), nw = uint8_t(ca[v].w >> 8);
+            if constexpr (kK == 16 && kW == 4) {
+              occ[image((lane & 8) ? cimg[v].y : cimg[v].x)] = (lane & 8) ? o : nw;
             } else {
-              if (com_i >= 0) occ[com_i] = uint8_t(com_n);
-              if (com_j >= 0) occ[com_j] = uint8_t(com_o);
+              occ[image(cimg[v].x)] = nw;
+              occ[image(cimg[v].y)] = o;
             }
-            const int first = kK == 16 ? (lane & 15) : cim;
-            if (first == 0) trk[com_slots & 0xFFFFu] = uint16_t(com_sites >> 16);
-            if (first == 1) trk[com_slots >> 16] = uint16_t(com_sites & 0xFFFFu);
+            const int first = kK == 16 && kW == 4 ? lane & 15 : im;
+            if (first < 2) trk[first ? cs[v].y >> 16 : cs[v].y & 0xFFFFu] = uint16_t(first ? cs[v].x : cs[v].x >> 16);
           } else {
-            if (com_i >= 0) occ[com_i] = uint8_t(com_n);
+            uint32_t nw = c_o[v] + 1u + (ca[v].w & 255u);
+            nw -= nw >= uint32_t(kS) ? uint32_t(kS) : 0u;
+            occ[image(ca[v].z)] = uint8_t(nw);
           }
         }
-        const bool mine = valid && ((com >> (r & 31)) & 1u);
-        de_made = mine ? dE : de_made;
-        if constexpr (!kCanonical) {
-          o_made = mine ? o_l : o_made;
-          n_made = mine ? n_l : n_made;
+        if ((kW == 1 || wave == 0) && lane < kK && ((com >> kd) & 1u)) {
+          de_l[da.w >> 16] = dE;
+          if constexpr (!kCanonical) on_l[da.w >> 16] = d_o | (d_n << 8);
         }
-        acc_bits |= uint64_t(com) << l0;
       }
-      l0 += stop;
+      open &= ~__builtin_amdgcn_ballot_w64(in && ((blocked >> (rank & 31)) & 1u) == 0);
       ++rnd;
       if constexpr (kW > 1)
         __syncthreads();  // the commits before the next round's reads
       else
         own_order();
-      if constexpr (kCanonical) {
-        // later moves of the block whose slots got other sites
-        if (com != 0 && l0 < n_in) {
-          bool stale = false;
-          uint32_t rest = com;
-          while (rest != 0) {
-            const int k = l0 - stop + int(__builtin_ctz(rest));
-            rest &= rest - 1u;
-            const int ta = __builtin_amdgcn_readlane(v_ta, k), tb = __builtin_amdgcn_readlane(v_tb, k);
-            stale = stale || v_ta == ta || v_ta == tb || v_tb == ta || v_tb == tb;
-          }
-          if (__builtin_amdgcn_ballot_w64(stale && lane >= l0) != 0) {
-            look_up();
-            if constexpr (kW > 1)
-              __syncthreads();
-            else
-              own_order();
-          }
-        }
-      }
-    }
-    n_acc += uint64_t(__builtin_popcountll(acc_bits));
-    if (acc_log != nullptr && tid < 2) {
-      const int64_t w = blk0 >> 5;
-      if (lane == 0) acc_log[w] = uint32_t(acc_bits);
-      if (lane == 1 && n_in > 32) acc_log[w + 1] = uint32_t(acc_bits >> 32);
     }
     // ---- the block's energies and samples: lane l after its own move
     if (kW == 1 || wave == 0) {
-      const double e_l = energy + wave_scan_f64(de_made);
+      const double de = de_l[lane];
+      const bool made = __double_as_longlong(de) != kRejected;
+      const uint64_t acc_bits = __builtin_amdgcn_ballot_w64(made);
+      n_acc += uint64_t(__builtin_popcountll(acc_bits));
+      if (acc_log != nullptr && lane < 2) {
+        const int64_t w = blk0 >> 5;
+        if (lane == 0) acc_log[w] = uint32_t(acc_bits);
+        if (lane == 1 && n_in > 32) acc_log[w + 1] = uint32_t(acc_bits >> 32);
+      }
+      const double e_l = energy + wave_scan_f64(made ? de : 0.0);
       const double d = lane < n_in ? e_l - e_ref : 0.0;
       sum_de += d;
       sum_de2 = fma(d, d, sum_de2);
       energy = readlane_f64(e_l, 63);
       if constexpr (!kCanonical) {
+        const int o = int(on_l[lane] & 255u), nw = int(on_l[lane] >> 8);
 #pragma unroll
         for (int b = 0; b < kBM; ++b) {
-          const double ds = o_made == n_made ? 0.0 : __dmul_rn(dphi_tab[(int(o_made) * kS + int(n_made)) * kBM + b], inv_n);
+          const double ds = o == nw ? 0.0 : __dmul_rn(dphi_tab[(o * kS + nw) * kBM + b], inv_n);
           const double s_l = sing[b] + wave_scan_f64(ds);
           const double s = lane < n_in ? s_l : 0.0;
           sum_s[b] += s;
@@ -544,6 +777,7 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
           sing[b] = readlane_f64(s_l, 63);
         }
       }
+      own_order();
     }
   }
 

@@ -2201,9 +2201,10 @@ void wl_launch(cemc_batch* b, int64_t n_checks, int64_t check_every, uint32_t* h
     int nm;
     bool adaptive;
     bool sgc;
+    int patch_kr;
     bool operator<(const WKey& o) const {
-      return std::tie(periodic, kr, glds, kbm, nm, adaptive, sgc) <
-             std::tie(o.periodic, o.kr, o.glds, o.kbm, o.nm, o.adaptive, o.sgc);
+      return std::tie(periodic, kr, glds, kbm, nm, adaptive, sgc, patch_kr) <
+             std::tie(o.periodic, o.kr, o.glds, o.kbm, o.nm, o.adaptive, o.sgc, o.patch_kr);
     }
   };
   std::map<WKey, std::pair<std::vector<int32_t>, uint32_t>> groups;
@@ -2233,8 +2234,22 @@ void wl_launch(cemc_batch* b, int64_t n_checks, int64_t check_every, uint32_t* h
         wl_lds_bytes(sweep_lds_bytes(occ_bytes, m->n_sites, n_rec, int(m->gtab.size())), nbins, adaptive);
     const uint32_t no_g = wl_lds_bytes(sweep_lds_bytes(occ_bytes, m->n_sites, n_rec, 0), nbins, adaptive);
     k.glds = with_g <= std::min(kGtabLdsBudget, limit);
-    const uint32_t lds = k.glds ? with_g : no_g;
-    require(lds <= limit, "the walker's chain and histogram do not fit in the workgroup's LDS");
+    uint32_t lds = k.glds ? with_g : no_g;
+    // a histogram of its own, no windows: the patch kernel's rounds of eight
+    k.patch_kr = 0;
+    const int P = int(m->patches.size());
+    if (!shared && !adaptive && P > 0 && P <= 64 && (k.sgc || m->n_sites <= 65535)) {
+      const int kr = P <= 16 ? 2 : (P <= 32 ? 4 : 8);
+      const uint32_t need = patch_lds_bytes(occ_bytes, k.sgc ? 0 : m->n_sites, int(m->ptab.size()),
+                                            k.sgc ? 0 : 8 * kr) + 16u * uint32_t(nbins);
+      if (need <= limit + sweep_static_lds() - kPatchStaticLds && patch_variant_ok(k.kbm, 8, kr, 1, true, !k.sgc)) {
+        k.patch_kr = kr;
+        k.kr = 0;
+        k.glds = false;
+        lds = need;
+      }
+    }
+    require(lds <= limit || k.patch_kr > 0, "the walker's chain and histogram do not fit in the workgroup's LDS");
     auto& g = groups[k];
     g.first.push_back(c);
     g.second = std::max(g.second, lds);
@@ -2283,6 +2298,7 @@ void wl_launch(cemc_batch* b, int64_t n_checks, int64_t check_every, uint32_t* h
     a.shared = shared ? b->d_wl : nullptr;
     a.adaptive = kv.first.adaptive;
     a.sgc = kv.first.sgc;
+    a.patch_kr = kv.first.patch_kr;
     a.log_base = shared ? chk * per_walker : 0;
     HIP_CHECK(launch_wl(a, b->stream));
     begin += a.n_chains;

@@ -88,6 +88,7 @@ struct LaunchWL {
   bool adaptive = false;          // some walker of the launch uses adaptive windows
   const WLDev* shared = nullptr;  // walkers on this leader's shared histogram (one check per launch)
   int64_t log_base = 0;           // accept-log bit of the launch's first counter
+  int patch_kr = 0;               // patch kernel: patches per lane, eight lanes per move (0: the one-move kernel)
 };
 // Dynamic LDS of one walker: the sweep layout of its chain (base bytes)
 // followed by its ln g, counts and known flags (and, with adaptive windows,

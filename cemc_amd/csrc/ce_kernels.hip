@@ -25,7 +25,6 @@
 
 #include "ce_sweep.h"
 #include "ce_patch_kernel.h"
-#include "ce_wl.h"
 
 
 namespace cemc {
@@ -922,8 +921,8 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
             }
   for (int cn = 0; cn < 2; ++cn)
     for (int w : {1, 2, 4, 8})
-      for (int kg : {4, 16, 64})
-        for (int kr : {1, 2, 3, 4, 6, 7, 9, 15})
+      for (int kg : {4, 8, 16, 64})
+        for (int kr : {1, 2, 3, 4, 6, 7, 8, 9, 15})
           for (int kbm : {1, 2, 3})
             for (int tl = 0; tl < 2; ++tl) {
               const void* fn = patch_fn(cn != 0, kbm, kg, kr, w, tl != 0);
@@ -980,7 +979,9 @@ hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   HookDev* hooks = a.hooks;
   int64_t time_limit = a.time_limit;
   if (a.kg != 0) {
-    void* pargs[] = {&params, &states, &models, &occ_pool, &trk_pool, &order, &n_moves, &log, &log_words, &time_limit};
+    PatchArgs p{params, states, models, occ_pool, trk_pool, order, n_moves, log, log_words, time_limit,
+                nullptr, nullptr, nullptr, nullptr, 0, 0};
+    void* pargs[] = {&p};
     return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), pargs, a.lds_bytes, stream);
   }
   if (a.field) {
@@ -995,6 +996,14 @@ hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
 uint32_t wl_lds_bytes(uint32_t base, int n_bins, bool adaptive) { return wl_layout(base, n_bins, adaptive).total; }
 
 hipError_t launch_wl(const LaunchWL& a, hipStream_t stream) {
+  if (a.patch_kr != 0) {
+    const void* pfn = patch_fn(!a.sgc, a.kbm, 8, a.patch_kr, 1, true);
+    if (pfn == nullptr || a.shared != nullptr || a.adaptive) return hipErrorInvalidValue;
+    PatchArgs p{a.params, a.states, a.models, a.occ_pool, a.trk_pool, a.chain_order, nullptr, a.accept_log, a.log_words,
+                0, a.walkers, a.logdos, a.hist, a.known, a.n_checks, a.check_every};
+    void* pargs[] = {&p};
+    return hipLaunchKernel(pfn, dim3(a.n_chains), dim3(64), pargs, a.lds_bytes, stream);
+  }
   if (!((a.kr == 0 && (a.kbm == 1 || a.kbm == 2 || a.kbm == 3 || a.kbm == 7)) ||
         ((a.kr == 2 || a.kr == 4 || a.kr == 8) && (a.kbm == 1 || a.kbm == 2 || a.kbm == 3))))
     return hipErrorInvalidValue;

@@ -3,7 +3,8 @@
 // patch_fn_w<W>(canonical, kbm, kg, kr, trk_lds), the kernel's address or nullptr
 // for a variant that is not built.  One wave: a quad per move, up to 60
 // patches; two or four waves: a row of 16 lanes per move, up to 64 patches;
-// two, four or eight waves: a wave per move, up to 448 patches.
+// two, four or eight waves: a wave per move, up to 448 patches.  kg 8: the
+// Wang-Landau kernel.
 #include "ce_patch_kernel.h"
 
 #ifndef CEMC_PATCH_WAVES
@@ -32,6 +33,17 @@ const void* row_fn(int kr) {
   return nullptr;
 }
 
+// Wang-Landau walkers: eight lanes per move, up to 64 patches
+template <bool C, int KBM>
+const void* walker_fn(int kr) {
+  if constexpr (W == 1) {
+    if (kr == 2) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 2, 1, 1, true, true>);
+    if (kr == 4) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 4, 1, 1, true, true>);
+    if (kr == 8) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 8, 1, 1, true, true>);
+  }
+  return nullptr;
+}
+
 template <bool C, int KBM, bool T>
 const void* wave_fn(int kr) {
   if constexpr (W >= 2) {
@@ -49,6 +61,8 @@ const void* pick(int kbm, int kg, int kr, bool trk_lds) {
     if (!trk_lds) return nullptr;
     return kbm == 1 ? row_fn<C, 1>(kr) : (kbm == 2 ? row_fn<C, 2>(kr) : (kbm == 3 ? row_fn<C, 3>(kr) : nullptr));
   }
+  if (kg == 8)
+    return kbm == 1 ? walker_fn<C, 1>(kr) : (kbm == 2 ? walker_fn<C, 2>(kr) : (kbm == 3 ? walker_fn<C, 3>(kr) : nullptr));
   if (kg != 64) return nullptr;
   if (!C || trk_lds)
     return kbm == 1 ? wave_fn<C, 1, true>(kr)

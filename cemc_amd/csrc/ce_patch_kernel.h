@@ -41,7 +41,7 @@
 // ms, 128 quaternary 8^3 chains 5.4 -> 3.0 ms (1.2 ms of it the kernel).
 #pragma once
 
-#include "ce_sweep.h"
+#include "ce_wl.h"
 
 namespace cemc {
 
@@ -58,6 +58,11 @@ __host__ __device__ inline PatchLayout patch_layout(int occ_bytes, int trk_sites
   L.total = L.near + align16(uint32_t(near_bytes));
   return L;
 }
+// One bin of a walker in LDS, after the chain's layout.
+struct __align__(16) PatchBin {
+  double lg;
+  uint32_t hist, known;
+};
 constexpr int kNearCells = 126;  // offsets within a halo of 2, and one for "none"
 
 namespace {
@@ -92,6 +97,8 @@ __device__ __attribute__((always_inline)) inline double group_lanes_sum_f64(doub
     v += dpp_f64<0xB1>(v);
     v += dpp_f64<0x4E>(v);
     return v;
+  } else if constexpr (kG == 8) {
+    return octet_sum_f64(v);
   } else if constexpr (kG == 16) {
     v += dpp_f64<0x128>(v);
     return octet_sum_f64(v);
@@ -109,17 +116,48 @@ constexpr long long kRejected = 0x7FF8DEAD00000000ll;
 // kBM: basis functions, one less than the species (1, 2, 3).  kP: moves that
 // a lane group evaluates per round.  kTrkLds: the tracker is held in LDS,
 // else in HBM, where only its lookups per block and its commits touch it.
-template <bool kCanonical, int kBM, int kG, int kR, int kW, int kP, bool kTrkLds>
-__global__ __launch_bounds__(64 * kW) void patch_kernel(
-    const ChainParams* __restrict__ params, ChainState* __restrict__ states, const ModelDev* __restrict__ models,
-    int8_t* __restrict__ occ_pool, uint16_t* __restrict__ trk_pool, const int32_t* __restrict__ chain_order,
-    const int64_t* __restrict__ n_moves, uint32_t* __restrict__ accept_log, int64_t log_words, int64_t time_limit) {
-  static_assert(kG == 4 || kG == 16 || kG == 64, "a quad, a row or the whole wave evaluates a move");
+//
+// kWL: Wang-Landau walkers with a histogram of their own and no adaptive
+// windows (WangLandauSampler::step, wang_landau_sampler.cpp:232-317) on
+// rounds of eight: ln g and the counts stay in LDS, and the round's energy
+// changes are decided one after the other on them, up to the first move that
+// an accepted one reaches.
+struct PatchArgs {
+  const ChainParams* params;
+  ChainState* states;
+  const ModelDev* models;
+  int8_t* occ_pool;
+  uint16_t* trk_pool;
+  const int32_t* chain_order;
+  const int64_t* n_moves;
+  uint32_t* accept_log;
+  int64_t log_words;
+  int64_t time_limit;
+  // walkers
+  WLDev* walkers;
+  double* logdos_pool;
+  uint32_t* hist_pool;
+  uint8_t* known_pool;
+  int64_t n_checks, check_every;
+};
+
+template <bool kCanonical, int kBM, int kG, int kR, int kW, int kP, bool kTrkLds, bool kWL = false>
+__global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
+  const ChainParams* __restrict__ params = args.params;
+  ChainState* __restrict__ states = args.states;
+  const ModelDev* __restrict__ models = args.models;
+  int8_t* __restrict__ occ_pool = args.occ_pool;
+  uint16_t* __restrict__ trk_pool = args.trk_pool;
+  const int32_t* __restrict__ chain_order = args.chain_order;
+  uint32_t* __restrict__ accept_log = args.accept_log;
+  const int64_t log_words = args.log_words, time_limit = args.time_limit;
+  static_assert(kG == 4 || kG == 8 || kG == 16 || kG == 64, "lanes per move");
+  static_assert(!kWL || (kW == 1 && kTrkLds), "a walker is one wave");
   constexpr int kS = kBM + 1;
   constexpr int kQ = kBM == 1 ? 6 : (kBM == 2 ? 5 : 4);  // members per patch (patch_members)
   constexpr int kPer = 64 / kG;                           // moves a wave evaluates side by side
   constexpr int kK = kW * kP * kPer;                       // moves per round
-  static_assert(kK == (kG == 64 ? 8 : 16), "rounds of 16, or of 8 with a wave per move");
+  static_assert(kK == (kG == 64 || kG == 8 ? 8 : 16), "rounds of 16, or of 8 with eight lanes or a wave per move");
   constexpr bool kNear = kCanonical && kG != 64;  // member weights by offset in LDS
   constexpr int kSlots = kG * kR;
   constexpr int kThreads = 64 * kW;
@@ -275,14 +313,37 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
   double energy = states[chain].energy;
   const uint64_t t0 = states[chain].moves_done;
   const double e_ref = states[chain].e_ref;
-  const int64_t nmov = n_moves[chain];
+  // ---- the walker: its bins follow the chain's layout in LDS, 16 bytes each,
+  // so that a move reads one and writes one
+  [[maybe_unused]] WLDev* __restrict__ wk = kWL ? args.walkers + chain : nullptr;
+  const int nb = kWL ? wk->n_bins : 0;
+  [[maybe_unused]] PatchBin* bins = reinterpret_cast<PatchBin*>(lds + L.total);
+  [[maybe_unused]] double e_min = 0.0, span = 1.0, nbd = 1.0, wl_f = 0.0, bins_per_ev = 0.0;
+  [[maybe_unused]] int cur = 0, first = 0;
+  [[maybe_unused]] PatchBin at_cur{0.0, 0, 0};  // the current bin
+  [[maybe_unused]] uint64_t n_out = 0, n_self = 0;
+  if constexpr (kWL) {
+    const int64_t boff = wk->bin_off;
+    for (int i = lane; i < nb; i += 64) {
+      bins[i] = PatchBin{args.logdos_pool[boff + i], args.hist_pool[boff + i], args.known_pool[boff + i]};
+    }
+    __syncthreads();
+    e_min = wk->e_min;
+    span = wk->e_max - e_min;
+    nbd = double(nb);
+    bins_per_ev = nbd / span;
+    wl_f = wk->f;
+    cur = wk->cur_bin;
+    first = wk->is_first;
+    at_cur = bins[cur];  // the host checks 0 <= cur < nb
+  }
   uint64_t n_acc = 0;
   double sum_de = 0.0, sum_de2 = 0.0;  // this lane's moves
   const double inv_n = 1.0 / double(N);
   double sing[kBM], sum_s[kBM], sum_s2[kBM], sum_se[kBM];
 #pragma unroll
   for (int d = 0; d < kBM; ++d) sing[d] = sum_s[d] = sum_s2[d] = sum_se[d] = 0.0;
-  if constexpr (!kCanonical) {
+  if constexpr (!kCanonical && !kWL) {
     // every wave sums alike, so the singlets do not depend on kW
     double part[kBM];
 #pragma unroll
@@ -303,7 +364,6 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
   const uint64_t seg_lo = pp->segoff_pk[0], seg_hi = pp->segoff_pk[1];
   uint32_t* acc_log = accept_log ? accept_log + int64_t(chain) * log_words : nullptr;
   const uint64_t t_begin = time_limit > 0 ? uint64_t(wall_clock64()) : 0u;
-  int64_t moves_made = nmov;
 
   // LDS written by this wave is read by it in program order; other waves are
   // ordered by barriers
@@ -431,29 +491,18 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
   };
 
   uint32_t rnd = 0;
-  for (int64_t blk0 = 0; blk0 < nmov; blk0 += 64) {
-    if (time_limit > 0 && blk0 > 0) {
-      int stop = int(uint64_t(wall_clock64()) - t_begin > uint64_t(time_limit));
-      if constexpr (kW > 1) {
-        int* f = &stop_flag[(blk0 >> 6) & 1];
-        if (tid == 0) *f = stop;
-        __syncthreads();
-        stop = *f;
-      }
-      if (stop) {
-        moves_made = blk0;
-        break;
-      }
-    }
-    // lane l decodes move blk0 + l
-    const Philox4 blk = philox4x64_10(t0 + uint64_t(blk0) + uint64_t(lane), 0, 0, 0, seed, uid);
-    const int n_in = int(nmov - blk0 < 64 ? nmov - blk0 : 64);
+  // One block: moves t_blk .. t_blk + n_in - 1 of the stream, n_in <= 64;
+  // accept bits from bit `log_at` of the chain's log.
+  auto make_block = [&](uint64_t t_blk, int n_in, int64_t log_at) {
+    // lane l decodes move t_blk + l
+    const Philox4 blk = philox4x64_10(t_blk + uint64_t(lane), 0, 0, 0, seed, uid);
     // Metropolis test of the reference (montecarlo.py:950-956): accept when
     // dE < 0 or u <= exp(-dE / kT).  dE against -kT log u decides it outside a
     // margin far above the rounding of log and exp; inside, exp is evaluated.
-    const double t_u = -kT * log(unit_double(blk.w3));
-    const double margin = 2e-12 * (kT + t_u);
-    const double2 thr{t_u - margin, t_u + margin};
+    // (Walkers: log u itself.)
+    const double log_u = log(unit_double(blk.w3));
+    const double t_u = -kT * log_u, margin = 2e-12 * (kT + t_u);
+    const double2 thr = kWL ? double2{log_u, 0.0} : double2{t_u - margin, t_u + margin};
     uint4 v_a{0, 0, 0, 0}, v_b{0, 0, 0, 0};
     uint2 v_s{0, 0};
     // padded index, packed cell and image word of a site
@@ -698,24 +747,77 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
       } else {
         dE = kCanonical ? tot : tot + dsingle_tab[int(d_o) * kS + int(d_n)];
       }
-      const bool valid = kd < n;
-      bool yes = dE < dt.x;
-      if (__builtin_amdgcn_ballot_w64(valid && !yes && !(dE > dt.y)) != 0) {
-        const double u = unit_double(__shfl(blk.w3, int(da.w >> 16), 64));
-        if (!yes && !(dE > dt.y)) yes = dE < 0.0 || u <= exp(-dE / kT);
+      uint32_t com = 0, blocked = 0;
+      if constexpr (kWL) {
+        // ---- slot after slot; every lane holds the walker's state
+        auto any = [](bool x) { return __builtin_amdgcn_ballot_w64(x) != 0; };  // of a value all lanes share
+        int k = 0;
+        for (; k < n; ++k) {
+          if ((uint32_t(__builtin_amdgcn_readlane(int(conf_d), k)) & com) != 0) break;
+          const double e_new = energy + readlane_f64(dE, k);
+          // Truncated bin (histogram.cpp:66-69; the conversion saturates) from
+          // a product; its rounding is below 1e-8 inside any histogram that
+          // fits here, so only near an edge the quotient itself is formed.
+          const double q = (e_new - e_min) * bins_per_ev;
+          int raw = int(q - 1e-8);
+          if (any(raw != int(q + 1e-8)))
+            raw = int(fmin(fmax(trunc((e_new - e_min) * nbd / span), -2147483648.0), 2147483647.0));
+          const int bin = __builtin_amdgcn_readfirstlane(raw);
+          if (uint32_t(bin) >= uint32_t(nb)) {
+            // undone; a walker that has been in range counts its current bin
+            // once more when the proposal lies above the top bin
+            // (wang_landau_sampler.cpp:251-260)
+            ++n_out;
+            if (first || bin <= nb) continue;
+          } else {
+            n_self += bin == cur ? 1u : 0u;
+            // accept if u < g(cur) / g(bin), or on the first in-range proposal
+            // (histogram.cpp:130-135); log u decides outside a margin far
+            // above the rounding of log and exp
+            const PatchBin at_bin = bins[bin];
+            const double diff = at_cur.lg - at_bin.lg;
+            const double over = diff - readlane_f64(dt.x, k);
+            bool take = any(over > 1e-12);
+            if (!take && (first || !any(over < -1e-12))) {
+              const int src = int(uint32_t(__builtin_amdgcn_readlane(int(da.w), k)) >> 16);
+              take = first || any(diff > 0.0 || unit_double(readlane_u64(blk.w3, src)) < exp(diff));
+            }
+            if (take) {
+              com |= 1u << k;
+              energy = e_new;
+              cur = bin;
+              at_cur = at_bin;
+              first = 0;
+            }
+          }
+          // Histogram::update (histogram.cpp:71-90); LDS operations of one
+          // wave complete in order, so the next slot reads it
+          at_cur.lg += wl_f;
+          at_cur.hist += 1u;
+          at_cur.known = 1u;
+          if (lane == 0) bins[cur] = at_cur;
+        }
+        blocked = ((1u << kK) - 1u) & ~((1u << k) - 1u);  // this slot and the later ones stay open
+        n_acc += uint64_t(__builtin_popcount(com));
+      } else {
+        const bool valid = kd < n;
+        bool yes = dE < dt.x;
+        if (__builtin_amdgcn_ballot_w64(valid && !yes && !(dE > dt.y)) != 0) {
+          const double u = unit_double(__shfl(blk.w3, int(da.w >> 16), 64));
+          if (!yes && !(dE > dt.y)) yes = dE < 0.0 || u <= exp(-dE / kT);
+        }
+        const uint32_t acc = uint32_t(__builtin_amdgcn_ballot_w64(valid && yes)) & ((1u << kK) - 1u);
+        // A move that an accepted, or a blocked, earlier one reaches is blocked:
+        // it stays open.  The others are made; they do not read what a blocked
+        // one may change, nor it what they change, so their order does not
+        // matter.
+        for (uint32_t next = acc; next != 0;) {
+          const uint32_t b = uint32_t(__builtin_amdgcn_ballot_w64(valid && (conf_d & (acc | blocked)) != 0)) & ((1u << kK) - 1u);
+          next = b & ~blocked;
+          blocked = b;
+        }
+        com = acc & ~blocked;
       }
-      const uint32_t acc = uint32_t(__builtin_amdgcn_ballot_w64(valid && yes)) & ((1u << kK) - 1u);
-      // A move that an accepted, or a blocked, earlier one reaches is blocked:
-      // it stays open.  The others are made; they do not read what a blocked
-      // one may change, nor it what they change, so their order does not
-      // matter.
-      uint32_t blocked = 0;
-      for (uint32_t next = acc; next != 0;) {
-        const uint32_t b = uint32_t(__builtin_amdgcn_ballot_w64(valid && (conf_d & (acc | blocked)) != 0)) & ((1u << kK) - 1u);
-        next = b & ~blocked;
-        blocked = b;
-      }
-      const uint32_t com = acc & ~blocked;
       if (com != 0) {
 #pragma unroll
         for (int v = 0; v < kCom; ++v) {
@@ -737,8 +839,13 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
           }
         }
         if ((kW == 1 || wave == 0) && lane < kK && ((com >> kd) & 1u)) {
-          de_l[da.w >> 16] = dE;
-          if constexpr (!kCanonical) on_l[da.w >> 16] = d_o | (d_n << 8);
+          if constexpr (kWL) {
+            const int64_t at = log_at + int64_t(da.w >> 16);
+            if (acc_log != nullptr && at < 32 * log_words) atomicOr(acc_log + (at >> 5), 1u << (at & 31));
+          } else {
+            de_l[da.w >> 16] = dE;
+            if constexpr (!kCanonical) on_l[da.w >> 16] = d_o | (d_n << 8);
+          }
         }
       }
       open &= ~__builtin_amdgcn_ballot_w64(in && ((blocked >> (rank & 31)) & 1u) == 0);
@@ -749,13 +856,13 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
         own_order();
     }
     // ---- the block's energies and samples: lane l after its own move
-    if (kW == 1 || wave == 0) {
+    if (!kWL && (kW == 1 || wave == 0)) {
       const double de = de_l[lane];
       const bool made = __double_as_longlong(de) != kRejected;
       const uint64_t acc_bits = __builtin_amdgcn_ballot_w64(made);
       n_acc += uint64_t(__builtin_popcountll(acc_bits));
       if (acc_log != nullptr && lane < 2) {
-        const int64_t w = blk0 >> 5;
+        const int64_t w = log_at >> 5;
         if (lane == 0) acc_log[w] = uint32_t(acc_bits);
         if (lane == 1 && n_in > 32) acc_log[w + 1] = uint32_t(acc_bits >> 32);
       }
@@ -779,6 +886,104 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
       }
       own_order();
     }
+  };
+
+  int64_t moves_made = 0;
+  [[maybe_unused]] int converged = 0;
+  [[maybe_unused]] uint64_t n_flat = 0;
+  if constexpr (kWL) {
+    const double flat_c = wk->flatness, f_min = wk->f_min;
+    converged = wk->converged;
+    int64_t steps = wk->steps, since_flat = wk->since_flat, prev_conv = wk->prev_conv;
+    int inv_active = wk->inv_active;
+    double inv_factor = wk->inv_factor, bin_change = wk->bin_change;
+    const bool inverse_time = wk->inverse_time != 0;
+    for (int64_t chk = 0; chk < args.n_checks && !converged && wk->status == 0; ++chk) {
+      for (int64_t blk0 = 0; blk0 < args.check_every; blk0 += 64) {
+        const int n_in = int(args.check_every - blk0 < 64 ? args.check_every - blk0 : 64);
+        make_block(t0 + uint64_t(moves_made), n_in, moves_made);
+        moves_made += n_in;
+      }
+      steps += args.check_every;
+      since_flat += args.check_every;
+      __syncthreads();
+      // Histogram::is_flat over the known bins (histogram.cpp:102-128); the
+      // sum is an unsigned 32-bit integer and the minimum starts at 100000000
+      uint32_t sum = 0u, cnt = 0u, mn = 100000000u;
+      for (int i = lane; i < nb; i += 64) {
+        const PatchBin at = bins[i];
+        if (at.known) {
+          sum += at.hist;
+          cnt += 1u;
+          mn = min(mn, at.hist);
+        }
+      }
+      sum = wave_add_u32(sum);
+      cnt = wave_add_u32(cnt);
+      mn = wave_min_u32(mn);
+      const double mean = double(sum) / double(cnt);
+      if (__builtin_amdgcn_readfirstlane(int(double(mn) > flat_c * mean)) != 0) {
+        // wang_landau_sampler.cpp:337-394, convergence time in steps
+        const double mc_time = double(steps) / nbd;
+        if (inverse_time && prev_conv >= 0 && since_flat > prev_conv) {
+          if (!inv_active) inv_factor = mc_time * wl_f;
+          inv_active = 1;
+        }
+        prev_conv = since_flat;
+        wl_f = inv_active ? inv_factor / mc_time : wl_f / 2.0;
+        ++n_flat;
+        for (int i = lane; i < nb; i += 64) bins[i].hist = 0u;
+        at_cur.hist = 0u;
+        __syncthreads();
+        bin_change = 0.0;
+        since_flat = 0;
+      }
+      if (wl_f < f_min) converged = 1;
+      __syncthreads();
+    }
+    const int64_t boff = wk->bin_off;
+    for (int i = lane; i < nb; i += 64) {
+      const PatchBin at = bins[i];
+      args.logdos_pool[boff + i] = at.lg;
+      args.hist_pool[boff + i] = at.hist;
+      args.known_pool[boff + i] = uint8_t(at.known);
+    }
+    if (lane == 0) {
+      wk->cur_bin = cur;
+      wk->is_first = first;
+      wk->n_moves += uint64_t(moves_made);
+      wk->n_accept += n_acc;
+      wk->n_outside += n_out;
+      wk->n_self += n_self;
+      wk->f = wl_f;
+      wk->converged = converged;
+      wk->n_flat += n_flat;
+      wk->inv_active = inv_active;
+      wk->inv_factor = inv_factor;
+      wk->bin_change = bin_change;
+      wk->steps = steps;
+      wk->since_flat = since_flat;
+      wk->prev_conv = prev_conv;
+    }
+  } else {
+    const int64_t nmov = args.n_moves[chain];
+    moves_made = nmov;
+    for (int64_t blk0 = 0; blk0 < nmov; blk0 += 64) {
+      if (time_limit > 0 && blk0 > 0) {
+        int stop = int(uint64_t(wall_clock64()) - t_begin > uint64_t(time_limit));
+        if constexpr (kW > 1) {
+          int* f = &stop_flag[(blk0 >> 6) & 1];
+          if (tid == 0) *f = stop;
+          __syncthreads();
+          stop = *f;
+        }
+        if (stop) {
+          moves_made = blk0;
+          break;
+        }
+      }
+      make_block(t0 + uint64_t(blk0), int(nmov - blk0 < 64 ? nmov - blk0 : 64), blk0);
+    }
   }
 
   // ---- write back
@@ -787,7 +992,13 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(
   for (int i = tid; i < N; i += kThreads) wocc[i] = occ[ref_of<true>(c, i).p];
   if constexpr (kCanonical && kTrkLds)
     for (int i = tid; i < N; i += kThreads) gtrk[i] = trk[i];
-  if (wave == 0) {
+  if (kWL && lane == 0) {
+    ChainState* st = states + chain;
+    st->energy = energy;
+    st->moves_done = t0 + uint64_t(moves_made);
+    st->n_accept += n_acc;
+  }
+  if (!kWL && wave == 0) {
     ChainState* st = states + chain;
     const double se = wave_sum_f64(sum_de), se2 = wave_sum_f64(sum_de2);
     if (lane == 0) {

@@ -169,3 +169,25 @@ def test_patch_kernel_matches_oracle(gpu, kind, species, shells, size, symm, cha
             np.testing.assert_allclose(th["var_singlet"], np.var(singlets, axis=0), rtol=0, atol=1e-12)
             cov = np.mean(np.array(singlets) * np.array(trace)[:, None], axis=0) - th["singlet"] * np.mean(trace)
             np.testing.assert_allclose(th["cov_singlet_energy"], cov, rtol=0, atol=1e-11 * st.n_sites)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("species,shells,size,half,bins", [
+    (2, {2: 4, 3: 2}, (5, 6, 7), 0.7, 33),          # two patches a lane, narrow range
+    (2, {2: 4, 3: 3, 4: 2}, 5, 3.0, 100),           # eight
+    (3, {2: 4, 3: 3, 4: 2}, 6, 0.4, 7),             # few bins, many proposals outside
+    (4, {2: 3, 3: 2, 4: 1}, (6, 5, 5), 2.0, 1000),  # four, most bins unvisited
+])
+def test_patch_walkers_match_oracle(gpu, species, shells, size, half, bins):
+    """Wang-Landau swaps on the patch kernel, checks that end inside a block:
+    histogram, ln g (bit for bit), f and lattice equal the oracle's."""
+    from test_wang_landau import _centred, _gpu_vs_oracle
+    s = FCCSettings(size, list("ABCD"[:species]), shells)
+    eci = seeded_ecis(s, 12, 0.02)
+    occ = random_occupation(s.n_sites, species, 4)
+    names = s.cf_names()
+    e0 = OracleUpdater(OracleModel(s, names), occ, brute_force_cf(s, occ, names), eci).get_energy()
+    print("patch walker", species, shells, size, flush=True)
+    got, _ = _gpu_vs_oracle(s, eci, occ, dict(_centred(e0, half, bins), f=1.0, f_min=1e-3, flatness=0.3,
+                                              cur_bin=bins // 2), 9, 333)
+    assert got["n_accept"] > 0

@@ -137,6 +137,13 @@ struct ModelDev {
   double fx_scale;
   const int64_t* gtab_fx;
   const uint32_t* duals;
+  // Species counts of the from-scratch correlation functions: entry c counts
+  // its sub-clusters' species (all members, n_species^size codes) in bins
+  // entry_bin[c] .., a record's entry in rec_bin; cf_bins bins in all.
+  int32_t cf_bins;
+  int32_t pad_bins;
+  const uint32_t* entry_bin;
+  const uint32_t* rec_bin;
   // Patches of the one translation group (n_patch 0: none were found or the
   // model has several groups): their tables as [code][d], d < n_bfs, the
   // first table all zeros (padding patches read it).

@@ -158,6 +158,10 @@ struct cemc_model {
   int32_t *d_cf_kind = nullptr, *d_cf_dec = nullptr, *d_cf_entry = nullptr, *d_cf_eq_off = nullptr;
   uint32_t* d_eq_decos = nullptr;
   ClusterEntry* d_entries = nullptr;
+  // species counts of the from-scratch correlation functions (ModelDev::entry_bin)
+  std::vector<uint32_t> entry_bin, rec_bin;
+  uint32_t cf_bins = 0;
+  uint32_t *d_entry_bin = nullptr, *d_rec_bin = nullptr;
   double* d_eci = nullptr;
   ModelDev view{};
   ModelDev* d_view = nullptr;
@@ -209,6 +213,8 @@ cemc_model::~cemc_model() {
   dev_free(d_cf_eq_off);
   dev_free(d_eq_decos);
   dev_free(d_entries);
+  dev_free(d_entry_bin);
+  dev_free(d_rec_bin);
   dev_free(d_eci);
   dev_free(d_view);
 }
@@ -585,6 +591,9 @@ void cemc_model::refresh_view() {
   v.eci = d_eci;
   v.field_ok = field_ok ? 1 : 0;
   v.fx_scale = fx_scale;
+  v.cf_bins = int(cf_bins);
+  v.entry_bin = d_entry_bin;
+  v.rec_bin = d_rec_bin;
   v.n_patch = int(patches.size());
   v.ptab_size = int(ptab.size());
   v.patches = d_patches;
@@ -846,6 +855,13 @@ static void build_model(cemc_model* m, const cemc_model_desc* d) {
   m->d_cf_eq_off = upload(m->cf_eq_off);
   m->d_eq_decos = upload(m->eq_decos);
   m->d_entries = upload(m->entries);
+  for (int c = 0; c < m->n_entries; ++c) {
+    m->entry_bin.push_back(m->cf_bins);
+    m->cf_bins += uint32_t(m->pow_s(m->entry_size[c]));
+  }
+  for (int e : m->rec_entry) m->rec_bin.push_back(m->entry_bin[e]);
+  m->d_entry_bin = upload(m->entry_bin);
+  m->d_rec_bin = upload(m->rec_bin);
   m->d_eci = upload(m->eci);
   m->refresh_view();
 }
@@ -986,6 +1002,11 @@ struct cemc_updater {
   int32_t* d_changes = nullptr;
   int32_t* d_restore = nullptr;
   int change_cap = 0;
+  // from-scratch correlation functions (set_occupation): the lattice's
+  // parameters, its id, the block partials and an energy, kept by the updater
+  ChainParams* d_cf_params = nullptr;
+  int32_t* d_cf_id = nullptr;
+  double* d_cf_partial = nullptr;  // n_cf x blocks, then the energy
   // work plan of updater_kernel: items and segments per translation group
   // (host copies of the segments give each change its item range)
   std::vector<UpdSeg> segs;
@@ -1066,6 +1087,9 @@ struct cemc_updater {
     dev_free(d_segs);
     dev_free(d_changes);
     dev_free(d_restore);
+    dev_free(d_cf_params);
+    dev_free(d_cf_id);
+    dev_free(d_cf_partial);
     if (stream) (void)hipStreamDestroy(stream);
   }
   unsigned current_slot() const { return current == 0 ? kMaxHistory - 1 : current - 1; }
@@ -2514,24 +2538,22 @@ int cemc_updater_set_occupation(cemc_updater* u, const int8_t* occupation) {
     updater_park(u);
     HIP_CHECK(hipStreamSynchronize(u->stream));
     u->occ.assign(occupation, occupation + N);
-    HIP_CHECK(hipMemcpy(u->d_occ, u->occ.data(), size_t(N), hipMemcpyHostToDevice));
-    ChainParams p;
-    std::memset(&p, 0, sizeof p);
-    p.model = 0;
-    p.n_sites = N;
-    for (int k = 0; k < ncf; ++k)
-      if (model->cf_kind[k] == CEMC_CF_SINGLET) p.j1[model->cf_dec[k]] = u->eci[k];
-    ChainParams* d_p = upload(std::vector<ChainParams>{p});
-    std::vector<double> cf;
-    try {
-      compute_cf(model->d_view, {p}, d_p, u->d_occ, {0}, ncf, &cf, nullptr, u->stream);
-    } catch (...) {
-      dev_free(d_p);
-      throw;
+    HIP_CHECK(hipMemcpyAsync(u->d_occ, u->occ.data(), size_t(N), hipMemcpyHostToDevice, u->stream));
+    // The functions go straight to the history's first slot (it holds only
+    // the new state, cf_history_tracker.cpp:146-149); the energy they give
+    // uses other ECIs than the updater's and is not read.
+    const int n_blocks = (N + 255) / 256;
+    if (u->d_cf_partial == nullptr) {
+      ChainParams p;
+      std::memset(&p, 0, sizeof p);
+      p.n_sites = N;
+      if (!u->d_cf_params) u->d_cf_params = upload(std::vector<ChainParams>{p});
+      if (!u->d_cf_id) u->d_cf_id = upload(std::vector<int32_t>{0});
+      HIP_CHECK(hipMalloc(&u->d_cf_partial, sizeof(double) * (size_t(ncf) * n_blocks + 1)));
     }
-    dev_free(d_p);
-    // history holds only the new state (cf_history_tracker.cpp:146-149)
-    HIP_CHECK(hipMemcpy(u->d_ring, cf.data(), sizeof(double) * ncf, hipMemcpyHostToDevice));
+    HIP_CHECK(launch_cf(model->d_view, u->d_cf_params, u->d_occ, u->d_cf_id, 1, N, u->d_cf_partial, u->d_ring,
+                        u->d_cf_partial + size_t(ncf) * n_blocks, u->stream));
+    HIP_CHECK(hipStreamSynchronize(u->stream));
     u->current = 1;
     u->buffer_size = 1;
     u->slot_epoch.assign(kMaxHistory, -1);

@@ -1013,6 +1013,7 @@ struct cemc_updater {
   std::vector<int32_t> grp_seg;  // n_groups + 1
   UpdItem* d_items = nullptr;
   UpdSeg* d_segs = nullptr;
+  double* d_tab = nullptr;
   UpdPlan plan{};
   uint32_t lds_bytes = 0;
   // pinned host memory: the energy read back by get_energy, the result a
@@ -1084,6 +1085,7 @@ struct cemc_updater {
     dev_free(d_slot_energy);
     dev_free(d_eci);
     dev_free(d_items);
+    dev_free(d_tab);
     dev_free(d_segs);
     dev_free(d_changes);
     dev_free(d_restore);
@@ -1214,16 +1216,33 @@ void updater_stage_copy(cemc_updater* u, int32_t* dst, const int32_t* src, size_
 
 // Work plan of updater_kernel for the updater's model (see UpdItem): for
 // each translation group g and cluster correlation function k with a cluster
-// entry at g, one segment of items (equivalent decoration e, record r of the
-// entry), in the order e-major; LDS passes of at most 4096 items.
+// entry at g, one segment of items: a record r of the entry with the function's
+// product table, or past the tables' limit an (equivalent decoration e, record
+// r), in the order e-major.
 void updater_build_plan(cemc_updater* u) {
   const cemc_model& m = *u->model;
-  const int ncf = m.n_cf;
+  const int ncf = m.n_cf, S = m.n_species, B = m.n_bfs;
+  constexpr uint32_t kLdsCap = 150u * 1024u;
+  // Product tables (UpdPlan::tab) give an item per (function, sub-cluster)
+  // instead of one per (function, decoration, sub-cluster).  The limit of 8 MB
+  // keeps their construction within milliseconds (six and more species with
+  // quadruplets pass it).
+  size_t tab_size = 0;
+  for (int g = 0; g < m.n_groups; ++g)
+    for (int k = 0; k < ncf; ++k) {
+      if (m.cf_kind[k] != CEMC_CF_CLUSTER) continue;
+      const int ent = m.cf_entry[size_t(g) * ncf + k];
+      if (ent >= 0) tab_size += size_t(m.entries[ent].size) * B * m.pow_s(m.entries[ent].size - 1);
+    }
+  const bool tabled = tab_size < (size_t(1) << 20);
+  std::vector<double> tab;
   std::vector<UpdItem> items;
   u->segs.clear();
   u->grp_seg.assign(size_t(m.n_groups) + 1, 0);
+  int most = 0;  // items and segments of a group
   for (int g = 0; g < m.n_groups; ++g) {
     u->grp_seg[g] = int32_t(u->segs.size());
+    const size_t first_item = items.size();
     for (int k = 0; k < ncf; ++k) {
       if (m.cf_kind[k] != CEMC_CF_CLUSTER) continue;
       const int ent = m.cf_entry[size_t(g) * ncf + k];
@@ -1233,29 +1252,54 @@ void updater_build_plan(cemc_updater* u) {
       UpdSeg sg{};
       sg.k = k;
       sg.begin = int32_t(items.size());
-      for (int e = e0; e < e1; ++e) {
+      for (int e = e0; e < (tabled ? e0 + 1 : e1); ++e) {
         const uint32_t deco = m.eq_decos[e];
         for (int r = 0; r < E.rec_count; ++r) {
           const SubRec rec = m.recs[size_t(E.rec_begin) + r];
           const int nm = rec_size(rec) - 1;
           UpdItem it{};
           for (int q = 0; q < nm; ++q) it.m[q] = m.periodic ? m.col_cells[rec_slot(rec, q)] : rec_slot(rec, q);
-          for (int pos = 0; pos <= nm; ++pos) {
-            const uint32_t d = (deco >> (8 * pos)) & 0xFFu;
-            require(d < 8u, "decoration index out of range");
-            it.aux |= d << (3 * pos);
+          if (tabled) {
+            it.aux = uint32_t(tab.size() + size_t(rec_refpos(rec)) * B * m.pow_s(nm)) | (uint32_t(nm) << 24);
+          } else {
+            for (int pos = 0; pos <= nm; ++pos) {
+              const uint32_t d = (deco >> (8 * pos)) & 0xFFu;
+              require(d < 8u, "decoration index out of range");
+              it.aux |= d << (3 * pos);
+            }
+            it.aux |= uint32_t(rec_refpos(rec)) << 12;
+            it.aux |= uint32_t(nm) << 14;
           }
-          it.aux |= uint32_t(rec_refpos(rec)) << 12;
-          it.aux |= uint32_t(nm) << 14;
           items.push_back(it);
           require(items.size() < (size_t(1) << 31), "too many updater items");
         }
       }
+      if (tabled) {
+        const int n = E.size, codes = m.pow_s(n - 1);
+        for (int r = 0; r < n; ++r)
+          for (int d = 0; d < B; ++d)
+            for (int code = 0; code < codes; ++code) {
+              double sum = 0.0;
+              for (int e = e0; e < e1; ++e) {
+                if (int((m.eq_decos[e] >> (8 * r)) & 0xFFu) != d) continue;
+                double prod = 1.0;
+                for (int pos = 0, rest = code; pos < n; ++pos) {
+                  if (pos == r) continue;
+                  prod *= m.basis[int((m.eq_decos[e] >> (8 * pos)) & 0xFFu) * S + rest % S];
+                  rest /= S;
+                }
+                sum += prod;
+              }
+              tab.push_back(sum);
+            }
+      }
       sg.end = int32_t(items.size());
-      sg.mul = double(unsigned(E.size)) / double(e1 - e0);
-      sg.div = double(E.norm * m.grp_count[g]);
+      sg.size = E.size;
+      sg.div = double(e1 - e0) * double(E.norm * m.grp_count[g]);
+      sg.inv = 1.0 / sg.div;
       u->segs.push_back(sg);
     }
+    most = std::max(most, int(items.size() - first_item) + int(u->segs.size()) - u->grp_seg[g]);
   }
   u->grp_seg[m.n_groups] = int32_t(u->segs.size());
   std::vector<int32_t> singlets;
@@ -1263,17 +1307,24 @@ void updater_build_plan(cemc_updater* u) {
     if (m.cf_kind[k] == CEMC_CF_SINGLET) singlets.push_back(int32_t(k | (m.cf_dec[k] << 16)));
   require(ncf < (1 << 16), "too many correlation functions for the updater");
   // the occupation is staged in LDS when it fits beside the rest (lattices
-  // up to ~100k sites); passes of up to 4096 items
-  constexpr uint32_t kLdsCap = 150u * 1024u;
-  const int occ_sites = updater_lds_bytes(ncf, 256, m.n_sites) <= kLdsCap ? m.n_sites : 0;
-  int chunk = 4096;
-  while (chunk > 256 && updater_lds_bytes(ncf, chunk, occ_sites) > kLdsCap) chunk -= 256;
-  u->lds_bytes = updater_lds_bytes(ncf, chunk, occ_sites);
+  // up to ~100k sites), then the product tables beside passes of 4096 items;
+  // passes of up to 4096 items, or of both changes of a swap where those fit
+  const int occ_sites = updater_lds_bytes(ncf, 256, 0, m.n_sites) <= kLdsCap ? m.n_sites : 0;
+  const int tab_n =
+      tab.size() < 16384 && updater_lds_bytes(ncf, 4096, int(tab.size()), occ_sites) <= kLdsCap ? int(tab.size()) : 0;
+  int chunk = std::max(4096, std::min(2 * most, 16384));
+  chunk = (chunk + 255) / 256 * 256;
+  while (chunk > 256 && updater_lds_bytes(ncf, chunk, tab_n, occ_sites) > kLdsCap) chunk -= 256;
+  u->lds_bytes = updater_lds_bytes(ncf, chunk, tab_n, occ_sites);
   require(u->lds_bytes <= kLdsCap, "too many correlation functions for the updater's LDS");
   u->d_items = upload(items);
   u->d_segs = upload(u->segs);
   require(singlets.size() <= size_t(kUpdMaxSinglets), "too many singlet correlation functions");
   for (size_t j = 0; j < singlets.size(); ++j) u->plan.singlets[j] = singlets[j];
+  if (!tab.empty()) u->d_tab = upload(tab);
+  u->plan.tab = u->d_tab;
+  u->plan.tab_n = tab_n;
+  u->plan.inv_n = 1.0 / double(m.n_sites);
   u->plan.items = u->d_items;
   u->plan.segs = u->d_segs;
   u->plan.trans = m.d_trans;
@@ -1419,7 +1470,12 @@ int updater_stage(cemc_updater* u, int site, int old_id, int new_id, std::vector
   packed.push_back(sb < se ? u->segs[se - 1].end : 0);
   packed.push_back(sb);
   packed.push_back(se);
-  packed.push_back(0);
+  int cell = 0;
+  if (m.periodic) {
+    const int l23 = m.dims[1] * m.dims[2], rem = site % l23;
+    cell = (site / l23) | ((rem / m.dims[2]) << 8) | ((rem % m.dims[2]) << 16);
+  }
+  packed.push_back(cell);
   return CEMC_OK;
 }
 

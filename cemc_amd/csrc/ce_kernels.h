@@ -116,23 +116,27 @@ struct InlineChanges {
 // Work plan of the updater kernel for one model.  The change of correlation
 // function k at a site of translation group g sums one product per
 // (equivalent decoration, sub-cluster record of the site) pair; those
-// products are the items of segment (g, k), and a change at a site of group
-// g touches the segments [grp_seg[g], grp_seg[g + 1]) (ce_updater.cpp:349-404).
+// products, or with product tables their sums over the decorations, are the
+// items of segment (g, k), and a change at a site of group g touches the
+// segments [grp_seg[g], grp_seg[g + 1]) (ce_updater.cpp:349-404).
 struct UpdItem {
   // members other than the reference site, in canonical order: closed-form
   // periodic lattices: wrapped cell offset x | y<<8 | z<<16; otherwise
   // translation-table column
   uint32_t m[3];
-  // decoration of position p in bits 3p..3p+2 (p = 0..3), the reference
-  // site's position << 12, members other than the reference site << 14
+  // one item per (function, decoration, sub-cluster): decoration of position p
+  // in bits 3p..3p+2 (p = 0..3), the reference site's position << 12, members
+  // other than the reference site << 14.
+  // With product tables (UpdPlan::tab), one item per (function, sub-cluster):
+  // table base | members << 24
   uint32_t aux;
 };
 struct UpdSeg {
   int32_t k;
   int32_t begin, end;  // items
-  int32_t pad;
-  double mul;  // cluster size / equivalent decorations
-  double div;  // normalisation C_p * T_g
+  int32_t size;  // cluster size
+  double div;    // equivalent decorations x normalisation C_p x T_g
+  double inv;    // 1 / div
 };
 // Everything the kernel needs besides the lattice travels in its arguments,
 // so no load waits on another one at the start.
@@ -147,6 +151,14 @@ struct UpdPlan {
   int32_t n_sites, n_cf, n_species, n_bfs, K, periodic;
   int32_t dims[3];
   int32_t occ_lds;          // 1: the occupation is staged in LDS
+  double inv_n;             // 1 / n_sites
+  // Product tables (nullptr: not used), staged in LDS where they fit (tab_n
+  // doubles, 0: read from memory).  For function k and reference position r: sum over the decorations e of k with
+  // e_r = d of the product of the other members' basis functions, entry
+  // (d, code) at base + d * n_species^members + code, code = sum over members
+  // of species * n_species^q.
+  const double* tab;
+  int32_t tab_n;
   double phi[kMaxBasis * kMaxSpecies];  // basis functions phi[d * n_species + s]
 };
 // Result of an updater launch in mapped, coherent host memory: the bits of
@@ -163,7 +175,8 @@ struct UpdResult {
 // Up to kUpdInline changes of the updater interface travel in the kernel
 // arguments, kUpdWords ints each: site, new | old << 8, src | dst << 16
 // (history slots), first item, end of items, first segment, end of segments,
-// unused; longer sequences are read from `changes` in device memory.
+// cell x | y << 8 | z << 16 (closed-form lattices); longer sequences are read
+// from `changes` in device memory.
 constexpr int kUpdInline = 8;
 constexpr int kUpdWords = 8;
 struct UpdChanges {
@@ -197,8 +210,8 @@ static_assert(sizeof(UpdCmd) == 64 * sizeof(uint64_t), "a command is one 8-byte 
 
 // Dynamic LDS of the updater kernel: correlation functions, segment sums,
 // ECIs and segments (per correlation function), item products of one pass,
-// and the occupation when staged (`occ_sites` bytes, 0 when not).
-uint32_t updater_lds_bytes(int n_cf, int chunk, int occ_sites);
+// product tables, and the occupation when staged (`occ_sites` bytes, 0 when not).
+uint32_t updater_lds_bytes(int n_cf, int chunk, int tab_doubles, int occ_sites);
 hipError_t launch_updater(const UpdPlan& plan, int8_t* occ, double* ring,
                           double* slot_energy, const UpdChanges& inl, const int32_t* changes, int n,
                           const double* eci, UpdResult* result, uint64_t* result_cf, uint32_t lds_bytes,

@@ -292,28 +292,45 @@ __global__ __launch_bounds__(1024) void cf_finalize_kernel(const ModelDev* __res
 // (ce_updater.cpp:313-406).  The correlation functions of the current slot
 // stay in LDS between changes.  Per change every thread forms the products of
 // its plan items (one dependent gather of the members' species) into LDS,
-// then wave w sums the segments w, w + 4, ... in a fixed order, so results do
+// then wave w sums the segments w, w + kUpdWaves, ... in a fixed order, so results do
 // not depend on timing.  After the last change E = N J.cf goes to the slot
 // and, when `result` is given, to mapped host memory, so the host reads it
 // without a copy or a stream wait.
-uint32_t updater_lds_bytes(int n_cf, int chunk, int occ_sites) {
+uint32_t updater_lds_bytes(int n_cf, int chunk, int tab_doubles, int occ_sites) {
   const int ncf_pad = (n_cf + 31) / 32 * 32;
   return uint32_t(3 * sizeof(double) + sizeof(UpdSeg)) * uint32_t(ncf_pad) +
-         uint32_t(sizeof(double)) * uint32_t(chunk) + uint32_t((occ_sites + 15) / 16 * 16);
+         uint32_t(sizeof(double)) * uint32_t(chunk + tab_doubles) + uint32_t((occ_sites + 15) / 16 * 16);
 }
+
+// What bounds a call: the poll over the bus and the answer (about 5 us), then
+// one chain of dependent steps in one workgroup: gathers, table reads, segment
+// sums, two barriers.  With the decorations of a function summed beforehand
+// (UpdPlan::tab) a change on the ternary four-body lattice has 2974 items, one
+// per (function, sub-cluster), so both changes of a swap fit one pass; all
+// waves of a compute unit share the items and the segment sums.
+// A pass of 32 swaps, kept or undone, on FCC 8^3, ternary four-body (71
+// functions, tables in LDS), with the lattice set anew: 8.5 ms with an item
+// per decoration on 256 threads, 0.95 ms with 512 threads, 0.80 ms with 1024;
+// of 64 swaps on FCC 10^3, binary pairs and triplets, 1.10 -> 0.70 ms.  Pairs
+// of changes and their undo, tables in memory: ternary 40^3, 251 functions,
+// 529 -> 79 us; quaternary 12^3, 112 functions, 157 -> 22 us; eight species
+// past the tables' size limit, 386 -> 98 us.
+constexpr int kUpdThreads = 1024;
+constexpr int kUpdWaves = kUpdThreads / 64;
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima).
 __device__ inline void vm_wait_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // Pointers into the updater's dynamic LDS: correlation functions of the
 // current slot, segment sums over earlier passes, ECIs, segments of the
-// change, item products of one pass, staged occupation.
+// change, item products of one pass, product tables, staged occupation.
 struct UpdLds {
   double* cfl;
   double* acc;
   double* ecil;
   UpdSeg* segl;
   double* prod;
+  double* tab;
   int8_t* occ_l;
 };
 __device__ inline UpdLds upd_lds_layout(const UpdPlan& plan, double* upd_lds) {
@@ -324,7 +341,8 @@ __device__ inline UpdLds upd_lds_layout(const UpdPlan& plan, double* upd_lds) {
   L.ecil = L.acc + ncf_pad;
   L.segl = reinterpret_cast<UpdSeg*>(L.ecil + ncf_pad);
   L.prod = reinterpret_cast<double*>(L.segl + ncf_pad);
-  L.occ_l = reinterpret_cast<int8_t*>(L.prod + plan.chunk);
+  L.tab = L.prod + plan.chunk;
+  L.occ_l = reinterpret_cast<int8_t*>(L.tab + plan.tab_n);
   return L;
 }
 
@@ -335,15 +353,16 @@ __device__ inline void updater_stage_fixed(const UpdPlan& plan, const int8_t* oc
                                            double* upd_lds, double* phi) {
   const int tid = int(threadIdx.x);
   const UpdLds L = upd_lds_layout(plan, upd_lds);
-  for (int k = tid; k < plan.n_cf; k += 256) L.ecil[k] = eci[k];
-  for (int i = tid; i < plan.n_bfs * plan.n_species; i += 256) phi[i] = plan.phi[i];
+  for (int k = tid; k < plan.n_cf; k += kUpdThreads) L.ecil[k] = eci[k];
+  for (int i = tid; i < plan.n_bfs * plan.n_species; i += kUpdThreads) phi[i] = plan.phi[i];
+  for (int i = tid; i < plan.tab_n; i += kUpdThreads) L.tab[i] = plan.tab[i];
   if constexpr (kOccLds) {
     // 4-byte words, then the last N mod 4 bytes (the allocation is aligned)
     const int N = plan.n_sites;
     const int nw4 = N >> 2;
     const uint32_t* src = reinterpret_cast<const uint32_t*>(occ);
     uint32_t* dst = reinterpret_cast<uint32_t*>(L.occ_l);
-    for (int i = tid; i < nw4; i += 256) dst[i] = src[i];
+    for (int i = tid; i < nw4; i += kUpdThreads) dst[i] = src[i];
     if (tid < (N & 3)) L.occ_l[4 * nw4 + tid] = occ[4 * nw4 + tid];
   }
 }
@@ -382,6 +401,7 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
                                             const double* __restrict__ eci, UpdResult* result,
                                             uint64_t* result_cf, double* upd_lds, double* phi, double* red,
                                             int held, UpdHeldGroup* hg) {
+#pragma clang fp contract(off)  // fused and change-by-change sums round alike
   const int tid = int(threadIdx.x);
   const int wave = tid >> 6, lane = tid & 63;
   const int S = plan.n_species;
@@ -411,21 +431,26 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
       return occ[i];
     }
   };
-  // items (m[0..2], aux) and segments (k, begin, end, pad; mul, div) are
+  // items (m[0..2], aux) and segments (k, begin, end, size; div, inv) are
   // held as vectors so that they stay in registers
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
   typedef double f64x2 __attribute__((ext_vector_type(2)));
   static_assert(sizeof(UpdItem) == 16 && sizeof(UpdSeg) == 32, "updater plan layout");
-  // cell coordinates of a site (closed-form periodic lattices)
-  auto cell_of = [&](int32_t site, int32_t& rx, int32_t& ry, int32_t& rz) {
+  // a / b with inv = 1 / b at hand: the product, then one step on its residual
+  auto divided = [](double a, double b, double inv) {
+    const double q = a * inv;
+    return __builtin_fma(__builtin_fma(-q, b, a), inv, q);
+  };
+  // cell coordinates of a change's site (closed-form periodic lattices): the
+  // host sends them with the change
+  auto cell_of = [&](int c, int32_t& rx, int32_t& ry, int32_t& rz) {
     rx = ry = rz = 0;
     if constexpr (kPeriodic) {
-      const int32_t l23 = plan.dims[1] * plan.dims[2];
-      rx = site / l23;
-      const int32_t rem = site - rx * l23;
-      ry = rem / plan.dims[2];
-      rz = rem - ry * plan.dims[2];
+      const int32_t w = word(c, 7);
+      rx = w & 0xFF;
+      ry = (w >> 8) & 0xFF;
+      rz = (w >> 16) & 0xFF;
     }
   };
   // product of one plan item for a change of `site` from `old` to `nw`,
@@ -437,7 +462,8 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
   auto product_of = [&](const u32x4& it, int32_t site, int32_t rx, int32_t ry, int32_t rz, int nw, int old,
                         auto&& spec) {
     const uint32_t aux = it.w;
-    const int nm = int((aux >> 14) & 3u);
+    const bool tabled = plan.tab != nullptr;
+    const int nm = tabled ? int(aux >> 24) : int((aux >> 14) & 3u);
     const int rp = int((aux >> 12) & 3u);
     int sp[3];
 #pragma unroll
@@ -456,6 +482,22 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
         if (q < nm) nb = plan.trans[int64_t(site) * plan.K + mq];
       }
       sp[q] = spec(nb);
+    }
+    if (tabled) {
+      // the products of all decorations of the function, summed per basis
+      // function at the reference site
+      const int w1 = nm > 1 ? S : 0, w2 = nm > 2 ? S * S : 0;
+      const int codes = S * (nm > 1 ? S : 1) * (nm > 2 ? S : 1);
+      const uint32_t at = (aux & 0xFFFFFFu) + uint32_t(sp[0] + w1 * sp[1] + w2 * sp[2]);
+      double v = 0.0;
+      if (plan.tab_n > 0) {
+        for (int d = 0; d < plan.n_bfs; ++d)
+          v = __builtin_fma(phi[d * S + nw] - phi[d * S + old], L.tab[at + d * codes], v);
+      } else {
+        for (int d = 0; d < plan.n_bfs; ++d)
+          v = __builtin_fma(phi[d * S + nw] - phi[d * S + old], plan.tab[at + d * codes], v);
+      }
+      return v;
     }
     double f[kMaxClusterSize];
 #pragma unroll
@@ -514,7 +556,7 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
     // meanwhile (loads and stores share one counter)
     const int src0 = word(0, 2) & 0xFFFF;
     if (kStage || src0 != held)
-      for (int k = tid; k < ncf; k += 256) cfl[k] = ring[int64_t(src0) * ncf + k];
+      for (int k = tid; k < ncf; k += kUpdThreads) cfl[k] = ring[int64_t(src0) * ncf + k];
     if constexpr (kStage) updater_stage_fixed<kOccLds>(plan, occ, eci, upd_lds, phi);
   }
   // The loads above complete before the first barrier in any case.  Waiting
@@ -530,18 +572,18 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
     double* dlt = prod + n * fm;                        // change of each (change, segment) pair
     if (!reuse) {
       if (sb0 + tid < se0) segl[tid] = UpdSeg{si0.x, si0.y, si0.z, si0.w, sd0.x, sd0.y};
-      for (int j = tid + 256; j < fseg; j += 256) segl[j] = plan.segs[sb0 + j];
-      for (int k = tid; k < ncf; k += 256) segof[k] = -1;
+      for (int j = tid + kUpdThreads; j < fseg; j += kUpdThreads) segl[j] = plan.segs[sb0 + j];
+      for (int k = tid; k < ncf; k += kUpdThreads) segof[k] = -1;
       barrier();
-      for (int j = tid; j < fseg; j += 256) segof[segl[j].k] = j;
+      for (int j = tid; j < fseg; j += kUpdThreads) segof[segl[j].k] = j;
     }
-    for (int g = tid; g < n * fm; g += 256) {
+    for (int g = tid; g < n * fm; g += kUpdThreads) {
       const int c = g / fm;
       const u32x4 it = g == tid ? it0 : items[ib0 + (g - c * fm)];
       const int site = word(c, 0);
       const int nw = word(c, 1) & 0xFF, old = (word(c, 1) >> 8) & 0xFF;
       int32_t rx, ry, rz;
-      cell_of(site, rx, ry, rz);
+      cell_of(c, rx, ry, rz);
       auto spec = [&](int32_t i) -> int {
         int v = species_at(i);
         for (int q = 0; q < c; ++q)
@@ -551,13 +593,13 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
       prod[g] = product_of(it, site, rx, ry, rz, nw, old, spec);
     }
     barrier();
-    for (int pj = wave; pj < n * fseg; pj += 4) {
+    for (int pj = wave; pj < n * fseg; pj += kUpdWaves) {
       const int c = pj / fseg;
       const UpdSeg g = segl[pj - c * fseg];
       double v = 0.0;
       for (int i = g.begin + lane; i < g.end; i += 64) v += prod[c * fm + (i - ib0)];
       v = wave_sum_f64(v);
-      if (lane == 0) dlt[pj] = ((0.0 + v) * g.mul) / g.div;
+      if (lane == 0) dlt[pj] = divided(v * double(g.size), g.div, g.inv);
     }
     barrier();
     // the occupation after every change of the call (all products are formed)
@@ -566,7 +608,7 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
         occ[word(c, 0)] = int8_t(word(c, 1) & 0xFF);
         if constexpr (kOccLds) occ_l[word(c, 0)] = int8_t(word(c, 1) & 0xFF);
       }
-    for (int k = tid; k < ncf; k += 256) {
+    for (int k = tid; k < ncf; k += kUpdThreads) {
       const int j = segof[k];
       int sd = -1;  // decoration of a singlet function (fixed indices: scalar loads of the arguments)
 #pragma unroll
@@ -577,7 +619,7 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
         if (j >= 0) v += dlt[c * fseg + j];
         if (sd >= 0) {
           const int nw = word(c, 1) & 0xFF, old = (word(c, 1) >> 8) & 0xFF;
-          v += (phi[sd * S + nw] - phi[sd * S + old]) / double(unsigned(N));
+          v += divided(phi[sd * S + nw] - phi[sd * S + old], double(unsigned(N)), plan.inv_n);
         }
         ring[int64_t((word(c, 2) >> 16) & 0xFFFF) * ncf + k] = v;
       }
@@ -607,26 +649,26 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
         vm_wait_all();
       }
       if (sb + tid < se) segl[tid] = UpdSeg{si0.x, si0.y, si0.z, si0.w, sd0.x, sd0.y};
-      for (int j = tid + 256; j < se - sb; j += 256) segl[j] = plan.segs[sb + j];
+      for (int j = tid + kUpdThreads; j < se - sb; j += kUpdThreads) segl[j] = plan.segs[sb + j];
       cur_sb = sb;
       // the staged data and the segments are visible after this barrier
       // (with the same group the barrier closing the change before suffices)
       barrier();
     }
     int32_t rx, ry, rz;
-    cell_of(site, rx, ry, rz);
+    cell_of(c, rx, ry, rz);
     auto product = [&](const u32x4& it) { return product_of(it, site, rx, ry, rz, nw, old, species_at); };
     for (int cb = ib; cb < ie; cb += plan.chunk) {
       const int ce = min(ie, cb + plan.chunk);
       int idx = cb + tid;
       if (cb == ib) {
         if (idx < ce) prod[idx - cb] = product(it0);
-        idx += 256;
+        idx += kUpdThreads;
       }
-      for (; idx < ce; idx += 256) prod[idx - cb] = product(items[idx]);
+      for (; idx < ce; idx += kUpdThreads) prod[idx - cb] = product(items[idx]);
       barrier();
       const bool last_pass = ce == ie;
-      for (int j = wave; j < se - sb; j += 4) {
+      for (int j = wave; j < se - sb; j += kUpdWaves) {
         const UpdSeg g = segl[j];
         const int lo = max(g.begin, cb), hi = min(g.end, ce);
         double v = 0.0;
@@ -635,7 +677,7 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
         if (lane == 0) {
           const double t = (cb == ib ? 0.0 : acc[j]) + v;
           if (last_pass) {
-            cfl[g.k] += (t * g.mul) / g.div;
+            cfl[g.k] += divided(t * double(g.size), g.div, g.inv);
           } else {
             acc[j] = t;
           }
@@ -653,7 +695,7 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
     for (int j = 0; j < kUpdMaxSinglets; ++j) {
       if (tid == j && j < plan.n_singlets) {
         const int k = plan.singlets[j] & 0xFFFF, d = plan.singlets[j] >> 16;
-        cfl[k] += (phi[d * S + nw] - phi[d * S + old]) / double(unsigned(N));
+        cfl[k] += divided(phi[d * S + nw] - phi[d * S + old], double(unsigned(N)), plan.inv_n);
       }
     }
     // every gather of this change is done (the pass barrier above)
@@ -662,23 +704,28 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
       if constexpr (kOccLds) occ_l[site] = int8_t(nw);
     }
     barrier();
-    for (int k = tid; k < ncf; k += 256) ring[int64_t(dst) * ncf + k] = cfl[k];
+    for (int k = tid; k < ncf; k += kUpdThreads) ring[int64_t(dst) * ncf + k] = cfl[k];
   }
   if (last_dst < 0) return held;
   // the final correlation functions to mapped host memory; the host marks
   // every value pending before the launch and waits for each, so these
   // stores need no ordering against the energy
   if (result_cf != nullptr)
-    for (int k = tid; k < ncf; k += 256)
+    for (int k = tid; k < ncf; k += kUpdThreads)
       __hip_atomic_store(&result_cf[k], uint64_t(__double_as_longlong(cfl[k])), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
   double part = 0.0;
-  for (int k = tid; k < ncf; k += 256) part += ecil[k] * cfl[k];
+  for (int k = tid; k < ncf; k += kUpdThreads) part = __builtin_fma(ecil[k], cfl[k], part);
   part = wave_sum_f64(part);
-  if (lane == 0) red[wave] = part;
-  barrier();
+  double sum = part;
+  if (ncf > 64) {  // else the first wave holds every function
+    if (lane == 0) red[wave] = part;
+    barrier();
+    sum = red[0];
+    for (int w = 1; w < kUpdWaves; ++w) sum += red[w];
+  }
   if (tid == 0) {
-    const double e = ((red[0] + red[1]) + (red[2] + red[3])) * double(unsigned(N));
+    const double e = sum * double(unsigned(N));
     slot_energy[last_dst] = e;
     if (result != nullptr)
       __hip_atomic_store(&result->energy_bits, uint64_t(__double_as_longlong(e)), __ATOMIC_RELAXED,
@@ -690,14 +737,14 @@ __device__ __forceinline__ int updater_body(const UpdPlan& plan, int8_t* occ, do
 // A launch for one call: the changes travel in the kernel arguments
 // (kInArgs) or in `changes` in device memory.
 template <bool kInArgs, bool kOccLds, bool kPeriodic>
-__global__ __launch_bounds__(256) void updater_kernel(UpdPlan plan, int8_t* occ, double* __restrict__ ring,
-                                                      double* __restrict__ slot_energy, UpdChanges inl,
-                                                      const int32_t* __restrict__ changes, int n,
-                                                      const double* __restrict__ eci, UpdResult* result,
-                                                      uint64_t* result_cf) {
+__global__ __launch_bounds__(kUpdThreads) void updater_kernel(UpdPlan plan, int8_t* occ, double* __restrict__ ring,
+                                                              double* __restrict__ slot_energy, UpdChanges inl,
+                                                              const int32_t* __restrict__ changes, int n,
+                                                              const double* __restrict__ eci, UpdResult* result,
+                                                              uint64_t* result_cf) {
   extern __shared__ double upd_lds[];
   __shared__ double phi[kMaxBasis * kMaxSpecies];
-  __shared__ double red[4];
+  __shared__ double red[kUpdWaves];
   auto word = [&](int c, int w) { return kInArgs ? inl.v[kUpdWords * c + w] : changes[kUpdWords * c + w]; };
   (void)updater_body<kOccLds, kPeriodic, true>(plan, occ, ring, slot_energy, word, n, eci, result, result_cf,
                                                 upd_lds, phi, red, -1, nullptr);
@@ -715,14 +762,13 @@ __global__ __launch_bounds__(256) void updater_kernel(UpdPlan plan, int8_t* occ,
 // ECIs, basis functions, staged occupation and the correlation functions of
 // the last destination slot stay in LDS.
 template <bool kOccLds, bool kPeriodic>
-__global__ __launch_bounds__(256) void updater_resident_kernel(UpdPlan plan, int8_t* occ, double* __restrict__ ring,
-                                                               double* __restrict__ slot_energy,
-                                                               const double* __restrict__ eci, UpdResult* result,
-                                                               uint64_t* result_cf, UpdMailbox* mb, int64_t next,
-                                                               int64_t idle_ticks) {
+__global__ __launch_bounds__(kUpdThreads) void updater_resident_kernel(
+    UpdPlan plan, int8_t* occ, double* __restrict__ ring, double* __restrict__ slot_energy,
+    const double* __restrict__ eci, UpdResult* result, uint64_t* result_cf, UpdMailbox* mb, int64_t next,
+    int64_t idle_ticks) {
   extern __shared__ double upd_lds[];
   __shared__ double phi[kMaxBasis * kMaxSpecies];
-  __shared__ double red[4];
+  __shared__ double red[kUpdWaves];
   __shared__ int32_t cmd[4 + kUpdCmdWords];  // op, n, want, nr, words
   const int tid = int(threadIdx.x);
   updater_stage_fixed<kOccLds>(plan, occ, eci, upd_lds, phi);
@@ -1210,8 +1256,8 @@ static hipError_t launch_updater_t(const UpdPlan& plan, int8_t* occ, double* rin
       limit = lds_bytes;
     }
   }
-  hipLaunchKernelGGL(fn, dim3(1), dim3(256), lds_bytes, stream, plan, occ, ring, slot_energy, inl, changes, n, eci,
-                     result, result_cf);
+  hipLaunchKernelGGL(fn, dim3(1), dim3(kUpdThreads), lds_bytes, stream, plan, occ, ring, slot_energy, inl, changes, n,
+                     eci, result, result_cf);
   return hipGetLastError();
 }
 
@@ -1247,8 +1293,8 @@ static hipError_t launch_resident_t(const UpdPlan& plan, int8_t* occ, double* ri
       limit = lds_bytes;
     }
   }
-  hipLaunchKernelGGL(fn, dim3(1), dim3(256), lds_bytes, stream, plan, occ, ring, slot_energy, eci, result, result_cf,
-                     mb, next, idle_ticks);
+  hipLaunchKernelGGL(fn, dim3(1), dim3(kUpdThreads), lds_bytes, stream, plan, occ, ring, slot_energy, eci, result,
+                     result_cf, mb, next, idle_ticks);
   return hipGetLastError();
 }
 

@@ -1602,7 +1602,14 @@ struct cemc_batch {
   double* d_adm_partial = nullptr;
   double* h_adm = nullptr;  // pinned: chain id in and energy out
   int adm_blocks = 0;
+  // small reads of the state (batch_read): mapped host memory, the flag in
+  // its first 64 bytes
+  static constexpr size_t kReadMax = 64u << 10;
+  std::mutex read_mutex;
+  uint8_t *h_read = nullptr, *d_read = nullptr;
+  uint64_t read_tag = 0;
   ~cemc_batch() {
+    if (h_read) (void)hipHostFree(h_read);
     if (h_adm) (void)hipHostFree(h_adm);
     dev_free(d_adm_id);
     dev_free(d_adm_e);
@@ -2195,6 +2202,52 @@ WLBins wl_download(cemc_batch* b) {
   HIP_CHECK(hipMemcpy(st.data(), b->d_wl, sizeof(WLDev) * st.size(), hipMemcpyDeviceToHost));
   b->wl = st;
   return h;
+}
+
+struct ReadPiece {
+  void* dst;
+  const void* src;  // device memory
+  size_t bytes;
+};
+
+// Copies up to kReadPieces pieces of the batch's state to the host, after the
+// work on its stream.  Up to 64 KB in all go through read_back_kernel (a copy
+// command per piece takes longer; above, the copy engine's rate decides).
+void batch_read(cemc_batch* b, const std::vector<ReadPiece>& pieces) {
+  ReadBack r{};
+  size_t total = 0;
+  for (size_t i = 0; i < pieces.size(); ++i) {
+    r.src[i] = pieces[i].src;
+    r.bytes[i] = uint32_t(pieces[i].bytes);
+    r.at[i] = uint32_t(total);
+    total += (pieces[i].bytes + 15) / 16 * 16;
+  }
+  if (total > cemc_batch::kReadMax) {
+    HIP_CHECK(hipStreamSynchronize(b->stream));
+    for (const auto& p : pieces)
+      if (p.bytes > 0) HIP_CHECK(hipMemcpy(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost));
+    return;
+  }
+  std::lock_guard<std::mutex> lock(b->read_mutex);
+  if (b->h_read == nullptr) {
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&b->h_read), 64 + cemc_batch::kReadMax,
+                            hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset(b->h_read, 0, 64);
+    HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&b->d_read), b->h_read, 0));
+  }
+  const uint64_t tag = ++b->read_tag;
+  uint64_t* flag = reinterpret_cast<uint64_t*>(b->h_read);
+  HIP_CHECK(launch_read_back(r, b->d_read + 64, reinterpret_cast<uint64_t*>(b->d_read), tag, b->stream));
+  const auto t0 = std::chrono::steady_clock::now();
+  for (uint32_t spin = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != tag; ++spin) {
+    if ((spin & 4095u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) {
+      HIP_CHECK(hipStreamSynchronize(b->stream));
+      if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != tag) throw DeviceError("the read-back kernel stored nothing");
+      break;
+    }
+    __builtin_ia32_pause();
+  }
+  for (size_t i = 0; i < pieces.size(); ++i) std::memcpy(pieces[i].dst, b->h_read + 64 + r.at[i], pieces[i].bytes);
 }
 
 // Re-packs the pools after walker `chain` got n_bins bins (its new values
@@ -2942,7 +2995,7 @@ int cemc_batch_get_energy(cemc_batch* b, double* energy) {
   return guarded([&] {
     require(b && energy, "NULL argument");
     std::vector<ChainState> st(b->n_chains);
-    HIP_CHECK(hipMemcpy(st.data(), b->d_states, sizeof(ChainState) * st.size(), hipMemcpyDeviceToHost));
+    batch_read(b, {{st.data(), b->d_states, sizeof(ChainState) * st.size()}});
     for (int c = 0; c < b->n_chains; ++c) energy[c] = st[c].energy;
   });
 }
@@ -2953,7 +3006,7 @@ int cemc_batch_get_occupation(cemc_batch* b, int32_t chain, int8_t* occupation) 
     require(chain >= 0 && chain < b->n_chains, "chain index out of range");
     require(!b->dynamic || b->active[chain], "slot is not in use");
     const ChainParams& p = b->params[chain];
-    HIP_CHECK(hipMemcpy(occupation, b->d_occ + p.occ_off, size_t(p.n_sites), hipMemcpyDeviceToHost));
+    batch_read(b, {{occupation, b->d_occ + p.occ_off, size_t(p.n_sites)}});
   });
 }
 
@@ -2961,7 +3014,7 @@ int cemc_batch_get_stats(cemc_batch* b, int64_t* moves_done, int64_t* n_accept, 
   return guarded([&] {
     require(b != nullptr, "NULL batch");
     std::vector<ChainState> st(b->n_chains);
-    HIP_CHECK(hipMemcpy(st.data(), b->d_states, sizeof(ChainState) * st.size(), hipMemcpyDeviceToHost));
+    batch_read(b, {{st.data(), b->d_states, sizeof(ChainState) * st.size()}});
     for (int c = 0; c < b->n_chains; ++c) {
       const double n = double(st[c].n_samples), r = st[c].e_ref;
       if (moves_done) moves_done[c] = int64_t(st[c].moves_done);
@@ -3289,8 +3342,14 @@ int cemc_batch_wl_get(cemc_batch* b, int32_t chain, cemc_wl_desc* desc, double* 
     require(b != nullptr, "NULL batch");
     require(chain >= 0 && chain < b->n_chains, "chain index out of range");
     require(!b->wl.empty() && b->wl[chain].n_bins > 0, "the chain carries no Wang-Landau walker");
-    const WLBins h = wl_download(b);
-    const WLDev& w = b->wl[chain];
+    WLDev w = b->wl[chain];
+    const size_t n = size_t(w.n_bins);
+    std::vector<ReadPiece> pieces{{&w, b->d_wl + chain, sizeof(WLDev)}};
+    if (logdos) pieces.push_back({logdos, b->d_wl_logdos + w.bin_off, sizeof(double) * n});
+    if (hist) pieces.push_back({hist, b->d_wl_hist + w.bin_off, sizeof(uint32_t) * n});
+    if (known) pieces.push_back({known, b->d_wl_known + w.bin_off, n});
+    batch_read(b, pieces);
+    b->wl[chain] = w;
     if (desc) {
       desc->n_bins = w.n_bins;
       desc->current_bin = w.cur_bin;
@@ -3301,12 +3360,6 @@ int cemc_batch_wl_get(cemc_batch* b, int32_t chain, cemc_wl_desc* desc, double* 
       desc->f = w.f;
       desc->f_min = w.f_min;
       desc->flatness = w.flatness;
-    }
-    for (int i = 0; i < w.n_bins; ++i) {
-      const size_t o = size_t(w.bin_off + i);
-      if (logdos) logdos[i] = h.logdos[o];
-      if (hist) hist[i] = int32_t(h.hist[o]);
-      if (known) known[i] = h.known[o];
     }
     if (counters) {
       counters[0] = int64_t(w.n_moves);

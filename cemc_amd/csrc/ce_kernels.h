@@ -106,6 +106,16 @@ hipError_t launch_cf(const ModelDev* models, const ChainParams* params, const in
 hipError_t launch_energy(const ModelDev* models, const ChainParams* params, const int8_t* occ_pool,
                          const int32_t* chain_ids, int n_chains, int max_sites, double* partial, double* energy_out,
                          hipStream_t stream);
+// Small pieces of a batch's state (a lattice; a walker and its bins) go to
+// mapped, coherent host memory by one launch: piece i to dst + at[i], then
+// `tag` to *flag.
+constexpr int kReadPieces = 4;
+struct ReadBack {
+  const void* src[kReadPieces];
+  uint32_t bytes[kReadPieces];  // 0: no piece
+  uint32_t at[kReadPieces];     // multiples of 4
+};
+hipError_t launch_read_back(const ReadBack& r, uint8_t* dst, uint64_t* flag, uint64_t tag, hipStream_t stream);
 // Up to kInlineChanges site/species pairs of a restore travel in the kernel
 // arguments, so an undo needs no copy to the device.
 constexpr int kInlineChanges = 8;

@@ -1581,6 +1581,7 @@ struct cemc_batch {
   // constraints and bias per chain (host copies; device arrays they point to)
   struct Hooks {
     bool on = false;
+    bool by_proposal = false;  // whether a proposal is valid does not depend on the state (patch kernel)
     HookDev dev{};
     uint8_t* d_allowed = nullptr;
     int32_t* d_nb = nullptr;
@@ -1933,7 +1934,8 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     }
     // records in VGPRs gather two members each when no record has three
     k.nm = (k.kr > 0 && !k.field && m->max_members <= 2) ? 2 : 3;
-    // chains with constraints or a bias: one wave, one move at a time
+    // chains with constraints or a bias: one wave, one move at a time (or
+    // patches, below)
     k.hooks = !b->hooks.empty() && b->hooks[c].on;
     if (k.hooks) {
       k.field = false;
@@ -1961,26 +1963,32 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     // 19.4, 19.6 ms; a mix of 48 chains 2.25, 1.83, 1.78 ms; one binary
     // chain 12.0 ms with any.  128 quaternary chains with 2, 4 and 8 waves:
     // 31, 21 and 18 ms.
-    if (forced_waves == 0 && b->spec_moves == 0 && !k.field && !k.hooks && !m->patches.empty() &&
-        (!canon || m->n_sites <= 65535)) {
+    // Chains with a constraint on the state (a pair constraint, a site open to
+    // some species, fixed species of SGC chains) or waste recycling stay on
+    // the one-move kernel.
+    if (forced_waves == 0 && b->spec_moves == 0 && !k.field && (!k.hooks || b->hooks[c].by_proposal) &&
+        !m->patches.empty() && (!canon || m->n_sites <= 65535)) {
       const int P = int(m->patches.size());
       const uint32_t room = limit + sweep_static_lds() - kPatchStaticLds;
       int waves = P <= 64 ? std::min(batch_waves, 4) : std::max(2, batch_waves);
       if (P > 60 && waves == 1) waves = 2;
-      const int kg = P > 64 ? 64 : (waves == 1 ? 4 : 16);
+      if (k.hooks) waves = 1;
+      const int kg = k.hooks ? 8 : (P > 64 ? 64 : (waves == 1 ? 4 : 16));
       int kr = 0;
       for (int r : {3, 6, 9, 15})
         if (kg == 4 && kr == 0 && P <= 4 * r) kr = r;
       for (int r : {1, 2, 4, 7})
-        if (kg != 4 && kr == 0 && P <= kg * r) kr = r;
+        if (kg >= 16 && kr == 0 && P <= kg * r) kr = r;
+      for (int r : {2, 4, 8})
+        if (kg == 8 && kr == 0 && P <= kg * r) kr = r;
       const int near_slots = canon && kg != 64 ? kg * kr : 0;
       bool trk_lds = true;
       uint32_t need = patch_lds_bytes(occ_bytes, trk_sites, int(m->ptab.size()), near_slots);
-      if (canon && need > room) {
+      if (canon && kg == 64 && need > room) {
         trk_lds = false;
         need = patch_lds_bytes(occ_bytes, 0, int(m->ptab.size()), near_slots);
       }
-      if (kr > 0 && need <= room && patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon)) {
+      if (kr > 0 && need <= room && patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon, k.hooks)) {
         k.kg = kg;
         k.kr = kr;
         k.waves = waves;
@@ -3228,6 +3236,7 @@ int cemc_batch_set_hooks(cemc_batch* b, int32_t chain, const cemc_hooks_desc* d)
       std::vector<int8_t> occ(static_cast<size_t>(N));
       HIP_CHECK(hipMemcpy(occ.data(), b->d_occ + b->params[chain].occ_off, size_t(N), hipMemcpyDeviceToHost));
       HookDev& v = h.dev;
+      h.by_proposal = true;
       v.fixed_species = d->fixed_species;
       v.max_attempts = d->max_attempts;
       v.pair_e1 = v.pair_e2 = -1;
@@ -3235,6 +3244,8 @@ int cemc_batch_set_hooks(cemc_batch* b, int32_t chain, const cemc_hooks_desc* d)
       v.recycle = d->recycle_waste ? 1 : 0;
       if (d->allowed) {
         for (int i = 0; i < N; ++i) require((d->allowed[i] >> S) == 0, "allowed-species mask names unknown species");
+        const int any = (1 << S) - 1;
+        h.by_proposal = std::all_of(d->allowed, d->allowed + N, [&](uint8_t v) { return v == 0 || v == any; });
         h.d_allowed = upload(std::vector<uint8_t>(d->allowed, d->allowed + N));
         v.allowed = h.d_allowed;
       }
@@ -3274,6 +3285,8 @@ int cemc_batch_set_hooks(cemc_batch* b, int32_t chain, const cemc_hooks_desc* d)
         v.bias_energy = tab[size_t(cnt)];
         st.energy += v.bias_energy;
       }
+      h.by_proposal = h.by_proposal && v.pair_e1 < 0 && v.recycle == 0 &&
+                      (v.fixed_species == 0 || b->params[chain].kind == CEMC_MOVE_CANONICAL);
       h.on = true;
     }
     HIP_CHECK(hipMemcpy(&b->d_states[chain].energy, &st.energy, sizeof(double), hipMemcpyHostToDevice));

@@ -26,11 +26,11 @@ struct LaunchSweep {
   int kbm;         // decoration slices read per record: n_bfs for up to 4 species (1, 2, 3), else 7
   int waves;       // wavefronts per chain: 1, 2, 4 or 8 (more than 1: kr > 0)
   int spec;        // moves per round: 1, or kSpecMoves (periodic, kr > 0)
-  int kg;          // patch kernel (ce_patch_kernel.h): lanes per move, 4, 16 or 64 (0: the sweep kernel); kr is then
-                   // the patches per lane
+  int kg;          // patch kernel (ce_patch_kernel.h): lanes per move, 4, 8 (hooks), 16 or 64 (0: the sweep kernel);
+                   // kr is then the patches per lane
   bool trk_lds;    // patch kernel: the tracker is held in LDS
   bool field;      // local-field kernel (periodic, one wave, kr > 0, kbm <= 3)
-  HookDev* hooks;  // per chain constraints and bias (one wave, one move per round), or nullptr
+  HookDev* hooks;  // per chain constraints and bias (one wave; sweep kernel: one move per round), or nullptr
   int nm;          // members gathered per record: 3, or 2 for records in VGPRs of models without quadruplets
   uint32_t* accept_log;  // optional: bit t of chain c at accept_log[c * log_words + t / 32]
   int64_t log_words;
@@ -52,7 +52,7 @@ uint32_t field_lds_bytes(int occ_bytes, int trk_sites, int n_fields, int gtab_in
 // kernel's static LDS.
 uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles, int near_slots);
 constexpr uint32_t kPatchStaticLds = 7u * 1024u;  // bound, checked when the limits are raised
-bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool canonical);
+bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool canonical, bool hooks = false);
 // Raises the dynamic-LDS limit of every sweep kernel instantiation to
 // `bytes` minus that kernel's static LDS.
 hipError_t sweep_set_max_lds(uint32_t bytes);

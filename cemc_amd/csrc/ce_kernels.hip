@@ -959,23 +959,23 @@ CEMC_DECLARE_SWEEP_FN(8, 0)
 CEMC_DECLARE_SWEEP_FN(8, 1)
 #undef CEMC_DECLARE_SWEEP_FN
 
-const void* patch_fn_w1(bool canonical, int kbm, int kg, int kr, bool trk_lds);
-const void* patch_fn_w2(bool canonical, int kbm, int kg, int kr, bool trk_lds);
-const void* patch_fn_w4(bool canonical, int kbm, int kg, int kr, bool trk_lds);
-const void* patch_fn_w8(bool canonical, int kbm, int kg, int kr, bool trk_lds);
+const void* patch_fn_w1(bool canonical, int kbm, int kg, int kr, bool trk_lds, bool hooks);
+const void* patch_fn_w2(bool canonical, int kbm, int kg, int kr, bool trk_lds, bool hooks);
+const void* patch_fn_w4(bool canonical, int kbm, int kg, int kr, bool trk_lds, bool hooks);
+const void* patch_fn_w8(bool canonical, int kbm, int kg, int kr, bool trk_lds, bool hooks);
 
-static const void* patch_fn(bool canonical, int kbm, int kg, int kr, int waves, bool trk_lds) {
+static const void* patch_fn(bool canonical, int kbm, int kg, int kr, int waves, bool trk_lds, bool hooks = false) {
   switch (waves) {
-    case 1: return patch_fn_w1(canonical, kbm, kg, kr, trk_lds);
-    case 2: return patch_fn_w2(canonical, kbm, kg, kr, trk_lds);
-    case 4: return patch_fn_w4(canonical, kbm, kg, kr, trk_lds);
-    case 8: return patch_fn_w8(canonical, kbm, kg, kr, trk_lds);
+    case 1: return patch_fn_w1(canonical, kbm, kg, kr, trk_lds, hooks);
+    case 2: return patch_fn_w2(canonical, kbm, kg, kr, trk_lds, hooks);
+    case 4: return patch_fn_w4(canonical, kbm, kg, kr, trk_lds, hooks);
+    case 8: return patch_fn_w8(canonical, kbm, kg, kr, trk_lds, hooks);
     default: return nullptr;
   }
 }
 
-bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool canonical) {
-  return patch_fn(canonical, kbm, kg, kr, waves, trk_lds) != nullptr;
+bool patch_variant_ok(int kbm, int kg, int kr, int waves, bool trk_lds, bool canonical, bool hooks) {
+  return patch_fn(canonical, kbm, kg, kr, waves, trk_lds, hooks) != nullptr;
 }
 
 uint32_t patch_lds_bytes(int occ_bytes, int trk_sites, int tab_doubles, int near_slots) {
@@ -1069,8 +1069,8 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
       for (int kg : {4, 8, 16, 64})
         for (int kr : {1, 2, 3, 4, 6, 7, 8, 9, 15})
           for (int kbm : {1, 2, 3})
-            for (int tl = 0; tl < 2; ++tl) {
-              const void* fn = patch_fn(cn != 0, kbm, kg, kr, w, tl != 0);
+            for (int tl = 0; tl < 3; ++tl) {
+              const void* fn = patch_fn(cn != 0, kbm, kg, kr, w, tl != 0, tl == 2);
               if (fn == nullptr) continue;
               hipFuncAttributes attr;
               hipError_t e = hipFuncGetAttributes(&attr, fn);
@@ -1100,8 +1100,8 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
 hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   const void* fn = nullptr;
   if (a.kg != 0) {
-    if (!a.periodic || a.field || a.hooks != nullptr) return hipErrorInvalidValue;
-    fn = patch_fn(a.canonical, a.kbm, a.kg, a.kr, a.waves, a.trk_lds);
+    if (!a.periodic || a.field || (a.kg == 8) != (a.hooks != nullptr)) return hipErrorInvalidValue;
+    fn = patch_fn(a.canonical, a.kbm, a.kg, a.kr, a.waves, a.trk_lds, a.hooks != nullptr);
   } else if (a.field) {
     if (!a.periodic || a.waves != 1 || a.hooks != nullptr) return hipErrorInvalidValue;
     fn = field_fn(a.canonical, a.kr, a.kbm);
@@ -1125,7 +1125,7 @@ hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   int64_t time_limit = a.time_limit;
   if (a.kg != 0) {
     PatchArgs p{params, states, models, occ_pool, trk_pool, order, n_moves, log, log_words, time_limit,
-                nullptr, nullptr, nullptr, nullptr, 0, 0};
+                nullptr, nullptr, nullptr, nullptr, 0, 0, hooks};
     void* pargs[] = {&p};
     return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), pargs, a.lds_bytes, stream);
   }
@@ -1145,7 +1145,7 @@ hipError_t launch_wl(const LaunchWL& a, hipStream_t stream) {
     const void* pfn = patch_fn(!a.sgc, a.kbm, 8, a.patch_kr, 1, true);
     if (pfn == nullptr || a.shared != nullptr || a.adaptive) return hipErrorInvalidValue;
     PatchArgs p{a.params, a.states, a.models, a.occ_pool, a.trk_pool, a.chain_order, nullptr, a.accept_log, a.log_words,
-                0, a.walkers, a.logdos, a.hist, a.known, a.n_checks, a.check_every};
+                0, a.walkers, a.logdos, a.hist, a.known, a.n_checks, a.check_every, nullptr};
     void* pargs[] = {&p};
     return hipLaunchKernel(pfn, dim3(a.n_chains), dim3(64), pargs, a.lds_bytes, stream);
   }

@@ -1,10 +1,10 @@
 // Instantiations of the patch kernel for one number of waves per chain,
 // CEMC_PATCH_WAVES (1, 2, 4, 8), one object each; exposes
-// patch_fn_w<W>(canonical, kbm, kg, kr, trk_lds), the kernel's address or nullptr
-// for a variant that is not built.  One wave: a quad per move, up to 60
+// patch_fn_w<W>(canonical, kbm, kg, kr, trk_lds, hooks), the kernel's address or
+// nullptr for a variant that is not built.  One wave: a quad per move, up to 60
 // patches; two or four waves: a row of 16 lanes per move, up to 64 patches;
 // two, four or eight waves: a wave per move, up to 448 patches.  kg 8: the
-// Wang-Landau kernel.
+// Wang-Landau kernel, or (hooks) chains with constraints or a bias.
 #include "ce_patch_kernel.h"
 
 #ifndef CEMC_PATCH_WAVES
@@ -33,13 +33,13 @@ const void* row_fn(int kr) {
   return nullptr;
 }
 
-// Wang-Landau walkers: eight lanes per move, up to 64 patches
-template <bool C, int KBM>
-const void* walker_fn(int kr) {
+// Wang-Landau walkers, or chains with hooks (H): eight lanes per move, up to 64 patches
+template <bool C, int KBM, bool H>
+const void* octet_fn(int kr) {
   if constexpr (W == 1) {
-    if (kr == 2) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 2, 1, 1, true, true>);
-    if (kr == 4) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 4, 1, 1, true, true>);
-    if (kr == 8) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 8, 1, 1, true, true>);
+    if (kr == 2) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 2, 1, 1, true, !H, H>);
+    if (kr == 4) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 4, 1, 1, true, !H, H>);
+    if (kr == 8) return reinterpret_cast<const void*>(&patch_kernel<C, KBM, 8, 8, 1, 1, true, !H, H>);
   }
   return nullptr;
 }
@@ -55,14 +55,19 @@ const void* wave_fn(int kr) {
   return nullptr;
 }
 
+template <bool C, bool H>
+const void* pick_octet(int kbm, int kr) {
+  return kbm == 1 ? octet_fn<C, 1, H>(kr) : (kbm == 2 ? octet_fn<C, 2, H>(kr) : (kbm == 3 ? octet_fn<C, 3, H>(kr) : nullptr));
+}
+
 template <bool C>
-const void* pick(int kbm, int kg, int kr, bool trk_lds) {
+const void* pick(int kbm, int kg, int kr, bool trk_lds, bool hooks) {
+  if (kg == 8) return hooks ? pick_octet<C, true>(kbm, kr) : pick_octet<C, false>(kbm, kr);
+  if (hooks) return nullptr;
   if (kg == (W == 1 ? 4 : 16)) {
     if (!trk_lds) return nullptr;
     return kbm == 1 ? row_fn<C, 1>(kr) : (kbm == 2 ? row_fn<C, 2>(kr) : (kbm == 3 ? row_fn<C, 3>(kr) : nullptr));
   }
-  if (kg == 8)
-    return kbm == 1 ? walker_fn<C, 1>(kr) : (kbm == 2 ? walker_fn<C, 2>(kr) : (kbm == 3 ? walker_fn<C, 3>(kr) : nullptr));
   if (kg != 64) return nullptr;
   if (!C || trk_lds)
     return kbm == 1 ? wave_fn<C, 1, true>(kr)
@@ -75,8 +80,8 @@ const void* pick(int kbm, int kg, int kr, bool trk_lds) {
 #define CEMC_PATCH_FN_NAME2(W_) patch_fn_w##W_
 #define CEMC_PATCH_FN_NAME(W_) CEMC_PATCH_FN_NAME2(W_)
 
-const void* CEMC_PATCH_FN_NAME(CEMC_PATCH_WAVES)(bool canonical, int kbm, int kg, int kr, bool trk_lds) {
-  return canonical ? pick<true>(kbm, kg, kr, trk_lds) : pick<false>(kbm, kg, kr, trk_lds);
+const void* CEMC_PATCH_FN_NAME(CEMC_PATCH_WAVES)(bool canonical, int kbm, int kg, int kr, bool trk_lds, bool hooks) {
+  return canonical ? pick<true>(kbm, kg, kr, trk_lds, hooks) : pick<false>(kbm, kg, kr, trk_lds, hooks);
 }
 
 }  // namespace cemc

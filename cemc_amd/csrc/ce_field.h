@@ -154,6 +154,8 @@ __global__ __launch_bounds__(64) void field_kernel(const ChainParams* __restrict
   c.DZ = c.L3;
   c.K = m.K;
   c.trans = m.trans;
+  c.trans_in_lds = false;
+  c.trans_l = nullptr;
 
   // ---- stage the lattice (padded box and the site of every cell), the
   // tracker, the integer tables and the species tables

@@ -1561,6 +1561,7 @@ struct cemc_batch {
     int nm;      // members gathered per record
     int kg;      // patch kernel: lanes per move (0: another kernel)
     bool trk_lds;  // patch kernel: the tracker in LDS
+    bool trans_lds;  // sweep kernel: the translation table in LDS
     int begin, count;
     uint32_t lds;
   };
@@ -1793,6 +1794,7 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     int nm;
     int kg = 0;
     bool trk_lds = true;
+    bool trans_lds = false;
     uint32_t lds;
   };
   // waves per chain: enough chains x waves to give every SIMD of the
@@ -1954,6 +1956,16 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       }
       k.nm = (k.kr > 0 && m->max_members <= 2) ? 2 : 3;
     }
+    // Table lattices: the translation table and the sites' groups in LDS, a
+    // look-up per member and one per flip, where they fit and every chain is
+    // still resident at once.
+    if (!m->periodic && m->n_sites <= 65535 && int64_t(m->n_sites) * m->K < int64_t(limit)) {
+      const uint32_t more = k.lds + sweep_trans_bytes(m->n_sites, m->K);
+      if (more <= limit && on_device <= int64_t(n_cu) * (kUnitLds / (more + sweep_static_lds() + 256u))) {
+        k.trans_lds = true;
+        k.lds = more;
+      }
+    }
     // patches, where no launch shape was asked for.  Up to 64 patches: about
     // one wave per SIMD over the device as above, four at most, which then
     // evaluate a round of 16 moves together (one wave: a quad per move;
@@ -2011,7 +2023,7 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       if (done[c] || k.periodic != k0.periodic || k.canonical != k0.canonical || k.kr != k0.kr ||
           k.glds != k0.glds || k.kbm != k0.kbm || k.waves != k0.waves || k.spec != k0.spec ||
           k.field != k0.field || k.hooks != k0.hooks || k.nm != k0.nm || k.kg != k0.kg ||
-          k.trk_lds != k0.trk_lds)
+          k.trk_lds != k0.trk_lds || k.trans_lds != k0.trans_lds)
         continue;
       done[c] = true;
       ids.push_back(c);
@@ -2023,7 +2035,8 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
       return int64_t(mx->n_sites) * mx->recs.size() > int64_t(my->n_sites) * my->recs.size();
     });
     b->classes.push_back(cemc_batch::Class{k0.periodic, k0.canonical, k0.kr, k0.glds, k0.kbm, k0.waves, k0.spec,
-                                           k0.field, k0.hooks, k0.nm, k0.kg, k0.trk_lds, int(order.size()), int(ids.size()), lds});
+                                           k0.field, k0.hooks, k0.nm, k0.kg, k0.trk_lds, k0.trans_lds,
+                                           int(order.size()), int(ids.size()), lds});
     order.insert(order.end(), ids.begin(), ids.end());
   }
   if (order.size() > b->order_cap || b->d_order == nullptr) {
@@ -2109,6 +2122,7 @@ void enqueue_sweeps(cemc_batch* b, uint32_t* d_log, int64_t log_words, int64_t t
     a.nm = cl.nm;
     a.kg = cl.kg;
     a.trk_lds = cl.trk_lds;
+    a.trans_lds = cl.trans_lds;
     a.accept_log = d_log;
     a.log_words = log_words;
     a.time_limit = time_limit;

@@ -38,11 +38,14 @@ struct LaunchSweep {
   // more than time_limit ticks of the constant-rate wall clock after the
   // chain's own start (0: no limit; ignored by the local-field kernel)
   int64_t time_limit = 0;
+  bool trans_lds = false;  // sweep kernel, table lattices: translation table and groups in LDS
 };
 
 // Dynamic LDS of one chain: occupation bytes (padded box on periodic
 // lattices), tracker entries (canonical chains), records held in LDS, table doubles.
 uint32_t sweep_lds_bytes(int occ_bytes, int trk_sites, int n_rec_lds, int gtab_doubles);
+// What a translation table of K columns and the sites' groups add to it.
+uint32_t sweep_trans_bytes(int n_sites, int K);
 bool sweep_variant_ok(int kr, bool gtab_lds, int kbm, int waves, int spec, bool periodic);
 // Dynamic LDS of one chain on the local-field kernel: padded occupation and
 // its site map, tracker entries, n_sites x B integer fields, integer tables.

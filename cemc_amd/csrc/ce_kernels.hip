@@ -33,6 +33,10 @@ uint32_t sweep_lds_bytes(int occ_bytes, int trk_sites, int n_rec_lds, int gtab_d
   return lds_layout(occ_bytes, trk_sites, n_rec_lds, gtab_doubles).total;
 }
 
+uint32_t sweep_trans_bytes(int n_sites, int K) {
+  return align16(uint32_t(n_sites) * uint32_t(K) * 2u) + align16(uint32_t(n_sites));
+}
+
 
 // ---------------------------------------------------------------------------
 // Correlation functions from scratch.  Block b of chain c counts, over the
@@ -1133,8 +1137,9 @@ hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
     void* fargs[] = {&params, &states, &models, &occ_pool, &trk_pool, &order, &n_moves, &log, &log_words, &hooks};
     return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), fargs, a.lds_bytes, stream);
   }
+  int trans_lds = a.trans_lds ? 1 : 0;
   void* args[] = {&params, &states, &models, &occ_pool, &trk_pool, &order, &n_moves, &log, &log_words, &hooks,
-                  &time_limit};
+                  &time_limit, &trans_lds};
   return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), args, a.lds_bytes, stream);
 }
 

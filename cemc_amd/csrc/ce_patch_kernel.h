@@ -217,6 +217,8 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
   c.DZ = c.L3;
   c.K = 0;
   c.trans = nullptr;
+  c.trans_in_lds = false;
+  c.trans_l = nullptr;
   const uint64_t im0 = m.imask[0], im1 = m.imask[1];
   const int occ_bytes = m.pdims[0] * c.P2 * c.P3;
   const PatchLayout L =

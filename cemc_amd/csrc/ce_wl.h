@@ -147,6 +147,8 @@ __global__ __launch_bounds__(64) void wl_kernel(const ChainParams* __restrict__ 
   c.DZ = c.L3;
   c.K = m.K;
   c.trans = m.trans;
+  c.trans_in_lds = false;
+  c.trans_l = nullptr;
   const bool multi_group = m.n_groups > 1 || m.has_background;
 
   // A lattice in site order (global memory) into the LDS occupation: on

@@ -27,25 +27,25 @@ sys.path.insert(0, ROOT)
 METRIC = "aggregate MC trial moves/sec at 1 MI355X (batched vs plain); p50/p99 job latency"
 HBM_PEAK_GBS = 8000.0
 # HBM bytes of one SGC launch of the default workload (1024 chains x 500
-# sweeps, 1 wave per chain, rounds of 8 moves): FETCH_SIZE and WRITE_SIZE per
-# dispatch, each scaled by what the counter reads for a copy kernel of known
-# size (x2.0 and x1.0).  Measured with rocprofv3 --pmc; summary in
-# profiles/sweep_kernel_sgc_binary_fcc10_1024chains.txt
-TRAFFIC_DEFAULT_LAUNCH = 3686400
-TRAFFIC_SHAPE = (1, 8, 1)
+# sweeps, automatic shape: patch kernel, 1 wave per chain): FETCH_SIZE and
+# WRITE_SIZE per dispatch, each scaled by what the counter reads for a copy
+# kernel of known size (x2.0 and x1.0).  Measured with rocprofv3 --pmc; summary
+# in profiles/kernels_by_workload.txt
+TRAFFIC_DEFAULT_LAUNCH = 3728000
+TRAFFIC_SHAPE = (0, 0, 0)  # autotune.AUTO
 
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-# What bounds the sweep kernel: neither bandwidth (the algorithmic bytes are
-# a few % of the measured LDS read rate and the lattices never leave LDS
-# during a launch) but each chain's dependent move sequence (evaluate ->
-# reduce -> decide -> commit), which the profiles' SQ counters show as a low
-# VALU issue fraction and waves that wait on their LDS and HBM table reads.
-LIMITER = ("latency of each chain's dependent move sequence: per-chain issue and LDS/L2 latency, not HBM or "
-           "LDS bandwidth (SQ counters in profiles/)")
+# What bounds the kernels: neither bandwidth (the lattices never leave LDS
+# during a launch) but each chain's dependent move sequence (gather -> table ->
+# sum -> decide -> commit), see the SQ counters in profiles/.  The algorithmic
+# bytes count one gather per member of every sub-cluster; the patch tables
+# answer them with fewer, so the fraction may exceed one.
+LIMITER = ("issue and LDS latency of each chain's dependent move sequence, not HBM bandwidth; algorithmic bytes count "
+           "every sub-cluster's members, which the patch tables need not gather (SQ counters in profiles/)")
 
 
 def roofline_of(algorithmic_bytes, kernel_ms, lds_peak):

@@ -34,11 +34,12 @@
 // once per launch.  Four-species models are bound by LDS reads instead (two
 // thirds of the cycles at eight waves).
 //
-// Measured against the sweep kernel's automatic shapes, per pass: 1024 binary
-// SGC chains of 500 sweeps 150 -> 71.5 ms, 256 ternary chains of 512-4096
-// sites 55.6 -> 18.9 ms, a mix of 48 binary and ternary chains 5.8 -> 1.8 ms,
-// 128 quaternary 32^3 replicas 56.7 -> 16.5 ms, one binary chain 23.9 -> 11.7
-// ms, 128 quaternary 8^3 chains 5.4 -> 3.0 ms (1.2 ms of it the kernel).
+// Measured against the sweep kernel's automatic shapes, per pass with its reads
+// of the results: 1024 binary SGC chains of 500 sweeps 150 -> 63.6 ms (the
+// kernel 134 -> 54), 256 ternary chains of 512-4096 sites 55.6 -> 18.0 ms, a mix
+// of 48 binary and ternary chains 5.8 -> 1.6 ms, 128 quaternary 32^3 replicas
+// 56.7 -> 16.6 ms, one binary chain 23.9 -> 11.7 ms, 128 quaternary 8^3 chains
+// 5.4 -> 2.3 ms (1.25 ms of it the kernel).
 #pragma once
 
 #include "ce_wl.h"

@@ -42,6 +42,7 @@
 // 5.4 -> 2.3 ms (1.25 ms of it the kernel).
 #pragma once
 
+#include "ce_patches.h"
 #include "ce_wl.h"
 
 namespace cemc {
@@ -281,8 +282,8 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
   }
   if constexpr (kNear)
     for (int i = tid; i < kNearCells * kSlots; i += kThreads) near_w[i] = 0;
-  // slots that a round does not fill hold a move from before; at first the
-  // cell (0, 0, 0)
+  // slots that a round does not fill hold a move from before (its sites are
+  // read, slot_swap takes its species as unchanged); at first the cell (0, 0, 0)
   if (lane < kK) {
     const uint32_t p0 = uint32_t((c.h * c.P2 + c.h) * c.P3 + c.h);
     slot_a[wave][lane] = kCanonical ? uint4{p0, p0, uint32_t(kNearCells - 1), 0} : uint4{p0, 0, p0, 0};
@@ -654,7 +655,11 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
       uint4 ca[kCom];
       uint2 cimg[kCom], cs[kCom];
 #pragma unroll
-      for (int t = 0; t < kP; ++t) ev[t] = my_a[(wave * kP + t) * kPer + (kG == 64 ? 0 : lane / kG)];
+      for (int t = 0; t < kP; ++t) {
+        const int slot = (wave * kP + t) * kPer + (kG == 64 ? 0 : lane / kG);
+        ev[t] = my_a[slot];
+        if constexpr (kCanonical) ev[t].w = slot_swap(ev[t].w, slot, n);
+      }
 #pragma unroll
       for (int v = 0; v < kPairs; ++v) {
         if constexpr (kCanonical) {

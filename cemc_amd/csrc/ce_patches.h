@@ -1,5 +1,5 @@
 // Patches: the sub-clusters of a site regrouped so that one table read covers
-// many of them.  Host code only (no HIP), so that it can be checked on the CPU.
+// many of them.  No HIP in here, so that it can be checked on the CPU.
 //
 // A flip of a site sums one table entry per sub-cluster that holds the site,
 // each chosen by the species of at most three other members.  Sub-clusters
@@ -34,6 +34,13 @@ constexpr int kPatchSites = 96;    // most distinct member sites the search take
 // Members per patch by species count: tables of S^q codes, 64 (two species),
 // 243 (three) and 256 (four), which keep every table of a model in LDS.
 inline int patch_members(int n_species) { return n_species == 2 ? 6 : (n_species == 3 ? 5 : (n_species == 4 ? 4 : 0)); }
+
+// Species a | b << 8 of the swap in slot `slot` of a round of n moves; `w` is
+// what the slot holds.  Slots past the last move hold a swap of an earlier
+// round: made since, it would shift its first site's species a second time and
+// index past the patch's table, so it counts as no swap.  (constexpr: the
+// kernel calls it too.)
+constexpr uint32_t slot_swap(uint32_t w, int slot, int n) { return slot < n ? w & 0xFFFFu : 0u; }
 
 // One sub-cluster as seen from the reference site: its other members (site
 // ids 0 .. n_sites-1 of the search) in code order, its table block, and the

@@ -696,7 +696,7 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
       // other where their members and entries would overflow the registers
       constexpr int kF = kCanonical ? 2 : 1;  // flips per move
       constexpr int kFlips = kP * kF;
-      constexpr int kT = kFlips * kR * kQ <= 100 ? kFlips : 1;
+      constexpr int kAtOnce = kFlips * kR * kQ <= 100 ? kFlips : 1;
       Axes ax[kPairs][kCanonical ? 4 : 1];
       uint32_t c_o[kCom], d_s = 0;
       auto other_loads = [&] {
@@ -725,12 +725,12 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
         }
       };
 #pragma unroll
-      for (int f0 = 0; f0 < kFlips; f0 += kT) {
-        Members mem[kT];
-        uint32_t near[kT][kNear ? kR : 1];
-        uint32_t own[kT];
+      for (int f0 = 0; f0 < kFlips; f0 += kAtOnce) {
+        Members mem[kAtOnce];
+        uint32_t near[kAtOnce][kNear ? kR : 1];
+        uint32_t own[kAtOnce];
 #pragma unroll
-        for (int u = 0; u < kT; ++u) {
+        for (int u = 0; u < kAtOnce; ++u) {
           const uint4 e = ev[(f0 + u) / kF];
           const bool second = kCanonical && (f0 + u) % 2 == 1;  // site j of a swap
           if constexpr (!kCanonical && kBM > 1) own[u] = occ[e.x];
@@ -741,10 +741,10 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
         }
         if (f0 == 0) other_loads();
         phase();
-        Entries g[kT];
-        double dphi[kT][kBM];
+        Entries g[kAtOnce];
+        double dphi[kAtOnce][kBM];
 #pragma unroll
-        for (int u = 0; u < kT; ++u) {
+        for (int u = 0; u < kAtOnce; ++u) {
           const uint4 e = ev[(f0 + u) / kF];
           const bool second = kCanonical && (f0 + u) % 2 == 1;
           int idx[kR];
@@ -775,7 +775,7 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
         if (f0 == 0) other_masks();
         phase();
 #pragma unroll
-        for (int u = 0; u < kT; ++u) {
+        for (int u = 0; u < kAtOnce; ++u) {
           const double v = total(g[u], dphi[u]);
           const int t = (f0 + u) / kF;
           if (kCanonical && (f0 + u) % 2 == 1)

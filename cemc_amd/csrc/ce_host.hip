@@ -2393,9 +2393,11 @@ void wl_launch(cemc_batch* b, int64_t n_checks, int64_t check_every, uint32_t* h
     k.glds = with_g <= std::min(kGtabLdsBudget, limit);
     uint32_t lds = k.glds ? with_g : no_g;
     // a histogram of its own, no windows: the patch kernel's rounds of eight
+    // (its bins per eV have to be finite)
     k.patch_kr = 0;
     const int P = int(m->patches.size());
-    if (!shared && !adaptive && P > 0 && P <= 64 && (k.sgc || m->n_sites <= 65535)) {
+    if (!shared && !adaptive && P > 0 && P <= 64 && (k.sgc || m->n_sites <= 65535) &&
+        std::isfinite(double(nbins) / (b->wl[c].e_max - b->wl[c].e_min))) {
       const int kr = P <= 16 ? 2 : (P <= 32 ? 4 : 8);
       const uint32_t need = patch_lds_bytes(occ_bytes, k.sgc ? 0 : m->n_sites, int(m->ptab.size()),
                                             k.sgc ? 0 : 8 * kr) + 16u * uint32_t(nbins);

@@ -836,10 +836,11 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
         for (; k < n; ++k) {
           if ((uint32_t(__builtin_amdgcn_readlane(int(conf_d), k)) & com) != 0) break;
           const double e_new = energy + readlane_f64(dE, k);
-          // Truncated bin (histogram.cpp:66-69; the conversion saturates) from
-          // a product; its rounding is below 1e-8 inside any histogram that
-          // fits here, so only near an edge the quotient itself is formed.
-          const double q = (e_new - e_min) * bins_per_ev;
+          // Truncated bin (histogram.cpp:66-69) from a product; its rounding is
+          // below 1e-8 inside any histogram that fits here, so only near an
+          // edge the quotient itself is formed.  Clamped before the
+          // conversion: far outside stays outside, and NaN lies below.
+          const double q = fmin(fmax((e_new - e_min) * bins_per_ev, -1e9), 1e9);
           int raw = int(q - 1e-8);
           if (any(raw != int(q + 1e-8)))
             raw = int(fmin(fmax(trunc((e_new - e_min) * nbd / span), -2147483648.0), 2147483647.0));

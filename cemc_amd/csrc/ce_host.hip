@@ -435,6 +435,15 @@ void cemc_model::build_patches() {
   ptab_base.clear();
   const int q = patch_members(n_species);
   if (q == 0 || !spec_ok || std::max({dims[0], dims[1], dims[2]}) > 127) return;
+  // The kernel makes moves past a blocked one: these must not write what the
+  // blocked one reads, and only whether it reaches them is tested.  So a site
+  // has to reach the sites that reach it (sub-clusters listed for each of
+  // their sites, as every lattice of the package lists them).
+  const int box = (2 * pad_h + 1) * (2 * pad_h + 1) * (2 * pad_h + 1);
+  for (int i = 0; i < box; ++i) {
+    const int j = box - 1 - i;  // the opposite offset
+    if ((imask[i >> 6] >> (i & 63) & 1u) != (imask[j >> 6] >> (j & 63) & 1u)) return;
+  }
   // per entry: the position permutations that keep every function
   std::vector<std::vector<std::array<int, 4>>> alike(n_entries);
   for (int c = 0; c < n_entries; ++c) {

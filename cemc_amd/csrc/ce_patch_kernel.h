@@ -10,8 +10,9 @@
 // evaluated against the same state.  A move that an accepted earlier one of
 // the round reaches (reads a site or shares a tracker slot with) is blocked,
 // and so is one that a blocked one reaches; the others are made at once, in
-// any order, since none reads what another writes.  Blocked moves stay open
-// for the next round.  (Ending the round at the first blocked move instead
+// any order, since none reads what another writes (interactions are mutual:
+// models where they are not have no patches).  Blocked moves stay open for the
+// next round.  (Ending the round at the first blocked move instead
 // made 5.6 moves of eight at the highest acceptances, now about 11 of 16.)
 //
 // Work split.  A flip needs 12 (two species, pairs to the 4th shell and

@@ -1,0 +1,51 @@
+"""Models at the edge of what the patch kernel takes, against the oracle."""
+import copy
+
+import numpy as np
+import pytest
+
+from cemc_amd.lattice import FCCSettings, random_occupation, seeded_ecis
+from oracle.brute_force import brute_force_cf
+from oracle.oracle import OracleModel, OracleUpdater
+
+pytestmark = pytest.mark.gpu
+
+
+def _chains_vs_oracle(s, eci, kind, temperature, n_moves, chains=1):
+    from cemc_amd.batch import ChainBatch
+    from cemc_amd.model import CEModel
+    S = len(s.unique_elements)
+    occ = random_occupation(s.n_sites, S, 3)
+    batch = ChainBatch([CEModel(s, eci)] * chains,
+                       [dict(kind=kind, temperature=temperature, occupation=occ, seed=3, uid=c) for c in range(chains)])
+    log = batch.run_logged(n_moves)
+    names = s.cf_names()
+    for c in {0, chains - 1}:
+        ora = OracleUpdater(OracleModel(s, names), occ, brute_force_cf(s, occ, names), eci)
+        bits, _, acc = ora.run(kind, 3, c, n_moves, temperature)
+        assert 0 < acc < n_moves
+        assert np.array_equal(np.unpackbits(log[c], bitorder="little")[:n_moves],
+                              np.unpackbits(bits, bitorder="little")[:n_moves])
+        assert np.array_equal(batch.occupation(c), ora.get_occupation())
+    return batch
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_one_sided_sub_clusters(gpu, kind):
+    """Pairs listed for one of their two sites only: a change at a site reaches
+    flips on one side of it, so a move past a blocked one may write what the
+    blocked one reads."""
+    s = copy.copy(FCCSettings((5, 5, 6), ["A", "B"], {2: 2}))
+    info = s.cluster_info[0]
+    dims = np.array(s.dims)
+    for name, cl in info.items():
+        if cl["size"] != 2:
+            continue
+        # keep the member whose wrapped offset comes first of +o and -o
+        keep = [k for k, sub in enumerate(cl["indices"])
+                if tuple(s.cells[sub[0]]) < tuple((-np.array(s.cells[sub[0]])) % dims)]
+        assert 2 * len(keep) == len(cl["indices"])
+        cl["indices"] = [cl["indices"][k] for k in keep]
+        cl["order"] = [cl["order"][k] for k in keep]
+    print("one-sided pairs", kind, flush=True)
+    _chains_vs_oracle(s, seeded_ecis(s, 5, 0.02), kind, 1200.0, 6000)

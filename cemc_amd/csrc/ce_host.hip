@@ -1991,7 +1991,13 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
         !m->patches.empty() && (!canon || m->n_sites <= 65535)) {
       const int P = int(m->patches.size());
       const uint32_t room = limit + sweep_static_lds() - kPatchStaticLds;
-      int waves = P <= 64 ? std::min(batch_waves, 4) : std::max(2, batch_waves);
+      // A pool's long job among crowds of 600-3000 short ones (chain_waves, 4
+      // waves against 1 or 2, moves per ms): swaps of two species 2590 ->
+      // 3320, three 3420 -> 4150, four 500 -> 650; flips of three 9660 ->
+      // 10300, four 1270 -> 1390, but of two 13300 -> 11400: a row has a lane
+      // for each of their 12 patches, and more waves only add barriers.
+      const int own = !canon && P <= 16 ? batch_waves : chain_waves;
+      int waves = P <= 64 ? std::min(own, 4) : std::max(2, own);
       if (P > 60 && waves == 1) waves = 2;
       if (k.hooks) waves = 1;
       const int kg = k.hooks ? 8 : (P > 64 ? 64 : (waves == 1 ? 4 : 16));

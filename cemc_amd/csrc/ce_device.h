@@ -177,8 +177,7 @@ struct ChainParams {
   uint64_t uid;
 };
 
-// Per-chain mutable state (kernel written).
-// Per-chain mutable state.  The sample sums run over the trial moves since
+// Per-chain mutable state (kernel written).  The sample sums run over the trial moves since
 // the last reset; each move samples the state after its accept/reject, as the
 // reference's observers do (cemc/mcmc/mc_observers.py:222-270).  Energies
 // enter relative to e_ref, the energy at that reset, which keeps the squared
@@ -196,7 +195,12 @@ struct ChainState {
   double sum_s[kMaxBasis];   // sum of singlet d
   double sum_s2[kMaxBasis];  // sum of singlet d squared
   double sum_se[kMaxBasis];  // sum of singlet d * (E - e_ref)
-  double pad1[3];
+  // patch kernel: a launch that ended inside a 64-move block of the stream left
+  // the block's energy changes behind (PatchArgs::tails), valid while energy
+  // and moves_done are still these
+  double blk_energy;   // energy at the block's start
+  double blk_end;      // energy
+  uint64_t blk_moves;  // moves_done
 };
 static_assert(sizeof(ChainState) == 256, "ChainState layout");
 

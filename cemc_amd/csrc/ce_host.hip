@@ -1554,6 +1554,7 @@ struct cemc_batch {
   ModelDev* d_models = nullptr;
   ChainParams* d_params = nullptr;
   ChainState* d_states = nullptr;
+  double* d_tails = nullptr;  // patch kernel: 64 per chain, made when a chain first runs on it
   int8_t* d_occ = nullptr;
   uint16_t* d_trk = nullptr;
   int64_t* d_nmoves = nullptr;
@@ -1640,6 +1641,7 @@ struct cemc_batch {
     dev_free(d_models);
     dev_free(d_params);
     dev_free(d_states);
+    dev_free(d_tails);
     dev_free(d_occ);
     dev_free(d_trk);
     dev_free(d_nmoves);
@@ -2054,6 +2056,8 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
                                            int(order.size()), int(ids.size()), lds});
     order.insert(order.end(), ids.begin(), ids.end());
   }
+  for (const auto& cl : b->classes)
+    if (cl.kg != 0 && b->d_tails == nullptr) HIP_CHECK(hipMalloc(&b->d_tails, sizeof(double) * 64 * size_t(n_chains)));
   if (order.size() > b->order_cap || b->d_order == nullptr) {
     dev_free(b->d_order);
     b->d_order = nullptr;
@@ -2138,6 +2142,7 @@ void enqueue_sweeps(cemc_batch* b, uint32_t* d_log, int64_t log_words, int64_t t
     a.kg = cl.kg;
     a.trk_lds = cl.trk_lds;
     a.trans_lds = cl.trans_lds;
+    a.tails = b->d_tails;
     a.accept_log = d_log;
     a.log_words = log_words;
     a.time_limit = time_limit;

@@ -38,6 +38,7 @@ struct LaunchSweep {
   // more than time_limit ticks of the constant-rate wall clock after the
   // chain's own start (0: no limit; ignored by the local-field kernel)
   int64_t time_limit = 0;
+  double* tails = nullptr;  // patch kernel: 64 doubles per chain (PatchArgs::tails)
   bool trans_lds = false;  // sweep kernel, table lattices: translation table and groups in LDS
 };
 

@@ -1110,7 +1110,7 @@ hipError_t sweep_set_max_lds(uint32_t bytes) {
 hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   const void* fn = nullptr;
   if (a.kg != 0) {
-    if (!a.periodic || a.field || (a.kg == 8) != (a.hooks != nullptr)) return hipErrorInvalidValue;
+    if (a.tails == nullptr || !a.periodic || a.field || (a.kg == 8) != (a.hooks != nullptr)) return hipErrorInvalidValue;
     fn = patch_fn(a.canonical, a.kbm, a.kg, a.kr, a.waves, a.trk_lds, a.hooks != nullptr);
   } else if (a.field) {
     if (!a.periodic || a.waves != 1 || a.hooks != nullptr) return hipErrorInvalidValue;
@@ -1135,7 +1135,7 @@ hipError_t launch_sweep(const LaunchSweep& a, hipStream_t stream) {
   int64_t time_limit = a.time_limit;
   if (a.kg != 0) {
     PatchArgs p{params, states, models, occ_pool, trk_pool, order, n_moves, log, log_words, time_limit,
-                nullptr, nullptr, nullptr, nullptr, 0, 0, hooks};
+                nullptr, nullptr, nullptr, nullptr, 0, 0, hooks, a.tails};
     void* pargs[] = {&p};
     return hipLaunchKernel(fn, dim3(a.n_chains), dim3(64 * a.waves), pargs, a.lds_bytes, stream);
   }
@@ -1156,7 +1156,7 @@ hipError_t launch_wl(const LaunchWL& a, hipStream_t stream) {
     const void* pfn = patch_fn(!a.sgc, a.kbm, 8, a.patch_kr, 1, true);
     if (pfn == nullptr || a.shared != nullptr || a.adaptive) return hipErrorInvalidValue;
     PatchArgs p{a.params, a.states, a.models, a.occ_pool, a.trk_pool, a.chain_order, nullptr, a.accept_log, a.log_words,
-                0, a.walkers, a.logdos, a.hist, a.known, a.n_checks, a.check_every, nullptr};
+                0, a.walkers, a.logdos, a.hist, a.known, a.n_checks, a.check_every, nullptr, nullptr};
     void* pargs[] = {&p};
     return hipLaunchKernel(pfn, dim3(a.n_chains), dim3(64), pargs, a.lds_bytes, stream);
   }

@@ -32,7 +32,9 @@
 // while the members are in flight; and what the next round does not need is
 // put off to the end of the block, where lane l holds move l: energies by one
 // prefix sum over the lanes, sample sums in per-lane accumulators added up
-// once per launch.  Four-species models are bound by LDS reads instead (two
+// once per launch.  Blocks are the 64-move blocks of the chain's stream, and a
+// launch that ends inside one leaves its energy changes to the next, so
+// energies do not depend on where launches end.  Four-species models are bound by LDS reads instead (two
 // thirds of the cycles at eight waves).
 //
 // Measured against the sweep kernel's automatic shapes, per pass with its reads
@@ -144,6 +146,9 @@ struct PatchArgs {
   int64_t n_checks, check_every;
   // constraints and bias
   HookDev* hooks;
+  // per chain the energy changes of a block that its last launch did not end
+  // (64, kRejected: none), valid as ChainState says
+  double* tails;
 };
 
 // kHook: chains with constraints or a bias whose constraints depend on the
@@ -354,6 +359,19 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
     first = wk->is_first;
     at_cur = bins[cur];  // the host checks 0 <= cur < nb
   }
+  if (!kWL && wave == 0) {
+    // A launch that starts inside a block takes over the changes that earlier
+    // launches made with the block's moves before it, and the energy at the
+    // block's start.  (Where the state was changed meanwhile: no change, and
+    // the energy as it is.)
+    const int k0 = int(t0 & 63u);
+    const ChainState& st = states[chain];
+    const bool carried =
+        k0 != 0 && st.blk_moves == t0 && __double_as_longlong(st.blk_end) == __double_as_longlong(energy);
+    if (carried) energy = st.blk_energy;
+    de_l[lane] = carried && lane < k0 ? args.tails[int64_t(chain) * 64 + lane] : __longlong_as_double(kRejected);
+    if constexpr (!kCanonical) on_l[lane] = 0;
+  }
   uint64_t n_acc = 0;
   double sum_de = 0.0, sum_de2 = 0.0;  // this lane's moves
   const double inv_n = 1.0 / double(N);
@@ -526,11 +544,13 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
   }
 
   uint32_t rnd = 0;
-  // One block: moves t_blk .. t_blk + n_in - 1 of the stream, n_in <= 64;
-  // accept bits from bit `log_at` of the chain's log.  Returns the moves made,
-  // n_in unless one of them has no valid proposal.
+  // One block: moves t_blk .. t_blk + n_in - 1 of the stream, n_in <= 64, from
+  // the launch's first move on; move t_blk has bit `log_at` of the chain's log
+  // (below 0: -log_at moves come before the launch).  Returns n_in, or less:
+  // the first move that has no valid proposal.
   auto make_block = [&](uint64_t t_blk, const int n_all, int64_t log_at) {
     int n_in = n_all;
+    const int lo = log_at < 0 ? -int(log_at) : 0;
     // lane l decodes move t_blk + l
     Philox4 blk = philox4x64_10(t_blk + uint64_t(lane), 0, 0, 0, seed, uid);
     // canonical: species a and b of a block's move, its tracker slots
@@ -554,7 +574,7 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
         bias_hi = at(bias_at + lane);
         bias_top = at(bias_at + 64);
       }
-      bool ok = lane >= n_in;
+      bool ok = lane < lo || lane >= n_in;
       for (int k = 0;;) {
         if (!ok) {
           if constexpr (kCanonical) {
@@ -620,11 +640,8 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
       v_a = uint4{uint32_t(r.p), uint32_t(r.x) | (uint32_t(r.y) << 8) | (uint32_t(r.z) << 16), image_word<true>(c, r),
                   bounded32(uint32_t(blk.w0), uint32_t(kS - 1)) | (uint32_t(lane) << 16)};
     }
-    if (kW == 1 || wave == 0) {
-      de_l[lane] = __longlong_as_double(kRejected);
-      if constexpr (!kCanonical) on_l[lane] = 0;
-    }
-    uint64_t open = n_in < 64 ? (uint64_t(1) << n_in) - 1u : ~uint64_t(0);  // moves not made yet
+    auto first_to_last = [&] { return (n_in < 64 ? (uint64_t(1) << n_in) - 1u : ~uint64_t(0)) & (~uint64_t(0) << lo); };
+    uint64_t open = first_to_last();  // moves not made yet
     while (open != 0) {
       // ---- the first kK open moves fill the slots
       const int rank = int(__builtin_amdgcn_mbcnt_hi(uint32_t(open >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(open), 0)));
@@ -972,15 +989,24 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
     if (!kWL && (kW == 1 || wave == 0)) {
       const double de = de_l[lane];
       const bool made = __double_as_longlong(de) != kRejected;
-      const uint64_t acc_bits = __builtin_amdgcn_ballot_w64(made);
+      const uint64_t acc_bits = __builtin_amdgcn_ballot_w64(made) & first_to_last();
       n_acc += uint64_t(__builtin_popcountll(acc_bits));
-      if (acc_log != nullptr && lane < 2) {
-        const int64_t w = log_at >> 5;
-        if (lane == 0) acc_log[w] = uint32_t(acc_bits);
-        if (lane == 1 && n_all > 32) acc_log[w + 1] = uint32_t(acc_bits >> 32);
+      if (acc_log != nullptr && lane < 3) {
+        const int64_t at = log_at + lo;
+        const int sh = int(at & 31);
+        const uint64_t bits = acc_bits >> lo;
+        const uint32_t part = lane == 0 ? uint32_t(bits << sh)
+                                        : (lane == 1 ? uint32_t(bits >> (32 - sh)) : (sh ? uint32_t(bits >> (64 - sh)) : 0u));
+        if (part != 0) atomicOr(acc_log + (at >> 5) + lane, part);
+      }
+      if (n_in < 64) {
+        // left to a launch that goes on here
+        args.tails[int64_t(chain) * 64 + lane] = de;
+        if (lane == 0) states[chain].blk_energy = energy;
       }
       const double e_l = energy + wave_scan_f64(made ? de : 0.0);
-      const double d = lane < n_in ? e_l - e_ref : 0.0;
+      const bool here = lane >= lo && lane < n_in;
+      const double d = here ? e_l - e_ref : 0.0;
       sum_de += d;
       sum_de2 = fma(d, d, sum_de2);
       energy = readlane_f64(e_l, 63);
@@ -990,13 +1016,15 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
         for (int b = 0; b < kBM; ++b) {
           const double ds = o == nw ? 0.0 : __dmul_rn(dphi_tab[(o * kS + nw) * kBM + b], inv_n);
           const double s_l = sing[b] + wave_scan_f64(ds);
-          const double s = lane < n_in ? s_l : 0.0;
+          const double s = here ? s_l : 0.0;
           sum_s[b] += s;
           sum_s2[b] = fma(s, s, sum_s2[b]);
           sum_se[b] = fma(s, d, sum_se[b]);
           sing[b] = readlane_f64(s_l, 63);
         }
       }
+      de_l[lane] = __longlong_as_double(kRejected);
+      if constexpr (!kCanonical) on_l[lane] = 0;
       own_order();
     }
     return n_in;
@@ -1082,7 +1110,7 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
   } else {
     const int64_t nmov = args.n_moves[chain];
     moves_made = nmov;
-    for (int64_t blk0 = 0; blk0 < nmov; blk0 += 64) {
+    for (int64_t blk0 = -int64_t(t0 & 63u); blk0 < nmov; blk0 += 64) {
       if (time_limit > 0 && blk0 > 0) {
         int stop = int(uint64_t(wall_clock64()) - t_begin > uint64_t(time_limit));
         if constexpr (kW > 1) {
@@ -1136,6 +1164,8 @@ __global__ __launch_bounds__(64 * kW) void patch_kernel(PatchArgs args) {
       st->n_samples += uint64_t(moves_made);
       st->sum_de += se;
       st->sum_de2 += se2;
+      st->blk_end = energy;
+      st->blk_moves = t0 + uint64_t(moves_made);
     }
     if constexpr (!kCanonical) {
 #pragma unroll

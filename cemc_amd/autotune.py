@@ -67,8 +67,10 @@ def tune(models, chains, candidates=(1, 2, 4, 8), per_round=(1, 8), fields=True,
     if cache_file and os.path.exists(cache_file):
         with open(cache_file) as f:
             _cache.update(json.load(f))
-    if sig in _cache:
-        entry = _cache[sig]
+    entry = _cache.get(sig)
+    # an entry from before the automatic choice was a candidate would keep the
+    # workload off the patch kernel: timed again
+    if entry is not None and shape_name(AUTO) in entry["rates"]:
         return tuple(entry["best"]), {parse_shape(k): r for k, r in entry["rates"].items()}
     scratch = ChainBatch(models, chains)
     moves = np.array([max(64, int(sweeps * m.n_sites)) for m in models], dtype=np.int64)

@@ -173,7 +173,7 @@ struct cemc_model {
   }
 
   // patches of the one translation group (ce_patches.h)
-  PatchCover cover;
+  std::shared_ptr<const PatchCover> cover;
   std::vector<PatchRec> patches;
   std::vector<double> ptab;
   std::vector<uint32_t> ptab_base;  // per table of the cover
@@ -430,7 +430,8 @@ void cemc_model::build_duals() {
 // are; bringing records into one order under these exchanges lets symmetry
 // images of a patch share a table.
 void cemc_model::build_patches() {
-  cover = PatchCover();
+  static PatchCovers covers;
+  cover.reset();
   patches.clear();
   ptab_base.clear();
   const int q = patch_members(n_species);
@@ -510,17 +511,15 @@ void cemc_model::build_patches() {
     }
     in.push_back(x);
   }
-  if (!PatchSearch(int(col_of_site.size()), in, q).run(&cover)) {
-    cover = PatchCover();
-    return;
-  }
+  cover = covers.get(int(col_of_site.size()), in, q);
+  if (cover == nullptr) return;
   // tables: a zero one for padding lanes, then one per type; a type that
   // leaves the last place unused holds no codes of it
   int part = n_bfs;
   for (int i = 0; i < q - 1; ++i) part *= n_species;
   std::vector<uint32_t> w_last;
   uint32_t off = uint32_t(part);
-  for (const auto& terms : cover.tables) {
+  for (const auto& terms : cover->tables) {
     bool full = false;
     for (const auto& t : terms)
       for (int m = 0; m < t.n; ++m) full = full || t.place[m] == q - 1;
@@ -529,7 +528,7 @@ void cemc_model::build_patches() {
     off += uint32_t(full ? part * n_species : part);
   }
   ptab.assign(off, 0.0);
-  for (const auto& p : cover.patches) {
+  for (const auto& p : cover->patches) {
     PatchRec rec{{0, 0, 0, 0, 0, 0}, ptab_base[p.table], w_last[p.table]};
     for (int i = 0; i < q; ++i) {
       if (p.site[i] < 0) continue;
@@ -549,7 +548,7 @@ void cemc_model::build_ptab() {
   for (size_t t = 0; t < ptab_base.size(); ++t) {
     const uint32_t end = t + 1 < ptab_base.size() ? ptab_base[t + 1] : uint32_t(ptab.size());
     const bool full = end - ptab_base[t] > uint32_t(part * n_bfs);
-    patch_table(cover.tables[t], n_species, full ? q : q - 1, n_bfs, n_bfs, code_bits(), gtab.data(),
+    patch_table(cover->tables[t], n_species, full ? q : q - 1, n_bfs, n_bfs, code_bits(), gtab.data(),
                 ptab.data() + ptab_base[t]);
   }
 }

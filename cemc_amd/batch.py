@@ -219,6 +219,20 @@ class ChainBatch:
                                                           ctypes.byref(r), ctypes.byref(g)))
         return w.value, r.value, bool(g.value)
 
+    def lanes_per_move(self, chain):
+        """Lanes that evaluate one of the chain's moves on the patch kernel (4, 8,
+        16 or 64); 0: the chain runs on another kernel."""
+        v = ctypes.c_int32()
+        _capi.check(self._lib.cemc_batch_get_lanes_per_move(self.handle, int(chain), ctypes.byref(v)))
+        return v.value
+
+    def wl_lanes_per_move(self, chain, shared=False):
+        """The same for the chain's Wang-Landau walker in wl_run (8 or 0)."""
+        v = ctypes.c_int32()
+        _capi.check(self._lib.cemc_batch_wl_get_lanes_per_move(self.handle, int(chain), int(bool(shared)),
+                                                               ctypes.byref(v)))
+        return v.value
+
     def set_temperature(self, chain, temperature):
         _capi.check(self._lib.cemc_batch_set_temperature(self.handle, int(chain), float(temperature)))
         self.temperatures[chain] = float(temperature)

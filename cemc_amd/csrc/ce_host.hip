@@ -2344,6 +2344,26 @@ void wl_store(cemc_batch* b, int chain, const WLDev& desc, const double* logdos,
   b->wl = next;
 }
 
+// Patches per lane of walker `c` on the patch kernel's rounds of eight, eight
+// lanes per move, and the LDS it takes; 0: the one-move kernel.  The patch
+// kernel takes walkers with a histogram of their own, without windows, whose
+// bins per eV are finite.
+int wl_patch_kr(const cemc_batch* b, int c, bool shared, uint32_t* lds) {
+  const cemc_model* m = b->models[b->params[c].model];
+  const WLDev& w = b->wl[c];
+  const bool sgc = b->params[c].kind == CEMC_MOVE_SGC;
+  const int P = int(m->patches.size());
+  if (shared || w.adaptive != 0 || P == 0 || P > 64 || (!sgc && m->n_sites > 65535) ||
+      !std::isfinite(double(w.n_bins) / (w.e_max - w.e_min)))
+    return 0;
+  const int kr = P <= 16 ? 2 : (P <= 32 ? 4 : 8);
+  *lds = patch_lds_bytes(m->pdims[0] * m->pdims[1] * m->pdims[2], sgc ? 0 : m->n_sites, int(m->ptab.size()),
+                         sgc ? 0 : 8 * kr) +
+         16u * uint32_t(w.n_bins);
+  const bool fits = *lds <= lds_limit() + sweep_static_lds() - kPatchStaticLds;
+  return fits && patch_variant_ok(m->read_slices(), 8, kr, 1, true, !sgc) ? kr : 0;
+}
+
 // One launch per kernel variant over the chains that carry a walker.
 // shared: every walker of the batch visits walker 0's histogram; each check
 // of check_every steps (rounded up to a multiple of the walker count, as
@@ -2411,21 +2431,12 @@ void wl_launch(cemc_batch* b, int64_t n_checks, int64_t check_every, uint32_t* h
     const uint32_t no_g = wl_lds_bytes(sweep_lds_bytes(occ_bytes, m->n_sites, n_rec, 0), nbins, adaptive);
     k.glds = with_g <= std::min(kGtabLdsBudget, limit);
     uint32_t lds = k.glds ? with_g : no_g;
-    // a histogram of its own, no windows: the patch kernel's rounds of eight
-    // (its bins per eV have to be finite)
-    k.patch_kr = 0;
-    const int P = int(m->patches.size());
-    if (!shared && !adaptive && P > 0 && P <= 64 && (k.sgc || m->n_sites <= 65535) &&
-        std::isfinite(double(nbins) / (b->wl[c].e_max - b->wl[c].e_min))) {
-      const int kr = P <= 16 ? 2 : (P <= 32 ? 4 : 8);
-      const uint32_t need = patch_lds_bytes(occ_bytes, k.sgc ? 0 : m->n_sites, int(m->ptab.size()),
-                                            k.sgc ? 0 : 8 * kr) + 16u * uint32_t(nbins);
-      if (need <= limit + sweep_static_lds() - kPatchStaticLds && patch_variant_ok(k.kbm, 8, kr, 1, true, !k.sgc)) {
-        k.patch_kr = kr;
-        k.kr = 0;
-        k.glds = false;
-        lds = need;
-      }
+    uint32_t patch_lds = 0;
+    k.patch_kr = wl_patch_kr(b, c, shared, &patch_lds);
+    if (k.patch_kr > 0) {
+      k.kr = 0;
+      k.glds = false;
+      lds = patch_lds;
     }
     require(lds <= limit || k.patch_kr > 0, "the walker's chain and histogram do not fit in the workgroup's LDS");
     auto& g = groups[k];
@@ -3234,6 +3245,32 @@ int cemc_batch_get_launch_shape(cemc_batch* b, int32_t chain, int32_t* waves, in
           return;
         }
     throw std::runtime_error("chain not found in any launch class");
+  });
+}
+
+int cemc_batch_get_lanes_per_move(cemc_batch* b, int32_t chain, int32_t* lanes) {
+  return guarded([&] {
+    require(b != nullptr && lanes != nullptr, "NULL argument");
+    require(chain >= 0 && chain < b->n_chains, "chain index out of range");
+    std::vector<int32_t> order(b->n_chains);
+    HIP_CHECK(hipMemcpy(order.data(), b->d_order, sizeof(int32_t) * order.size(), hipMemcpyDeviceToHost));
+    for (const auto& cl : b->classes)
+      for (int i = cl.begin; i < cl.begin + cl.count; ++i)
+        if (order[i] == chain) {
+          *lanes = cl.kg;
+          return;
+        }
+    throw std::runtime_error("chain not found in any launch class");
+  });
+}
+
+int cemc_batch_wl_get_lanes_per_move(cemc_batch* b, int32_t chain, int32_t shared, int32_t* lanes) {
+  return guarded([&] {
+    require(b != nullptr && lanes != nullptr, "NULL argument");
+    require(chain >= 0 && chain < b->n_chains, "chain index out of range");
+    require(!b->wl.empty() && b->wl[chain].n_bins > 0, "the chain carries no Wang-Landau walker");
+    uint32_t lds = 0;
+    *lanes = wl_patch_kr(b, chain, shared != 0, &lds) > 0 ? 8 : 0;
   });
 }
 

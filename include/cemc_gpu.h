@@ -307,11 +307,25 @@ CEMC_API int cemc_batch_get_energy_path(cemc_batch* batch, int32_t chain, int32_
  * held in registers (0: records in LDS), the sub-clusters' energy tables in
  * LDS (1) or HBM (0).  By default (no waves, moves per round or field path
  * asked for) chains on closed-form periodic lattices with one translation
- * group and up to four species run on the patch kernel, which reads tables
- * of whole groups of sub-clusters from LDS instead: it reports its patches
- * per lane as the second value and 0 as the third. */
+ * group and two to four species run on the patch kernel, which reads tables
+ * of whole groups of sub-clusters ("patches") from LDS instead: it reports
+ * its patches per lane as the second value and 0 as the third.  It takes
+ * models with every site movable, cluster offsets of at most two cells along
+ * each axis, dimensions of at most 127, sub-clusters listed for each of their
+ * sites (a site reaches the sites that reach it), at most 96 distinct member
+ * sites and at most 448 patches (64 for chains with constraints or a bias and
+ * for Wang-Landau walkers), where lattice, tracker (swaps; at most 65535
+ * sites; with four species and more than 64 patches it may stay in HBM) and
+ * patch tables fit in the workgroup's LDS.  Chains with constraints or a bias
+ * also need constraints that depend on the proposal alone: sites open to
+ * every species or to none, no pair constraint, no waste recycling, and
+ * fixed species only for swaps.  Every other chain runs on the sweep kernel,
+ * with the same moves. */
 CEMC_API int cemc_batch_get_launch_shape(cemc_batch* batch, int32_t chain, int32_t* waves,
                                          int32_t* records_per_lane, int32_t* tables_in_lds);
+/* Lanes that evaluate one move of the chain on the patch kernel (4, 8, 16 or
+ * 64); 0: the chain runs on another kernel. */
+CEMC_API int cemc_batch_get_lanes_per_move(cemc_batch* batch, int32_t chain, int32_t* lanes);
 /* Temperature of one chain (parallel tempering uses it to exchange replicas). */
 CEMC_API int cemc_batch_set_temperature(cemc_batch* batch, int32_t chain, double temperature);
 
@@ -447,6 +461,11 @@ CEMC_API int cemc_batch_wl_run(cemc_batch* batch, int64_t n_checks, int64_t chec
  * its t-th step. */
 CEMC_API int cemc_batch_wl_run_shared(cemc_batch* batch, int64_t n_checks, int64_t check_every,
                                       uint32_t* accept_bits, int64_t words_per_chain, double* kernel_ms);
+/* Lanes that evaluate one move of the chain's walker on the patch kernel in
+ * cemc_batch_wl_run (shared 0) or cemc_batch_wl_run_shared (shared 1): 8, or
+ * 0 for the one-move kernel (shared histograms, adaptive windows, more than
+ * 64 patches, models that the patch kernel does not take). */
+CEMC_API int cemc_batch_wl_get_lanes_per_move(cemc_batch* batch, int32_t chain, int32_t shared, int32_t* lanes);
 
 /* ------------------------------------------------------------------ pool
  * A batch whose chains join and leave while it runs: the resident state of

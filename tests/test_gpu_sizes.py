@@ -132,6 +132,7 @@ def test_quaternary_32_cube_tempering_matches_oracle(gpu):
     w, kr, glds = batch.launch_shape(0)
     print("quaternary 32^3 launch shape", (w, kr, glds), flush=True)
     assert w == 8 and not glds
+    assert batch.lanes_per_move(0) == 64  # the patch kernel
     for r in range(2):
         cf, _ = batch.cf(r)
         assert np.max(np.abs(cf - np.array([cf8[r][n] for n in names]))) <= 1e-12

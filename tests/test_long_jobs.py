@@ -29,6 +29,7 @@ def test_long_job_in_a_crowd(gpu, species, shells, kind, waves):
     moves[700] = 1 << 21
     pool.run_sliced(moves, 1.0)
     assert pool.launch_shape(700)[0] == waves
+    assert pool.lanes_per_move(700) == (4 if waves == 1 else (64 if len(species) == 4 else 16))
     assert pool.launch_shape(0)[0] == (1 if len(species) < 4 else 2)
     done = pool.stats()["moves"]
     assert 64 < done[700] < moves[700] and done[0] == 64

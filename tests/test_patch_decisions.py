@@ -36,6 +36,7 @@ def test_margin_decisions_use_the_chains_temperature(gpu, kind, species, chains,
         if biased:
             for c in range(chains):
                 batch.set_hooks(c, bias_species=0, bias_table=bias)
+        assert batch.lanes_per_move(0) == (8 if biased else (4 if chains > 512 else 16))
         e0 = batch.energies()
         batch.run(1)
         return batch.stats()["accepted"], batch.energies() - e0

@@ -48,4 +48,25 @@ def test_one_sided_sub_clusters(gpu, kind):
         cl["indices"] = [cl["indices"][k] for k in keep]
         cl["order"] = [cl["order"][k] for k in keep]
     print("one-sided pairs", kind, flush=True)
-    _chains_vs_oracle(s, seeded_ecis(s, 5, 0.02), kind, 1200.0, 6000)
+    batch = _chains_vs_oracle(s, seeded_ecis(s, 5, 0.02), kind, 1200.0, 6000)
+    assert batch.lanes_per_move(0) == 0
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("size,lanes", [((127, 5, 5), 16), ((128, 5, 5), 0), ((5, 5, 127), 16), ((5, 128, 5), 0)])
+def test_longest_axes(gpu, kind, size, lanes):
+    """Cell differences of the pair test take a byte per axis, up to 253 at 127
+    cells; longer lattices run on the sweep kernel."""
+    s = FCCSettings(size, ["A", "B"], {2: 4, 3: 2})
+    print("longest axes", size, kind, flush=True)
+    batch = _chains_vs_oracle(s, seeded_ecis(s, 5, 0.02), kind, 1200.0, 6000)
+    assert batch.lanes_per_move(0) == lanes
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_more_patches_than_the_kernel_takes(gpu, kind):
+    """1001 patches (448 at most): the sweep kernel."""
+    s = FCCSettings(5, ["A", "B", "C", "D"], {2: 4, 3: 4, 4: 4})
+    print("many patches", kind, flush=True)
+    batch = _chains_vs_oracle(s, seeded_ecis(s, 5, 0.005), kind, 1200.0, 600)
+    assert batch.lanes_per_move(0) == 0

@@ -112,18 +112,25 @@ def test_patch_entries_sum_to_the_subclusters_entries(search, make, species, q):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", [0, 1])
-@pytest.mark.parametrize("species,shells,size,symm,chains", [
-    (2, {2: 4, 3: 2}, 10, True, 1),            # 12 patches
-    (2, {2: 4, 3: 2}, (5, 7, 6), True, 700),   # smallest box of the halo, one wave each
-    (2, {2: 4, 3: 3, 4: 2}, 5, True, 300),     # 47 patches, two waves
-    (3, {2: 3, 3: 2}, (6, 5, 9), False, 3),    # no shared tables
-    (3, {2: 4, 3: 3, 4: 2}, 9, True, 2),       # 59 patches, four waves
-    (3, {2: 4, 3: 3, 4: 2}, 5, True, 600),
-    (4, {2: 3, 3: 2, 4: 1}, (5, 6, 5), True, 2),
-    (4, {2: 3, 3: 3, 4: 3}, 5, True, 1),       # 426 patches, eight waves
-    (4, {2: 3, 3: 3, 4: 3}, 6, True, 300),     # and two
+@pytest.mark.parametrize("species,shells,size,symm,chains,lanes,waves,per_lane", [
+    (2, {2: 4, 3: 2}, 10, True, 1, 16, 4, 1),             # 12 patches
+    (2, {2: 4, 3: 2}, (5, 7, 6), True, 700, 4, 1, 3),     # smallest box of the halo, one wave each
+    (2, {2: 4, 3: 3, 4: 2}, 5, True, 300, 16, 2, 4),      # 47 patches, two waves
+    (3, {2: 3, 3: 2}, (6, 5, 9), False, 3, 16, 4, 1),     # no shared tables
+    (3, {2: 4, 3: 3, 4: 2}, 9, True, 2, 16, 4, 4),        # 59 patches, four waves
+    (3, {2: 4, 3: 3, 4: 2}, 5, True, 600, 4, 1, 15),
+    (4, {2: 3, 3: 2, 4: 1}, (5, 6, 5), True, 2, 16, 4, 2),
+    (4, {2: 3, 3: 3, 4: 3}, 5, True, 1, 64, 8, 7),        # 426 patches, eight waves
+    (4, {2: 3, 3: 3, 4: 3}, 6, True, 300, 64, 2, 7),      # and two
+    (4, {2: 3, 3: 2}, (5, 6, 5), True, 600, 4, 1, 6),     # 24 patches, a quad each
+    (4, {2: 3, 3: 2, 4: 1}, 5, True, 600, 4, 1, 9),       # 32
+    (2, {2: 3, 3: 3, 4: 3}, 5, True, 1, 64, 8, 4),        # 164 patches, a wave per move: eight waves
+    (2, {2: 3, 3: 3, 4: 3}, 5, True, 200, 64, 4, 4),      # and four
+    (3, {2: 4, 3: 4}, 5, True, 1, 64, 8, 2),              # 96 patches
+    (3, {2: 3, 3: 3, 4: 3}, 5, True, 300, 64, 2, 4),      # 220
+    (4, {2: 3, 3: 3}, 5, True, 200, 64, 4, 2),            # 84
 ])
-def test_patch_kernel_matches_oracle(gpu, kind, species, shells, size, symm, chains):
+def test_patch_kernel_matches_oracle(gpu, kind, species, shells, size, symm, chains, lanes, waves, per_lane):
     """Flips, and swaps whose sites interact (small cells), in launches that
     end inside a round and a block: accept bits and lattices equal the
     oracle's, energies and sample sums to rounding."""
@@ -139,6 +146,8 @@ def test_patch_kernel_matches_oracle(gpu, kind, species, shells, size, symm, cha
                        [dict(kind=kind, temperature=float(t), occupation=occ, seed=8, uid=c, chem_pot=mu)
                         for c, t in enumerate(temps)])
     print("patches", species, shells, size, "kind", kind, "chains", chains, batch.launch_shape(0), flush=True)
+    assert batch.lanes_per_move(0) == lanes
+    assert batch.launch_shape(0)[:2] == (waves, per_lane)
     parts = [1, 7, 64, 65, 330]
     logs = [batch.run_logged(n) for n in parts]
     total = sum(parts)
@@ -188,6 +197,7 @@ def test_patch_walkers_match_oracle(gpu, species, shells, size, half, bins):
     names = s.cf_names()
     e0 = OracleUpdater(OracleModel(s, names), occ, brute_force_cf(s, occ, names), eci).get_energy()
     print("patch walker", species, shells, size, flush=True)
-    got, _ = _gpu_vs_oracle(s, eci, occ, dict(_centred(e0, half, bins), f=1.0, f_min=1e-3, flatness=0.3,
-                                              cur_bin=bins // 2), 9, 333)
+    got, batch = _gpu_vs_oracle(s, eci, occ, dict(_centred(e0, half, bins), f=1.0, f_min=1e-3, flatness=0.3,
+                                                  cur_bin=bins // 2), 9, 333)
     assert got["n_accept"] > 0
+    assert batch.wl_lanes_per_move(0) == 8 and batch.wl_lanes_per_move(0, shared=True) == 0

@@ -49,6 +49,7 @@ def _assert_same(a, b, chains):
 def test_energies_do_not_depend_on_where_launches_end(gpu, species, shells, size, kind, n, hooked):
     whole, parts = _batch(species, shells, size, kind, n, hooked)
     print("split", species, kind, n, whole.launch_shape(0), flush=True)
+    assert whole.lanes_per_move(0) > 0
     cuts = [1, 7, 0, 64, 100, 28, 333]
     whole.run(sum(cuts))
     for m in cuts:
@@ -64,7 +65,7 @@ def test_energies_do_not_depend_on_where_launches_end(gpu, species, shells, size
 ])
 def test_time_slices_continue_each_chains_stream(gpu, species, shells, kind, n, waves):
     whole, slices = _batch(species, shells, 8, kind, n)
-    assert whole.launch_shape(0)[0] == waves
+    assert whole.launch_shape(0)[0] == waves and whole.lanes_per_move(0) > 0
     moves = 12000
     print("slices", species, kind, n, flush=True)
     whole.run(moves)

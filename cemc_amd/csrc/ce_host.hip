@@ -2353,7 +2353,7 @@ int wl_patch_kr(const cemc_batch* b, int c, bool shared, uint32_t* lds) {
   const WLDev& w = b->wl[c];
   const bool sgc = b->params[c].kind == CEMC_MOVE_SGC;
   const int P = int(m->patches.size());
-  if (shared || w.adaptive != 0 || P == 0 || P > 64 || (!sgc && m->n_sites > 65535) ||
+  if (shared || w.adaptive != 0 || uint32_t(w.n_bins) > lds_limit() || P == 0 || P > 64 || (!sgc && m->n_sites > 65535) ||
       !std::isfinite(double(w.n_bins) / (w.e_max - w.e_min)))
     return 0;
   const int kr = P <= 16 ? 2 : (P <= 32 ? 4 : 8);
@@ -2424,6 +2424,8 @@ void wl_launch(cemc_batch* b, int64_t n_checks, int64_t check_every, uint32_t* h
     const int occ_bytes = m->periodic ? m->pdims[0] * m->pdims[1] * m->pdims[2] : m->n_sites;
     const int n_rec = k.kr == 0 ? int(m->recs.size()) : 0;
     const int nbins = shared ? 0 : b->wl[c].n_bins;
+    // a bin takes 13 bytes and more; beyond this the sizes below would overflow
+    require(uint32_t(nbins) <= limit, "the walker's chain and histogram do not fit in the workgroup's LDS");
     const bool adaptive = !shared && b->wl[c].adaptive != 0;
     k.adaptive = adaptive;
     const uint32_t with_g =

@@ -50,3 +50,20 @@ def test_range_narrower_than_the_smallest_bins(gpu):
     got, _ = _gpu_vs_oracle(s, eci, random_occupation(s.n_sites, 2, 2),
                             dict(n_bins=20, e_min=0.0, e_max=1e-310, f=1.0, cur_bin=10), 3, 100)
     assert got["n_accept"] > 0
+
+
+def test_more_bins_than_the_lds_holds(gpu):
+    """2^28 bins of 16 bytes are 2^32 bytes, which must not pass for none."""
+    from cemc_amd.batch import ChainBatch
+    from cemc_amd.model import CEModel
+    s = FCCSettings(5, ["A", "B"], {2: 2})
+    batch = ChainBatch([CEModel(s, seeded_ecis(s, 3, 0.02))],
+                       [dict(kind=0, temperature=900.0, seed=4, uid=0, occupation=random_occupation(s.n_sites, 2, 2))])
+    print("walker with 2^28 bins", flush=True)
+    batch.wl_set(0, 1 << 28, -1.0, 1.0, 1.0)
+    assert batch.wl_lanes_per_move(0) == 0
+    with pytest.raises(ValueError, match="do not fit"):
+        batch.wl_run(1, 10)
+    batch.wl_set(0, 20, -1.0, 1.0, 1.0)
+    batch.wl_run(1, 10)
+    assert batch.wl_get(0)["n_moves"] == 10

@@ -130,6 +130,7 @@ SIGNATURES = [
     ("cemc_batch_set_energy_path", ctypes.c_int, [_vp, ctypes.c_int32]),
     ("cemc_batch_get_energy_path", ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)]),
     ("cemc_batch_get_launch_shape", ctypes.c_int, [_vp, ctypes.c_int32, _i32p, _i32p, _i32p]),
+    ("cemc_batch_set_patches", ctypes.c_int, [_vp, ctypes.c_int32]),
     ("cemc_batch_get_lanes_per_move", ctypes.c_int, [_vp, ctypes.c_int32, _i32p]),
     ("cemc_batch_wl_get_lanes_per_move", ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32, _i32p]),
     ("cemc_batch_set_temperature", ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_double]),

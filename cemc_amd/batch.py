@@ -219,6 +219,11 @@ class ChainBatch:
                                                           ctypes.byref(r), ctypes.byref(g)))
         return w.value, r.value, bool(g.value)
 
+    def set_patches(self, always):
+        """False (default): the patch kernel where the chain allows it and few of
+        its moves conflict; True: wherever the chain allows it.  Same moves."""
+        _capi.check(self._lib.cemc_batch_set_patches(self.handle, int(bool(always))))
+
     def lanes_per_move(self, chain):
         """Lanes that evaluate one of the chain's moves on the patch kernel (4, 8,
         16 or 64); 0: the chain runs on another kernel."""

@@ -177,6 +177,7 @@ struct cemc_model {
   std::vector<PatchRec> patches;
   std::vector<double> ptab;
   std::vector<uint32_t> ptab_base;  // per table of the cover
+  double flip_sd = 0.0;             // of a flip's energy change over random neighbourhoods, eV (build_ptab)
   PatchRec* d_patches = nullptr;
   double* d_ptab = nullptr;
 
@@ -551,6 +552,35 @@ void cemc_model::build_ptab() {
     patch_table(cover->tables[t], n_species, full ? q : q - 1, n_bfs, n_bfs, code_bits(), gtab.data(),
                 ptab.data() + ptab_base[t]);
   }
+  // spread of a flip's energy change: its sub-clusters' variances over the
+  // members' species and the two species of the flip, added up
+  const int k = code_bits(), Pc = 1 << (3 * k);
+  std::map<std::pair<int, int>, int> count;  // (entry, reference position) -> sub-clusters
+  for (size_t r = 0; r < recs.size(); ++r) ++count[{rec_entry[r], rec_refpos(recs[r])}];
+  double var = 0.0;
+  for (const auto& kv : count) {
+    const int c = kv.first.first, nm = entry_size[c] - 1, codes = pow_s(nm);
+    const double* G = gtab.data() + entry_goff[c] + kv.first.second * deco_slices() * Pc;
+    double sum = 0.0;
+    for (int o = 0; o < n_species; ++o)
+      for (int n = 0; n < n_species; ++n) {
+        if (n == o) continue;
+        double m1 = 0.0, m2 = 0.0;
+        for (int at = 0; at < codes; ++at) {
+          int code = 0;
+          for (int m = 0, rest = at; m < nm; ++m, rest /= n_species) code |= (rest % n_species) << (k * m);
+          double de = 0.0;
+          for (int d = 0; d < n_bfs; ++d)
+            de += (basis[d * n_species + n] - basis[d * n_species + o]) * G[d * Pc + code];
+          m1 += de;
+          m2 += de * de;
+        }
+        m1 /= codes;
+        sum += m2 / codes - m1 * m1;
+      }
+    var += kv.second * sum / (n_species * (n_species - 1));
+  }
+  flip_sd = std::sqrt(std::max(var, 0.0));
 }
 
 void cemc_model::refresh_view() {
@@ -1579,6 +1609,12 @@ struct cemc_batch {
   std::vector<Class> classes;
   int64_t classes_version = 0;  // bumped whenever the launch classes change
   int forced_waves = 0;
+  bool always_patches = false;  // the patch kernel wherever a chain allows it
+  // chains kept off the patch kernel since their moves conflict too often, the
+  // limits that decided it, and whether a temperature crossed one since
+  std::vector<char> conflicting;
+  std::vector<double> conflict_limit;
+  bool reshape = false;
   size_t order_cap = 0;         // entries allocated at d_order
   // pool mode: chains join and leave; slots [0, n_chains) with active flags
   bool dynamic = false;
@@ -1783,6 +1819,23 @@ void range_free(std::map<int64_t, int64_t>& free_map, int64_t off, int64_t len) 
 // rounds of kSpecMoves moves.
 constexpr double kRoundShare = 0.12;
 
+// Chance that two moves of a chain conflict because the first is made: the
+// share of sites that a flip interacts with (times four for the sites of two
+// swaps) times the acceptance.  In equilibrium a Metropolis move whose energy
+// changes spread like a normal law of standard deviation sd is accepted with
+// probability erfc(sd / (sqrt(8) kT)).  With sd from random neighbourhoods
+// this was within 0.08 of the rates measured for swaps at 1000 and 2500 K on
+// eight FCC models of two to four species (6^3 to 10^3 sites), and too high for
+// ordered or strongly biased states.
+double conflict_chance(const cemc_model* m, const ChainParams& p, double enough) {
+  const bool canon = p.kind == CEMC_MOVE_CANONICAL;
+  const int box = __builtin_popcountll(m->imask[0]) + __builtin_popcountll(m->imask[1]);
+  const double share = double(box) * (canon ? 4.0 : 1.0) / double(m->n_sites);
+  if (share <= enough) return share;
+  const double sd = m->flip_sd * (canon ? std::sqrt(2.0) : 1.0);
+  return share * std::erfc(sd / (std::sqrt(8.0) * p.kT));
+}
+
 void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>* nm = nullptr) {
   const int n_chains = b->n_chains;
   // pool batches launch only the active chains that have moves to make
@@ -1818,6 +1871,9 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
   }
   int n_launch = 0;
   for (int c = 0; c < n_chains; ++c) n_launch += included(c) ? 1 : 0;
+  b->conflicting.assign(n_chains, 0);
+  b->conflict_limit.assign(n_chains, HUGE_VAL);
+  b->reshape = false;
   // chains on the device during this launch: the pool's own and, for a
   // pool, those the other pools have in flight
   const int64_t on_device = n_launch + (b->dynamic ? g_pool_chains[current_device_index()].load() : 0);
@@ -1988,9 +2044,23 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     // Chains with a constraint on the state (a pair constraint, a site open to
     // some species, fixed species of SGC chains) or waste recycling stay on
     // the one-move kernel.
+    // Chains whose moves mostly conflict make one or two moves a round, where
+    // one move at a time is faster: small cells at high acceptance.  Time of the
+    // sweep kernel over the patch kernel's, by the conflict chance (FCC 5^3 to
+    // 10^3, 3 to 84 patches): up to 256 chains 0.96-1.6 at 0.4-0.6 and 0.65-1.02
+    // above 0.8; 1024 chains 0.93-2.0 at 0.2-0.3 and 0.58-1.1 above 0.4; 4096
+    // chains 0.99-1.9 at 0.1-0.15 and 0.55-1.6 at 0.2-0.3.  With 164 and more
+    // patches 0.82-0.96 above 0.8, for any number.  Below, the patch kernel wins:
+    // 1.2 to 7.  (Walkers and chains with hooks have no such limit: their one-move
+    // kernels were slower at every conflict chance, 1.01 to 17.)
     if (forced_waves == 0 && b->spec_moves == 0 && !k.field && (!k.hooks || b->hooks[c].by_proposal) &&
         !m->patches.empty() && (!canon || m->n_sites <= 65535)) {
       const int P = int(m->patches.size());
+      if (!b->always_patches && !k.hooks) {
+        b->conflict_limit[c] =
+            P > 128 ? 0.8 : (on_device <= int64_t(2) * n_cu ? 0.55 : (on_device <= int64_t(4) * n_cu ? 0.3 : 0.15));
+        b->conflicting[c] = conflict_chance(m, b->params[c], b->conflict_limit[c]) > b->conflict_limit[c];
+      }
       const uint32_t room = limit + sweep_static_lds() - kPatchStaticLds;
       // A pool's long job among crowds of 600-3000 short ones (chain_waves, 4
       // waves against 1 or 2, moves per ms): swaps of two species 2590 ->
@@ -2016,7 +2086,8 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
         trk_lds = false;
         need = patch_lds_bytes(occ_bytes, 0, int(m->ptab.size()), near_slots);
       }
-      if (kr > 0 && need <= room && patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon, k.hooks)) {
+      if (!b->conflicting[c] && kr > 0 && need <= room &&
+          patch_variant_ok(k.kbm, kg, kr, waves, trk_lds, canon, k.hooks)) {
         k.kg = kg;
         k.kr = kr;
         k.waves = waves;
@@ -2181,6 +2252,7 @@ void batch_launch(cemc_batch* b, const int64_t* n_moves, int64_t moves, bool tim
     HIP_CHECK(hipMemsetAsync(d_log, 0, sizeof(uint32_t) * size_t(b->n_chains) * log_words, b->stream));
   }
   if (b->dynamic) derive_classes(b, b->forced_waves, &nm);
+  if (b->reshape) derive_classes(b, b->forced_waves);
   HIP_CHECK(hipMemcpyAsync(b->d_nmoves, nm.data(), sizeof(int64_t) * nm.size(), hipMemcpyHostToDevice, b->stream));
   // a pool's chains count as on the device from the launch until the wait
   // below returns (or throws)
@@ -3219,6 +3291,7 @@ int cemc_batch_get_energy_path(cemc_batch* b, int32_t chain, int32_t* path) {
   return guarded([&] {
     require(b != nullptr && path != nullptr, "NULL argument");
     require(chain >= 0 && chain < b->n_chains, "chain index out of range");
+    if (b->reshape) derive_classes(b, b->forced_waves);
     std::vector<int32_t> order(b->n_chains);
     HIP_CHECK(hipMemcpy(order.data(), b->d_order, sizeof(int32_t) * order.size(), hipMemcpyDeviceToHost));
     for (const auto& cl : b->classes)
@@ -3236,6 +3309,7 @@ int cemc_batch_get_launch_shape(cemc_batch* b, int32_t chain, int32_t* waves, in
   return guarded([&] {
     require(b != nullptr, "NULL batch");
     require(chain >= 0 && chain < b->n_chains, "chain index out of range");
+    if (b->reshape) derive_classes(b, b->forced_waves);
     std::vector<int32_t> order(b->n_chains);
     HIP_CHECK(hipMemcpy(order.data(), b->d_order, sizeof(int32_t) * order.size(), hipMemcpyDeviceToHost));
     for (const auto& cl : b->classes)
@@ -3250,10 +3324,21 @@ int cemc_batch_get_launch_shape(cemc_batch* b, int32_t chain, int32_t* waves, in
   });
 }
 
+int cemc_batch_set_patches(cemc_batch* b, int32_t always) {
+  return guarded([&] {
+    require(b != nullptr, "NULL batch");
+    require(always == 0 || always == 1, "patches must be 0 (automatic) or 1 (wherever a chain allows them)");
+    HIP_CHECK(hipStreamSynchronize(b->stream));
+    b->always_patches = always != 0;
+    if (!b->dynamic) derive_classes(b, b->forced_waves);
+  });
+}
+
 int cemc_batch_get_lanes_per_move(cemc_batch* b, int32_t chain, int32_t* lanes) {
   return guarded([&] {
     require(b != nullptr && lanes != nullptr, "NULL argument");
     require(chain >= 0 && chain < b->n_chains, "chain index out of range");
+    if (b->reshape) derive_classes(b, b->forced_waves);
     std::vector<int32_t> order(b->n_chains);
     HIP_CHECK(hipMemcpy(order.data(), b->d_order, sizeof(int32_t) * order.size(), hipMemcpyDeviceToHost));
     for (const auto& cl : b->classes)
@@ -3283,6 +3368,13 @@ int cemc_batch_set_temperature(cemc_batch* b, int32_t chain, double temperature)
     require(temperature > 0.0 && std::isfinite(temperature), "temperature must be positive");
     b->params[chain].kT = temperature * kBoltzmannEV;
     HIP_CHECK(hipMemcpy(&b->d_params[chain].kT, &b->params[chain].kT, sizeof(double), hipMemcpyHostToDevice));
+    // chosen anew at the next launch (pools choose at every launch)
+    if (!b->dynamic && chain < int(b->conflicting.size()) && b->conflict_limit[chain] < HUGE_VAL) {
+      const double limit = b->conflict_limit[chain];
+      if ((conflict_chance(b->models[b->params[chain].model], b->params[chain], limit) > limit) !=
+          (b->conflicting[chain] != 0))
+        b->reshape = true;
+    }
   });
 }
 

@@ -320,9 +320,17 @@ CEMC_API int cemc_batch_get_energy_path(cemc_batch* batch, int32_t chain, int32_
  * also need constraints that depend on the proposal alone: sites open to
  * every species or to none, no pair constraint, no waste recycling, and
  * fixed species only for swaps.  Every other chain runs on the sweep kernel,
- * with the same moves. */
+ * with the same moves, and so do chains of small cells at high acceptance
+ * (cemc_batch_set_patches). */
 CEMC_API int cemc_batch_get_launch_shape(cemc_batch* batch, int32_t chain, int32_t* waves,
                                          int32_t* records_per_lane, int32_t* tables_in_lds);
+/* 0 (default): the patch kernel where a chain allows it (see
+ * cemc_batch_get_launch_shape), unless its moves conflict so often that one
+ * move at a time is faster: small cells at high acceptance, judged from the
+ * model's energies and the chain's temperature at each launch.  1: wherever a
+ * chain allows it.  Moves, accept sequences and lattices are the same, energies
+ * agree to rounding. */
+CEMC_API int cemc_batch_set_patches(cemc_batch* batch, int32_t always);
 /* Lanes that evaluate one move of the chain on the patch kernel (4, 8, 16 or
  * 64); 0: the chain runs on another kernel. */
 CEMC_API int cemc_batch_get_lanes_per_move(cemc_batch* batch, int32_t chain, int32_t* lanes);

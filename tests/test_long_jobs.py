@@ -22,6 +22,7 @@ def test_long_job_in_a_crowd(gpu, species, shells, kind, waves):
     occ = random_occupation(s.n_sites, len(species), 1)
     n = 1100
     pool = ChainPool(n, 1, n * 512, n * 512)
+    pool.set_patches(True)
     print("long job", species, kind, flush=True)
     moves = np.full(n, 64, dtype=np.int64)
     for c in range(n):

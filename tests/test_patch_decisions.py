@@ -33,6 +33,7 @@ def test_margin_decisions_use_the_chains_temperature(gpu, kind, species, chains,
     def after_one_move(temps):
         batch = ChainBatch([model] * chains, [dict(kind=kind, temperature=float(t), occupation=occ, seed=11, uid=c)
                                               for c, t in enumerate(temps)])
+        batch.set_patches(True)
         if biased:
             for c in range(chains):
                 batch.set_hooks(c, bias_species=0, bias_table=bias)

@@ -11,13 +11,14 @@ from oracle.oracle import OracleModel, OracleUpdater
 pytestmark = pytest.mark.gpu
 
 
-def _chains_vs_oracle(s, eci, kind, temperature, n_moves, chains=1):
+def _chains_vs_oracle(s, eci, kind, temperature, n_moves, chains=1, always=True):
     from cemc_amd.batch import ChainBatch
     from cemc_amd.model import CEModel
     S = len(s.unique_elements)
     occ = random_occupation(s.n_sites, S, 3)
     batch = ChainBatch([CEModel(s, eci)] * chains,
                        [dict(kind=kind, temperature=temperature, occupation=occ, seed=3, uid=c) for c in range(chains)])
+    batch.set_patches(always)
     log = batch.run_logged(n_moves)
     names = s.cf_names()
     for c in {0, chains - 1}:
@@ -70,3 +71,43 @@ def test_more_patches_than_the_kernel_takes(gpu, kind):
     print("many patches", kind, flush=True)
     batch = _chains_vs_oracle(s, seeded_ecis(s, 5, 0.005), kind, 1200.0, 600)
     assert batch.lanes_per_move(0) == 0
+
+
+@pytest.mark.parametrize("size,kind,temperature,chains,lanes", [
+    (5, 0, 2500.0, 1, 0),     # every swap reaches most of the cell, most are made
+    (5, 0, 250.0, 1, 16),     # few are made
+    (5, 1, 2500.0, 1, 16),    # a flip reaches 0.44 of the cell
+    (5, 1, 2500.0, 600, 0),
+    (8, 0, 1000.0, 4, 16),
+    (6, 0, 700.0, 1100, 0),   # more chains than SIMDs: conflicts cost more
+    (10, 0, 700.0, 1100, 4),
+])
+def test_chains_whose_moves_mostly_conflict(gpu, size, kind, temperature, chains, lanes):
+    """Small cells at high acceptance run one move at a time."""
+    s = FCCSettings(size, ["A", "B"], {2: 4, 3: 2})
+    print("conflicting chains", size, kind, temperature, chains, flush=True)
+    batch = _chains_vs_oracle(s, seeded_ecis(s, 3, 0.02), kind, temperature, 500, chains, always=False)
+    assert batch.lanes_per_move(0) == lanes
+
+
+def test_a_temperature_that_changes_the_kernel(gpu):
+    """Annealing a small cell: one move at a time while it is hot, then the
+    patch kernel, move for move the oracle's."""
+    from cemc_amd.batch import ChainBatch
+    from cemc_amd.model import CEModel
+    s = FCCSettings(5, ["A", "B"], {2: 4, 3: 2})
+    eci = seeded_ecis(s, 3, 0.02)
+    occ = random_occupation(s.n_sites, 2, 3)
+    names = s.cf_names()
+    ora = OracleUpdater(OracleModel(s, names), occ, brute_force_cf(s, occ, names), eci)
+    batch = ChainBatch([CEModel(s, eci)], [dict(kind=0, temperature=2500.0, occupation=occ, seed=3, uid=0)])
+    done = 0
+    print("annealing", flush=True)
+    for temperature, lanes in ((2500.0, 0), (300.0, 16), (290.0, 16), (2000.0, 0)):
+        batch.set_temperature(0, temperature)
+        batch.run(777)
+        assert batch.lanes_per_move(0) == lanes
+        ora.run(0, 3, 0, 777, temperature, move_begin=done)
+        done += 777
+        assert np.array_equal(batch.occupation(0), ora.get_occupation())
+        assert abs(batch.energies()[0] - ora.get_energy()) <= 1e-10 * s.n_sites

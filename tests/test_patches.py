@@ -145,6 +145,7 @@ def test_patch_kernel_matches_oracle(gpu, kind, species, shells, size, symm, cha
     batch = ChainBatch([CEModel(st, eci)] * chains,
                        [dict(kind=kind, temperature=float(t), occupation=occ, seed=8, uid=c, chem_pot=mu)
                         for c, t in enumerate(temps)])
+    batch.set_patches(True)
     print("patches", species, shells, size, "kind", kind, "chains", chains, batch.launch_shape(0), flush=True)
     assert batch.lanes_per_move(0) == lanes
     assert batch.launch_shape(0)[:2] == (waves, per_lane)

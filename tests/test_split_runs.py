@@ -20,6 +20,8 @@ def _batch(species, shells, size, kind, n, hooked=False):
     make = lambda: ChainBatch([model] * n, [dict(kind=kind, temperature=400.0 + 2000.0 * c / n, occupation=occ,  # noqa: E731
                                                  seed=6, uid=c, chem_pot=mu) for c in range(n)])
     batches = make(), make()
+    for b in batches:
+        b.set_patches(True)
     if hooked:
         allowed = np.where(np.arange(s.n_sites) % 10 == 0, 0, 2 ** len(species) - 1).astype(np.uint8)
         for b in batches:
@@ -93,6 +95,7 @@ def test_a_state_changed_between_launches(gpu):
     print("state changed between launches", flush=True)
     b = ChainBatch([model], [dict(kind=1, temperature=900.0, occupation=occ, seed=6, uid=0, first_move=37)])
     table = np.arange(s.n_sites + 1) * 0.01
+    b.set_patches(True)
     for step in range(4):
         b.run(41)
         if step == 1:

@@ -41,16 +41,25 @@ def log(*a):
 
 # What bounds the kernels: neither bandwidth (the lattices never leave LDS
 # during a launch) but each chain's dependent move sequence (gather -> table ->
-# sum -> decide -> commit), see the SQ counters in profiles/.  The algorithmic
-# bytes count one gather per member of every sub-cluster; the patch tables
-# answer them with fewer, so the fraction may exceed one.
-LIMITER = ("issue and LDS latency of each chain's dependent move sequence, not HBM bandwidth; algorithmic bytes count "
-           "every sub-cluster's members, which the patch tables need not gather (SQ counters in profiles/)")
+# sum -> decide -> commit), see the SQ counters in profiles/.
+LIMITER = ("issue and LDS latency of each chain's dependent move sequence, neither HBM nor LDS bandwidth: the bytes "
+           "are the members and table entries a move reads, from LDS (SQ counters in profiles/)")
+
+
+def bytes_per_flip(model, patches):
+    """Bytes that one flip's energy change reads: on the patch kernel a byte
+    per member and a table entry per patch, else 5 bytes per non-changed member
+    of every sub-cluster (a translation entry and a species)."""
+    if patches:
+        n, q = model.patches()
+        return float(n * (q + 8 * (model.n_species - 1)))
+    return 5.0 * model.gathers_per_flip()
 
 
 def roofline_of(algorithmic_bytes, kernel_ms, lds_peak):
-    """Roofline object of one launch: algorithmic bytes / launch time against
-    HBM's published peak, and against the LDS read rate measured here."""
+    """Roofline object of one launch: the bytes its moves read / launch time,
+    against HBM's published peak, and against the LDS read rate measured
+    here."""
     achieved = algorithmic_bytes / (kernel_ms * 1e-3) / 1e9
     out = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": achieved / HBM_PEAK_GBS, "traffic": None, "limiter": LIMITER}
@@ -207,7 +216,7 @@ def ternary_uneven(n_chains=256, sweeps=200, seed=3, lds_peak=None, cpu=True):
     shapes = sorted({batch.launch_shape(c) for c in range(n_chains)})
     total = int(moves.sum())
     m0 = models[int(sizes[0])][1]
-    bytes_per_move = 10.0 * m0.gathers_per_flip()
+    bytes_per_move = 2.0 * bytes_per_flip(m0, batch.lanes_per_move(0) > 0)
     out = {"workload": "ternary FCC, 256 canonical chains, L^3 with L in 8..16 (512-4096 sites), pairs<=4th, "
                        "triplets<=3rd, quadruplets<=2nd shell, %d sweeps each, one launch" % sweeps,
            "value": total / wall, "unit": "moves/s", "moves": total, "kernel_ms": kernel_ms, "wall_s": wall,
@@ -262,7 +271,7 @@ def tempering(n_rep=128, cycles=2000, L=32, seed=9, lds_peak=None, cpu=True):
     state = pt.state()
     total = cycles * n_rep * st.n_sites
     acc = state["n_accept"].sum() / max(state["n_try"].sum(), 1)
-    bytes_per_move = 10.0 * model.gathers_per_flip()
+    bytes_per_move = 2.0 * bytes_per_flip(model, batch.lanes_per_move(0) > 0)
     out = {"workload": "quaternary FCC 32^3 (32768 sites), <=4-body to the 3rd shell (%d CFs, %d sub-clusters per "
                        "site), %d replicas 200-2000 K, exchange every sweep, %d of the workload's 2000 sweeps%s"
                        % (model.n_cf, model.n_subclusters, n_rep, cycles,
@@ -491,12 +500,12 @@ def main():
     plain_value = 200000 / plain_wall
     log("plain: %.3e moves/s (kernel %.2f ms)" % (plain_value, plain_ms))
 
-    bytes_per_flip = 5.0 * model.gathers_per_flip()
-    launch_bytes = bytes_per_flip * moves_per_chain * len(chains)
+    bytes_per_move = bytes_per_flip(model, batch.lanes_per_move(0) > 0)
+    launch_bytes = bytes_per_move * moves_per_chain * len(chains)
     default_shape = len(chains) == 1024 and args.sweeps == 500 and tuple(tune_w) == TRAFFIC_SHAPE
     roofline = roofline_of(launch_bytes, avg_kernel_ms, lds_meas)
     roofline.update({"traffic": TRAFFIC_DEFAULT_LAUNCH if default_shape else None, "hbm_copy_measured": hbm_meas,
-                     "bytes_per_move": bytes_per_flip, "kernel_ms": avg_kernel_ms})
+                     "bytes_per_move": bytes_per_move, "kernel_ms": avg_kernel_ms})
     out = {
         "metric": METRIC, "value": value, "unit": "moves/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": ms_step, "higher_is_better": True, "scaling": "weak",

@@ -92,6 +92,7 @@ SIGNATURES = [
     ("cemc_model_create", ctypes.c_int, [ctypes.POINTER(ModelDesc), ctypes.POINTER(_vp)]),
     ("cemc_model_set_ecis", ctypes.c_int, [_vp, _dp]),
     ("cemc_model_is_periodic", ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
+    ("cemc_model_patches", ctypes.c_int, [_vp, _i32p, _i32p]),
     ("cemc_model_destroy", ctypes.c_int, [_vp]),
     ("cemc_updater_create", ctypes.c_int, [_vp, _i8p, _dp, _dp, ctypes.POINTER(_vp)]),
     ("cemc_updater_destroy", ctypes.c_int, [_vp]),

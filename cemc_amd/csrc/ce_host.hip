@@ -2675,6 +2675,14 @@ int cemc_model_is_periodic(const cemc_model* m, int* periodic) {
   });
 }
 
+int cemc_model_patches(const cemc_model* m, int32_t* patches, int32_t* members) {
+  return guarded([&] {
+    require(m && patches && members, "NULL argument");
+    *patches = int32_t(m->patches.size());
+    *members = m->patches.empty() ? 0 : patch_members(m->n_species);
+  });
+}
+
 int cemc_model_destroy(cemc_model* m) {
   return guarded([&] { delete m; });
 }

@@ -231,6 +231,13 @@ class CEModel:
                     tot += len(cl["indices"]) * (int(cl["size"]) - 1)
         return tot
 
+    def patches(self):
+        """(patches of a site, members of each) of the patch kernel; (0, 0)
+        where the model has none."""
+        p, q = ctypes.c_int32(), ctypes.c_int32()
+        _capi.check(_capi.load().cemc_model_patches(self.handle, ctypes.byref(p), ctypes.byref(q)))
+        return p.value, q.value
+
     def close(self):
         if getattr(self, "handle", None):
             _capi.load().cemc_model_destroy(self.handle)

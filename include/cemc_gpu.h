@@ -103,6 +103,9 @@ CEMC_API int cemc_model_create(const cemc_model_desc* desc, cemc_model** out);
 CEMC_API int cemc_model_set_ecis(cemc_model* model, const double* eci);
 /* 1 when the closed-form periodic neighbour path is active, else 0. */
 CEMC_API int cemc_model_is_periodic(const cemc_model* model, int* periodic);
+/* Patches of a site (0: the model has none) and members of each; see
+ * cemc_batch_get_launch_shape. */
+CEMC_API int cemc_model_patches(const cemc_model* model, int32_t* patches, int32_t* members);
 CEMC_API int cemc_model_destroy(cemc_model* model);
 
 /* --------------------------------------------------------------- updater

@@ -552,33 +552,33 @@ void cemc_model::build_ptab() {
     patch_table(cover->tables[t], n_species, full ? q : q - 1, n_bfs, n_bfs, code_bits(), gtab.data(),
                 ptab.data() + ptab_base[t]);
   }
-  // spread of a flip's energy change: its sub-clusters' variances over the
-  // members' species and the two species of the flip, added up
-  const int k = code_bits(), Pc = 1 << (3 * k);
+  // Spread of a flip's energy change sum_d dphi_d G_d: the products of dphi over
+  // the flips' two species, times the covariances of the slices G_d over the
+  // members' species, added up over the sub-clusters.
+  const int S = n_species, B = n_bfs, k = code_bits(), Pc = 1 << (3 * k);
+  double flips[kMaxBasis][kMaxBasis] = {};
+  for (int o = 0; o < S; ++o)
+    for (int n = 0; n < S; ++n)
+      for (int d = 0; d < B; ++d)
+        for (int e = 0; e < B; ++e)
+          flips[d][e] += (basis[d * S + n] - basis[d * S + o]) * (basis[e * S + n] - basis[e * S + o]) / (S * (S - 1));
   std::map<std::pair<int, int>, int> count;  // (entry, reference position) -> sub-clusters
   for (size_t r = 0; r < recs.size(); ++r) ++count[{rec_entry[r], rec_refpos(recs[r])}];
   double var = 0.0;
   for (const auto& kv : count) {
     const int c = kv.first.first, nm = entry_size[c] - 1, codes = pow_s(nm);
     const double* G = gtab.data() + entry_goff[c] + kv.first.second * deco_slices() * Pc;
-    double sum = 0.0;
-    for (int o = 0; o < n_species; ++o)
-      for (int n = 0; n < n_species; ++n) {
-        if (n == o) continue;
-        double m1 = 0.0, m2 = 0.0;
-        for (int at = 0; at < codes; ++at) {
-          int code = 0;
-          for (int m = 0, rest = at; m < nm; ++m, rest /= n_species) code |= (rest % n_species) << (k * m);
-          double de = 0.0;
-          for (int d = 0; d < n_bfs; ++d)
-            de += (basis[d * n_species + n] - basis[d * n_species + o]) * G[d * Pc + code];
-          m1 += de;
-          m2 += de * de;
-        }
-        m1 /= codes;
-        sum += m2 / codes - m1 * m1;
+    double m1[kMaxBasis] = {}, m2[kMaxBasis][kMaxBasis] = {};
+    for (int at = 0; at < codes; ++at) {
+      int code = 0;
+      for (int m = 0, rest = at; m < nm; ++m, rest /= S) code |= (rest % S) << (k * m);
+      for (int d = 0; d < B; ++d) {
+        m1[d] += G[d * Pc + code] / codes;
+        for (int e = 0; e < B; ++e) m2[d][e] += G[d * Pc + code] * G[e * Pc + code] / codes;
       }
-    var += kv.second * sum / (n_species * (n_species - 1));
+    }
+    for (int d = 0; d < B; ++d)
+      for (int e = 0; e < B; ++e) var += kv.second * flips[d][e] * (m2[d][e] - m1[d] * m1[e]);
   }
   flip_sd = std::sqrt(std::max(var, 0.0));
 }

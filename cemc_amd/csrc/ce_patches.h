@@ -508,7 +508,8 @@ inline void patch_table(const std::vector<PatchTerm>& terms, int n_species, int 
       for (const PatchTerm& t : terms) {
         int rc = 0;
         for (int m = 0; m < t.n; ++m) rc |= sp[t.place[m]] << (bits * m);
-        sum += (long double)rec[t.block + (uint32_t(d) << (3 * bits)) + rc] / t.share;
+        const long double x = rec[t.block + (uint32_t(d) << (3 * bits)) + rc];
+        sum += t.share == 1 ? x : x / t.share;
       }
       dst[size_t(stride) * code + d] = double(sum);
     }

@@ -1890,6 +1890,33 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     std::nth_element(left.begin(), left.begin() + left.size() / 2, left.end());
     long_moves = std::max<int64_t>(8 * left[left.size() / 2], int64_t(1) << 20);
   }
+  // Chains whose moves mostly conflict make one or two moves of a patch round,
+  // where one move at a time is faster: small cells at high acceptance.  Time
+  // of the sweep kernel over the patch kernel's, by the conflict chance (FCC 5^3
+  // to 10^3, 3 to 84 patches): up to 256 chains 0.96-1.6 at 0.4-0.6 and 0.65-1.02
+  // above 0.8; 1024 chains 0.93-2.0 at 0.2-0.3 and 0.58-1.1 above 0.4; 4096
+  // chains 0.99-1.9 at 0.1-0.15 and 0.55-1.6 at 0.2-0.3.  With 164 and more
+  // patches 0.82-0.96 above 0.8, for any number.  Below, the patch kernel wins:
+  // 1.2 to 7.  (Walkers and chains with hooks have no such limit: their one-move
+  // kernels were slower at every conflict chance, 1.01 to 17.)  A pool does so
+  // only when nine in ten of its chains conflict: in mixed pools the second
+  // kernel's launches cost more than they save (5000 jobs of 6^3-24^3 sites: p50
+  // 1.50 s, with the split 1.95 s; p99 21.5 and 23.3 s).
+  if (!b->always_patches) {
+    int n_conflicting = 0;
+    for (int c = 0; c < n_chains; ++c) {
+      const cemc_model* m = b->models[b->params[c].model];
+      if (!included(c) || m->patches.empty() || (!b->hooks.empty() && b->hooks[c].on)) continue;
+      const double limit = m->patches.size() > 128 ? 0.8
+                           : on_device <= int64_t(2) * n_cu ? 0.55
+                           : on_device <= int64_t(4) * n_cu ? 0.3
+                                                            : 0.15;
+      b->conflict_limit[c] = limit;
+      b->conflicting[c] = conflict_chance(m, b->params[c], limit) > limit;
+      n_conflicting += b->conflicting[c];
+    }
+    if (b->dynamic && 10 * int64_t(n_conflicting) < 9 * int64_t(n_launch)) b->conflicting.assign(n_chains, 0);
+  }
   std::vector<Key> keys(n_chains);
   std::vector<bool> done(n_chains, false);
   for (int c = 0; c < n_chains; ++c) {
@@ -2044,23 +2071,9 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
     // Chains with a constraint on the state (a pair constraint, a site open to
     // some species, fixed species of SGC chains) or waste recycling stay on
     // the one-move kernel.
-    // Chains whose moves mostly conflict make one or two moves a round, where
-    // one move at a time is faster: small cells at high acceptance.  Time of the
-    // sweep kernel over the patch kernel's, by the conflict chance (FCC 5^3 to
-    // 10^3, 3 to 84 patches): up to 256 chains 0.96-1.6 at 0.4-0.6 and 0.65-1.02
-    // above 0.8; 1024 chains 0.93-2.0 at 0.2-0.3 and 0.58-1.1 above 0.4; 4096
-    // chains 0.99-1.9 at 0.1-0.15 and 0.55-1.6 at 0.2-0.3.  With 164 and more
-    // patches 0.82-0.96 above 0.8, for any number.  Below, the patch kernel wins:
-    // 1.2 to 7.  (Walkers and chains with hooks have no such limit: their one-move
-    // kernels were slower at every conflict chance, 1.01 to 17.)
     if (forced_waves == 0 && b->spec_moves == 0 && !k.field && (!k.hooks || b->hooks[c].by_proposal) &&
         !m->patches.empty() && (!canon || m->n_sites <= 65535)) {
       const int P = int(m->patches.size());
-      if (!b->always_patches && !k.hooks) {
-        b->conflict_limit[c] =
-            P > 128 ? 0.8 : (on_device <= int64_t(2) * n_cu ? 0.55 : (on_device <= int64_t(4) * n_cu ? 0.3 : 0.15));
-        b->conflicting[c] = conflict_chance(m, b->params[c], b->conflict_limit[c]) > b->conflict_limit[c];
-      }
       const uint32_t room = limit + sweep_static_lds() - kPatchStaticLds;
       // A pool's long job among crowds of 600-3000 short ones (chain_waves, 4
       // waves against 1 or 2, moves per ms): swaps of two species 2590 ->

@@ -111,3 +111,23 @@ def test_a_temperature_that_changes_the_kernel(gpu):
         done += 777
         assert np.array_equal(batch.occupation(0), ora.get_occupation())
         assert abs(batch.energies()[0] - ora.get_energy()) <= 1e-10 * s.n_sites
+
+
+def test_pools_whose_chains_conflict(gpu):
+    """A pool of small hot cells runs one move at a time, a mixed one does not
+    split its launches."""
+    from cemc_amd.batch import ChainPool
+    from cemc_amd.model import CEModel
+    s = FCCSettings(5, ["A", "B"], {2: 4, 3: 2})
+    model = CEModel(s, seeded_ecis(s, 3, 0.02))
+    occ = random_occupation(s.n_sites, 2, 3)
+    n = 20
+    pool = ChainPool(n, 1, n * 128, n * 128)
+    for c in range(n):
+        assert pool.add(model, dict(kind=0, temperature=2500.0, occupation=occ, seed=3, uid=c)) == c
+    print("pools", flush=True)
+    for cold, lanes in ((0, 0), (2, 0), (3, 16)):
+        for c in range(cold):
+            pool.set_temperature(c, 250.0)
+        pool.run(np.full(n, 100, dtype=np.int64))
+        assert pool.lanes_per_move(n - 1) == lanes

@@ -31,7 +31,7 @@ HBM_PEAK_GBS = 8000.0
 # WRITE_SIZE per dispatch, each scaled by what the counter reads for a copy
 # kernel of known size (x2.0 and x1.0).  Measured with rocprofv3 --pmc; summary
 # in profiles/kernels_by_workload.txt
-TRAFFIC_DEFAULT_LAUNCH = 3728000
+TRAFFIC_DEFAULT_LAUNCH = 4297000
 TRAFFIC_SHAPE = (0, 0, 0)  # autotune.AUTO
 
 

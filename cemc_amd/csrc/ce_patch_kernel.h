@@ -12,8 +12,10 @@
 // and so is one that a blocked one reaches; the others are made at once, in
 // any order, since none reads what another writes (interactions are mutual:
 // models where they are not have no patches).  Blocked moves stay open for the
-// next round.  (Ending the round at the first blocked move instead
-// made 5.6 moves of eight at the highest acceptances, now about 11 of 16.)
+// next round.  (Ending the round at the first blocked move instead made 5.6
+// moves of eight for hot flips on 10^3 sites, now about 11 of 16; swaps there at
+// acceptance 0.7 make 4.2.  Where most moves conflict the host keeps a chain off
+// this kernel, conflict_chance.)
 //
 // Work split.  A flip needs 12 (two species, pairs to the 4th shell and
 // triplets to the 2nd), 59 (three species, four-body clusters) or 426 (four
@@ -24,25 +26,26 @@
 //
 // What bounds it: instruction issue and LDS latency of the dependent chain of
 // a round, not bandwidth (binary SGC chains, counters per move: 18 VALU, 4
-// LDS and 3 scalar instructions, 27 of 45 quad-cycles issuing, 16 waiting;
-// the sweep kernel issued 43 VALU and 10 LDS).  So the loads of a phase are
-// issued together before the first wait (one binary chain, 40000 swaps: 14.6
-// -> 12.0 ms by that and by reading the tracker in the round instead of
-// comparing every commit with every lane); which moves reach which is tested
-// while the members are in flight; and what the next round does not need is
-// put off to the end of the block, where lane l holds move l: energies by one
-// prefix sum over the lanes, sample sums in per-lane accumulators added up
-// once per launch.  Blocks are the 64-move blocks of the chain's stream, and a
-// launch that ends inside one leaves its energy changes to the next, so
-// energies do not depend on where launches end.  Four-species models are bound by LDS reads instead (two
-// thirds of the cycles at eight waves).
+// LDS and 3 scalar instructions, 27 of 42 quad-cycles issuing, 11 waiting; the
+// sweep kernel's rounds of eight: 37 VALU, 8 LDS and 9 scalar, 60 of 90
+// issuing).  So the loads of a phase are issued together before the first wait
+// (one binary chain, 40000 swaps: 14.6 -> 12.0 ms by that and by reading the
+// tracker in the round instead of comparing every commit with every lane);
+// which moves reach which is tested while the members are in flight; and what
+// the next round does not need is put off to the end of the block, where lane l
+// holds move l: energies by one prefix sum over the lanes, sample sums in
+// per-lane accumulators added up once per launch.  Blocks are the 64-move blocks
+// of the chain's stream, and a launch that ends inside one leaves its energy
+// changes to the next, so energies do not depend on where launches end.
+// Four-species models are bound by LDS reads instead: 125 a swap, three
+// bank-conflict cycles each, 28 % of the cycles issuing at eight waves.
 //
 // Measured against the sweep kernel's automatic shapes, per pass with its reads
-// of the results: 1024 binary SGC chains of 500 sweeps 150 -> 63.6 ms (the
-// kernel 134 -> 54), 256 ternary chains of 512-4096 sites 55.6 -> 18.0 ms, a mix
-// of 48 binary and ternary chains 5.8 -> 1.6 ms, 128 quaternary 32^3 replicas
-// 56.7 -> 16.6 ms, one binary chain 23.9 -> 11.7 ms, 128 quaternary 8^3 chains
-// 5.4 -> 2.3 ms (1.25 ms of it the kernel).
+// of the results: 1024 binary SGC chains of 500 sweeps 149 -> 63 ms (the
+// kernel 133 -> 53), 256 ternary chains of 512-4096 sites 56 -> 18 ms, a mix of
+// 48 binary and ternary chains 5.8 -> 1.6 ms, 128 quaternary 32^3 replicas 56.3
+// -> 16.3 ms, one binary chain 23.9 -> 11.8 ms, 128 quaternary 8^3 chains 5.4 ->
+// 2.3 ms (1.24 ms of it the kernel), 64 binary walkers 44.5 -> 24.1 ms.
 #pragma once
 
 #include "ce_patches.h"

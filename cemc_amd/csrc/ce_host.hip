@@ -1905,8 +1905,9 @@ void derive_classes(cemc_batch* b, int forced_waves, const std::vector<int64_t>*
   if (!b->always_patches) {
     int n_conflicting = 0;
     for (int c = 0; c < n_chains; ++c) {
+      if (!included(c) || (!b->hooks.empty() && b->hooks[c].on)) continue;
       const cemc_model* m = b->models[b->params[c].model];
-      if (!included(c) || m->patches.empty() || (!b->hooks.empty() && b->hooks[c].on)) continue;
+      if (m->patches.empty()) continue;
       const double limit = m->patches.size() > 128 ? 0.8
                            : on_device <= int64_t(2) * n_cu ? 0.55
                            : on_device <= int64_t(4) * n_cu ? 0.3

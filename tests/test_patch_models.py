@@ -131,3 +131,19 @@ def test_pools_whose_chains_conflict(gpu):
             pool.set_temperature(c, 250.0)
         pool.run(np.full(n, 100, dtype=np.int64))
         assert pool.lanes_per_move(n - 1) == lanes
+
+
+def test_pools_with_empty_slots(gpu):
+    """Launches of a pool that never had a chain, and of one whose chains left."""
+    from cemc_amd.batch import ChainPool
+    from cemc_amd.model import CEModel
+    s = FCCSettings(5, ["A", "B"], {2: 4, 3: 2})
+    pool = ChainPool(4, 1, 4 * 128, 4 * 128)
+    print("empty pool", flush=True)
+    pool.run(np.zeros(4, dtype=np.int64))
+    model = CEModel(s, seeded_ecis(s, 3, 0.02))
+    c = pool.add(model, dict(kind=0, temperature=900.0, occupation=random_occupation(s.n_sites, 2, 3), seed=3, uid=0))
+    pool.run(np.where(np.arange(4) == c, 100, 0))
+    assert pool.stats()["moves"][c] == 100
+    pool.remove(c)
+    pool.run(np.zeros(4, dtype=np.int64))
